@@ -17,7 +17,7 @@
 // layer's weights (M = output channels, in 16-channel tiles) times a 16-cell
 // row of its input (N), K over (tap, input channel) in chunks of 32, the
 // input brick and the weights staged in LDS. The weight gradient (k_wgrad)
-// uses v_mfma_f32_16x16x16_f16 with K over cells.
+// uses the same product with K over cells.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -39,8 +39,6 @@ typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-constexpr int WAVES = 4;  // wavefronts per workgroup of the weight-gradient kernels
-constexpr int THREADS = 64 * WAVES;
 #ifndef FSP_CONV_WAVES
 #define FSP_CONV_WAVES 8  // 8 measured faster than 4 at 256x256x128 (1.03 vs 1.31 ms per forward)
 #endif
@@ -90,7 +88,7 @@ struct ConvArgs {
   const _Float16* in;    // [cells_in][CIN]
   const _Float16* wt;    // [npad(COUT)][K]; K = kpad(CIN), kfwd for row pairs; k_conv_up: k_pack_up's layout
   const float* bias;     // [COUT] (forward only)
-  const _Float16* skip;  // [cells][COUT] (k_conv_up)
+  const _Float16* skip;  // [cells][COUT] (k_conv_up: added; k_conv EPI 3: the ReLU's activation)
   _Float16* out;         // [cells][COUT]
   float* yout;           // head: [cells]
   const int32_t* gate;   // return at once while *gate == 0 (null: always run)
@@ -115,7 +113,9 @@ __host__ __device__ constexpr int tap_offset(int tap, int hx, int hy) {
 }
 
 // EPI 0: bias + ReLU -> binary16; 1: bias -> f32 channel 0 (head);
-// 2: plain product -> binary16 (backward data). The upsampling layers (input
+// 2: plain product -> binary16 (backward data); 3: the same, zero where the
+// activation a.skip is not positive (backward data through a ReLU; a pass of
+// its own over the gradient took 11 us per 8-channel layer at 128^3). The upsampling layers (input
 // from the coarser level, skip added before the ReLU) run k_conv_up.
 //
 // D[co][cell] = W[co][k] X[k][cell] on v_mfma_f32_16x16x32_f16: the weights
@@ -129,7 +129,7 @@ __host__ __device__ constexpr int tap_offset(int tap, int hx, int hy) {
 template <int CIN, int COUT, int EPI>
 __global__ void __launch_bounds__(CTHREADS, FSP_CONV_MIN_WAVES) k_conv(ConvArgs a) {
   using Bk = ConvBrick<CIN, COUT>;
-  constexpr bool PAIR = EPI != 2 && pair_rows(CIN, COUT);
+  constexpr bool PAIR = EPI < 2 && pair_rows(CIN, COUT);
   constexpr int TPW = PAIR ? Bk::TPW / 2 : Bk::TPW;
   constexpr int NT = npad(COUT) / 16;
   constexpr int KP = PAIR ? kfwd(CIN, COUT) : kpad(CIN);
@@ -300,6 +300,10 @@ __global__ void __launch_bounds__(CTHREADS, FSP_CONV_MIN_WAVES) k_conv(ConvArgs 
       if (EPI == 2) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] = (_Float16)val[e];
+      } else if (EPI == 3) {
+        const h4 h = *reinterpret_cast<const h4*>(a.skip + cell * COUT + co);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (float)h[e] > 0.f ? (_Float16)val[e] : (_Float16)0.f;
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -478,101 +482,246 @@ __global__ void __launch_bounds__(CTHREADS, FSP_CONV_MIN_WAVES) k_conv_up(ConvAr
 }
 
 // ---------------------------------------------------------------- weight gradient
-// Partial dW[co][k] = sum over the cells of one partition of g[cell][co] *
-// in[cell + tap][ci] (k = tap*CIN + ci), one wavefront per (partition, k
-// chunk, co tile); D = A B with A[co][cell] = g, B[cell][k] = shifted input.
+// dW[co][tap][ci] = sum over cells of g[cell][co] * in[cell + tap][ci], and
+// db[co] = sum of g[cell][co], as products D[co][(dz, dy, ci)] = A B with
+// K = 32 cells on v_mfma_f32_16x16x32_f16.
+//
+// Both operands run over cells in K, which the channels-last layout holds
+// last, so a workgroup stages a brick of 16 cells x BY rows x BZ planes of g
+// and its input halo in LDS transposed: one row of cells per channel. A K
+// chunk is two rows of 16 cells; a lane's eight K values are eight
+// consecutive cells of one channel, one ds_read_b128. The three taps of dx
+// share that read: the shifted operands are funnel shifts of it with the
+// cell before and the cell after (the cells x0 + 16 and x0 - 1 of a row lie
+// in one dword after it). Without the shared read and the staging (one wavefront
+// per (partition, 16 columns) gathering 2-byte values from memory, and one
+// workgroup per channel for db) a 128^3 gradient took 3.3 ms in its weight
+// products, 1.2 ms in their reduction and 11.3 ms in the bias sums; now 0.38
+// ms and 0.06 ms, the bias sums among the products (all of loss and gradients
+// 17.2 -> 0.95 ms). The 8 -> 8 layer at 128^3 takes 45 us for 67 MB (1.5 TB/s):
+// its workgroups alternate between loading a brick and multiplying it.
+//
+// A tile of 16 columns is 16 input channels at one (dz, dy), or two or four
+// (dz, dy) of 8 or 4 channels; a "triple" is that tile at dx = -1, 0, 1.
+// Wavefronts are split into GROUPS (output-channel tile, input-channel half)
+// of 9 triples at most, which keeps the accumulators (108 registers) and the
+// operands of a wavefront in registers, and share the brick's chunks within
+// a group. A workgroup walks bricks gridDim.x apart, accumulates in
+// registers, folds its wavefronts in LDS in a fixed order and writes one
+// partial; k_wgrad_reduce folds the partials.
+template <int CIN, int COUT>
+struct WgradBrick {
+  static constexpr int BX = 16, BY = 8, BZ = (CIN >= 16 || COUT >= 32) ? 4 : 8;
+  static constexpr int HY = BY + 2, HZ = BZ + 2;
+  static constexpr int SUB = CIN >= 16 ? 1 : 16 / CIN;  // (dz, dy) per tile
+  static constexpr int NC = CIN >= 16 ? CIN / 16 : 1;   // input-channel tiles
+  static constexpr int MT = npad(COUT) / 16;
+  static constexpr int GROUPS = MT * NC;
+  static constexpr int TR = (9 + SUB - 1) / SUB;  // triples per group
+  static constexpr int WV = 8;                    // wavefronts per workgroup
+  static constexpr int SLICES = WV / GROUPS;
+  static constexpr int XR = 24;  // halves per (row, channel) of the input: 16 cells, (x16, x-1), 16-byte rows
+  static constexpr int TILES = GROUPS * TR * 3;
+  static constexpr int ELEMS = TILES * 256 + npad(COUT);  // one partial: the tiles, then the bias sums
+  static constexpr int IN_HALVES = HZ * HY * CIN * XR, G_HALVES = BZ * BY * COUT * 16;
+  static constexpr size_t STAGE_BYTES = 2 * (size_t)(IN_HALVES + G_HALVES);
+  static constexpr size_t LDS_BYTES = STAGE_BYTES > (size_t)ELEMS * 4 ? STAGE_BYTES : (size_t)ELEMS * 4;
+  static_assert(WV % GROUPS == 0 && (CIN == 4 || CIN % 8 == 0) && (COUT == 1 || COUT % 8 == 0), "tiles");
+};
+
 struct WgradArgs {
-  int nx, ny, nz, cnx, cny, cnz;
-  const _Float16* g;    // [cells][gs]: gradient at the layer's pre-activation (channels 0..COUT-1)
-  int gs;
-  const _Float16* in;   // layer input
-  float* partial;       // [parts][npad(COUT)][kpad(CIN)]
-  int parts;
+  int nx, ny, nz, cnx, cny, cnz;  // cells of g; cells of the input (the coarse grid when UP)
+  const _Float16* g;              // [cells][gs]: gradient at the layer's pre-activation (channels 0..COUT-1)
+  const _Float16* in;             // layer input
+  float* partial;                 // [gridDim.x][ELEMS]
 };
 
 template <int CIN, int COUT, int UP>
-__global__ void __launch_bounds__(THREADS) k_wgrad(WgradArgs a) {
-  constexpr int MT = npad(COUT) / 16;
-  constexpr int KP = kpad(CIN);
-  constexpr int CHUNKS = KP / 16;
-  const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * WAVES + (threadIdx.x >> 6);
-  const int jobs = CHUNKS * MT;
-  if (wave >= jobs * a.parts) return;
-  const int job = wave % jobs, part = wave / jobs;
-  const int ch = job % CHUNKS, mt = job / CHUNKS;
-  const int m = lane & 15, g4 = lane >> 4;
-  const int kk = ch * 16 + m;  // this lane's B column
-  const int tap = kk / CIN, ci = kk - tap * CIN;
-  const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-  const int co = mt * 16 + m;  // this lane's A row
-  const int segs = a.nx / 16;
-  const long total = (long)segs * a.ny * a.nz;
-  const long per = (total + a.parts - 1) / a.parts;
-  const long s0 = per * part, s1 = s0 + per < total ? s0 + per : total;
-  f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-  for (long s = s0; s < s1; ++s) {
-    const int seg = (int)(s % segs);
-    const long row = s / segs;
-    const int y = (int)(row % a.ny), z = (int)(row / a.ny);
-    const size_t rowbase = ((size_t)z * a.ny + y) * a.nx + seg * 16;
-    h4 av, bv;
+__global__ void __launch_bounds__(512, 2) k_wgrad(WgradArgs a) {
+  using Bk = WgradBrick<CIN, COUT>;
+  constexpr int NT = 64 * Bk::WV;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[Bk::LDS_BYTES];
+  _Float16* xin = reinterpret_cast<_Float16*>(smem);
+  _Float16* gl = xin + Bk::IN_HALVES;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m = lane & 15, g4 = lane >> 4, half = g4 & 1, ry = g4 >> 1;
+  const int grp = wave % Bk::GROUPS, slice = wave / Bk::GROUPS;
+  const int mt = grp / Bk::NC, nc = grp % Bk::NC;
+  const int co = COUT >= 16 ? mt * 16 + m : m % COUT;  // rows past COUT repeat: their products are not kept
+  const int ci = CIN >= 16 ? nc * 16 + m : m % CIN;
+  const int bx = a.nx / Bk::BX, by = (a.ny + Bk::BY - 1) / Bk::BY, bz = (a.nz + Bk::BZ - 1) / Bk::BZ;
+  f4 acc[Bk::TR][3], accb = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int xc = seg * 16 + 4 * g4 + v;
-      av[v] = co < COUT ? a.g[(rowbase + 4 * g4 + v) * a.gs + co] : (_Float16)0;
-      _Float16 b = 0;
-      const int xx = xc + dx, yy = y + dy, zz = z + dz;
-      if (tap < 27 && xx >= 0 && xx < a.nx && yy >= 0 && yy < a.ny && zz >= 0 && zz < a.nz) {
-        size_t q;
-        if (UP) q = ((size_t)(zz >> 1) * a.cny + (yy >> 1)) * a.cnx + (xx >> 1);
-        else q = ((size_t)zz * a.ny + yy) * a.nx + xx;
-        b = a.in[q * CIN + ci];
+  for (int t = 0; t < Bk::TR; ++t)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) acc[t][d] = f4{0.f, 0.f, 0.f, 0.f};
+  const _Float16 one = (_Float16)1.0f;
+  const h8 ones = h8{one, one, one, one, one, one, one, one};
+
+  for (int b = (int)blockIdx.x; b < bx * by * bz; b += (int)gridDim.x) {
+    const int x0 = (b % bx) * Bk::BX, y0 = ((b / bx) % by) * Bk::BY, z0 = (b / (bx * by)) * Bk::BZ;
+    // stage: an item is a pair of cells (x, x + 1) -- or (x0 + 16, x0 - 1) --
+    // of one row and up to eight channels; every load of a thread is in
+    // flight before its first LDS write; cells outside the grid are zero
+    constexpr int VH = CIN >= 8 ? 8 : 4, VPC = CIN / VH;
+    typedef uint32_t hv __attribute__((ext_vector_type(VH / 2)));
+    constexpr int ITEMS = Bk::HZ * Bk::HY * 9 * VPC, PER = (ITEMS + NT - 1) / NT;
+    hv lo[PER], hi[PER];
+    auto load = [&](int xx, int yy, int zz, int part) {
+      hv v = hv(0u);
+      if (xx >= 0 && xx < a.nx && yy >= 0 && yy < a.ny && zz >= 0 && zz < a.nz) {
+        const size_t q = UP ? ((size_t)(zz >> 1) * a.cny + (yy >> 1)) * a.cnx + (xx >> 1)
+                            : ((size_t)zz * a.ny + yy) * a.nx + xx;
+        v = *reinterpret_cast<const hv*>(a.in + q * CIN + part * VH);
       }
-      bv[v] = b;
-    }
-    acc = __builtin_amdgcn_mfma_f32_16x16x16f16(av, bv, acc, 0, 0, 0);
-  }
-  // lane holds D[co 4*g4+v][k m] of this (co tile, k chunk)
-  float* P = a.partial + (size_t)part * npad(COUT) * KP;
+      return v;
+    };
 #pragma unroll
-  for (int v = 0; v < 4; ++v) P[(size_t)(mt * 16 + 4 * g4 + v) * KP + ch * 16 + m] = acc[v];
-}
-
-// Sum of the partitions in order; dW in the flat parameter layout, scaled
-// by 1/scale; flags a non-finite value.
-__global__ void k_wgrad_reduce(const float* partial, int parts, int cin, int cout, float inv_scale, float* grad,
-                               int* bad) {
-  const int KP = kpad(cin), NP = npad(cout);
-  const int n = cout * 27 * cin;
-  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x) {
-    const int co = q / (27 * cin), k = q - co * 27 * cin;
-    float s = 0.f;
-    for (int p = 0; p < parts; ++p) s += partial[((size_t)p * NP + co) * KP + k];
-    s *= inv_scale;
-    if (!isfinite(s)) *bad = 1;
-    grad[q] = s;
+    for (int r = 0; r < PER; ++r) {
+      const int q = tid + r * NT;
+      const int part = q % VPC, xi = (q / VPC) % 9, row = q / (9 * VPC);
+      const int yy = y0 + row % Bk::HY - 1, zz = z0 + row / Bk::HY - 1;
+      const bool in = q < ITEMS;
+      lo[r] = in ? load(xi < 8 ? x0 + 2 * xi : x0 + 16, yy, zz, part) : hv(0u);
+      hi[r] = in ? load(xi < 8 ? x0 + 2 * xi + 1 : x0 - 1, yy, zz, part) : hv(0u);
+    }
+    constexpr int GVH = COUT >= 8 ? 8 : 1, GVPC = COUT / GVH, GS = COUT < 4 ? 4 : COUT;  // GS: channels g holds
+    constexpr int GITEMS = Bk::BZ * Bk::BY * 8 * GVPC, GPER = (GITEMS + NT - 1) / NT;
+    h8 glo[GPER], ghi[GPER];
+#pragma unroll
+    for (int r = 0; r < GPER; ++r) {
+      const int q = tid + r * NT;
+      const int part = q % GVPC, xi = (q / GVPC) % 8, row = q / (8 * GVPC);
+      const int yy = y0 + row % Bk::BY, zz = z0 + row / Bk::BY;
+      glo[r] = h8(0);
+      ghi[r] = h8(0);
+      if (q < GITEMS && yy < a.ny && zz < a.nz) {
+        const _Float16* src = a.g + (((size_t)zz * a.ny + yy) * a.nx + x0 + 2 * xi) * GS + part * GVH;
+        if (GVH == 8) {
+          glo[r] = *reinterpret_cast<const h8*>(src);
+          ghi[r] = *reinterpret_cast<const h8*>(src + GS);
+        } else {
+          glo[r][0] = src[0];
+          ghi[r][0] = src[GS];
+        }
+      }
+    }
+    __syncthreads();  // the previous brick's operands have been read
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+      const int q = tid + r * NT;
+      if (q >= ITEMS) break;
+      const int part = q % VPC, xi = (q / VPC) % 9, row = q / (9 * VPC);
+      uint32_t* dst = reinterpret_cast<uint32_t*>(xin + (size_t)(row * CIN + part * VH) * Bk::XR) + xi;
+#pragma unroll
+      for (int c = 0; c < VH; ++c) {
+        // channel c of the two cells in one dword (cell x low)
+        const uint32_t l = lo[r][c >> 1], h = hi[r][c >> 1];
+        dst[c * (Bk::XR / 2)] = (c & 1) ? ((h & 0xFFFF0000u) | (l >> 16)) : ((h << 16) | (l & 0xFFFFu));
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < GPER; ++r) {
+      const int q = tid + r * NT;
+      if (q >= GITEMS) break;
+      const int part = q % GVPC, xi = (q / GVPC) % 8, row = q / (8 * GVPC);
+      typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+      h2* dst = reinterpret_cast<h2*>(gl + (size_t)(row * COUT + part * GVH) * 16) + xi;
+#pragma unroll
+      for (int c = 0; c < GVH; ++c) dst[c * 8] = h2{glo[r][c], ghi[r][c]};
+    }
+    __syncthreads();
+    for (int ch = slice; ch < Bk::BZ * Bk::BY / 2; ch += Bk::SLICES) {
+      const int z = ch / (Bk::BY / 2), y = 2 * (ch % (Bk::BY / 2)) + ry;
+      const h8 av = *reinterpret_cast<const h8*>(gl + ((z * Bk::BY + y) * COUT + co) * 16 + 8 * half);
+      accb = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, ones, accb, 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < Bk::TR; ++t) {
+        const int d0 = CIN >= 16 ? t : t * Bk::SUB + m / CIN;
+        const int d = d0 < 9 ? d0 : 8;  // columns past the nine (dz, dy) repeat the last: not kept
+        const _Float16* row = xin + (((z + d / 3) * Bk::HY + y + d % 3) * CIN + ci) * Bk::XR;
+        const uint4 w = *reinterpret_cast<const uint4*>(row + 8 * half);
+        const uint32_t prev = *reinterpret_cast<const uint32_t*>(row + (half ? 6 : 16));   // cell before, high half
+        const uint32_t next = *reinterpret_cast<const uint32_t*>(row + (half ? 16 : 8));   // cell after, low half
+        const uint32_t s01 = __builtin_amdgcn_alignbit(w.y, w.x, 16), s12 = __builtin_amdgcn_alignbit(w.z, w.y, 16),
+                       s23 = __builtin_amdgcn_alignbit(w.w, w.z, 16);
+        const uint4 before = make_uint4(__builtin_amdgcn_alignbit(w.x, prev, 16), s01, s12, s23);
+        const uint4 after = make_uint4(s01, s12, s23, __builtin_amdgcn_alignbit(next, w.w, 16));
+        acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, *reinterpret_cast<const h8*>(&before), acc[t][0], 0, 0, 0);
+        acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, *reinterpret_cast<const h8*>(&w), acc[t][1], 0, 0, 0);
+        acc[t][2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, *reinterpret_cast<const h8*>(&after), acc[t][2], 0, 0, 0);
+      }
+    }
   }
-}
-
-// Bias gradient: sum over cells of g[cell][co], one workgroup per channel.
-__global__ void __launch_bounds__(256) k_bgrad(const _Float16* g, size_t cells, int gs, float inv_scale, float* grad,
-                                               int* bad) {
-  __shared__ float red[256];
-  const int co = blockIdx.x;
-  float s = 0.f;
-  for (size_t c = threadIdx.x; c < cells; c += 256) s += (float)g[c * gs + co];
-  red[threadIdx.x] = s;
+  // fold the wavefronts of each group in LDS, slice after slice
+  float* red = reinterpret_cast<float*>(smem);
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+#pragma unroll
+  for (int s = 0; s < Bk::SLICES; ++s) {
+    if (slice == s) {
+#pragma unroll
+      for (int t = 0; t < Bk::TR; ++t)
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            float* e = red + ((grp * Bk::TR + t) * 3 + d) * 256 + (4 * g4 + v) * 16 + m;
+            *e = s == 0 ? acc[t][d][v] : *e + acc[t][d][v];
+          }
+      if (nc == 0 && m == 0)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          float* e = red + Bk::TILES * 256 + mt * 16 + 4 * g4 + v;
+          *e = s == 0 ? accb[v] : *e + accb[v];
+        }
+    }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    const float v = red[0] * inv_scale;
-    if (!isfinite(v)) *bad = 1;
-    grad[co] = v;
+  float* P = a.partial + (size_t)blockIdx.x * Bk::ELEMS;
+  for (int q = tid; q < Bk::ELEMS; q += NT) P[q] = red[q];
+}
+
+// Sum of the partials into dW (flat parameter layout) and db, scaled by
+// 1/scale; flags a non-finite value. A workgroup takes 64 consecutive
+// elements of the partials and splits the partitions over its 16
+// wavefronts, folded in order (one thread per weight walking every
+// partition: 103 us per layer, a chain of dependent rounds of loads).
+template <int CIN, int COUT>
+__global__ void __launch_bounds__(1024) k_wgrad_reduce(const float* partial, int parts, float inv_scale, float* grad,
+                                                       int* bad) {
+  using Bk = WgradBrick<CIN, COUT>;
+  __shared__ float red[16][64];
+  const int col = (int)threadIdx.x & 63, slice = (int)threadIdx.x >> 6;
+  const int e = (int)blockIdx.x * 64 + col;
+  int out = -1;  // the element's place in the gradient
+  if (e < Bk::TILES * 256) {
+    const int tile = e / 256, r = (e % 256) / 16, n = e % 16;
+    const int grp = tile / (Bk::TR * 3), t = (tile / 3) % Bk::TR, dx = tile % 3;
+    const int co = (grp / Bk::NC) * 16 + r;
+    const int d = CIN >= 16 ? t : t * Bk::SUB + n / CIN, ci = CIN >= 16 ? (grp % Bk::NC) * 16 + n : n % CIN;
+    if (co < COUT && d < 9) out = (co * 27 + d * 3 + dx) * CIN + ci;
+  } else if (e - Bk::TILES * 256 < COUT) {
+    out = COUT * 27 * CIN + e - Bk::TILES * 256;
   }
+  float s = 0.f;
+  if (out >= 0) {
+    int p = slice;
+    for (; p + 7 * 16 < parts; p += 8 * 16) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = partial[(size_t)(p + 16 * u) * Bk::ELEMS + e];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += v[u];
+    }
+    for (; p < parts; p += 16) s += partial[(size_t)p * Bk::ELEMS + e];
+  }
+  red[slice][col] = s;
+  __syncthreads();
+  if (slice != 0 || out < 0) return;
+  for (int w = 1; w < 16; ++w) s += red[w][col];
+  s *= inv_scale;
+  if (!isfinite(s)) *bad = 1;
+  grad[out] = s;
 }
 
 // ---------------------------------------------------------------- elementwise
@@ -606,39 +755,82 @@ __global__ void k_pool(const _Float16* in, _Float16* out, int cnx, int cny, int 
     *reinterpret_cast<h8*>(out + ((size_t)row * cnx + i) * C + 8 * g) = o;
   }
 }
-// g_fine = g_coarse[parent] / 8 (+ add[fine])
-__global__ void k_pool_back(const _Float16* gc, const _Float16* add, _Float16* gf, int fnx, int fny, int fnz, int C) {
-  const size_t total = (size_t)fnx * fny * fnz * C;
-  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (size_t)gridDim.x * blockDim.x) {
-    const int c = (int)(q % C);
-    const size_t cell = q / C;
-    const int i = (int)(cell % fnx), j = (int)((cell / fnx) % fny), k = (int)(cell / ((size_t)fnx * fny));
+// The elementwise passes of the backward gradient take eight channels (16
+// bytes) of one cell per thread, one thread per item, and apply the ReLU
+// (g = 0 where the activation h is not positive) to the value they store, in
+// place of a pass of its own (10 us per layer at 128^3 at level 0). Block
+// (64, 4): x runs over (cell x, group of eight channels), y over rows.
+__device__ __forceinline__ h8 relu_masked(const float v[8], const h8 h) {
+  h8 o;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) o[c] = (float)h[c] > 0.f ? (_Float16)v[c] : (_Float16)0.f;
+  return o;
+}
+// g_fine = (g_coarse[parent] / 8 + add[fine]) where h > 0
+template <int C>
+__global__ void __launch_bounds__(256) k_pool_back(const _Float16* gc, const _Float16* add, const _Float16* h,
+                                                   _Float16* gf, int fnx, int fny, int fnz) {
+  constexpr int G = C / 8;
+  const int t = blockIdx.x * 64 + threadIdx.x;
+  if (t >= fnx * G) return;
+  const int i = t / G, c0 = 8 * (t % G), rows = fny * fnz;
+  for (int row = blockIdx.y * 4 + threadIdx.y; row < rows; row += gridDim.y * 4) {
+    const int j = row % fny, k = row / fny;
     const size_t p = ((size_t)(k >> 1) * (fny >> 1) + (j >> 1)) * (fnx >> 1) + (i >> 1);
-    float v = (float)gc[p * C + c] * 0.125f;
-    if (add) v += (float)add[q];
-    gf[q] = (_Float16)v;
+    const size_t q = ((size_t)row * fnx + i) * C + c0;
+    const h8 g = *reinterpret_cast<const h8*>(gc + p * C + c0), ad = *reinterpret_cast<const h8*>(add + q);
+    const h8 hv = *reinterpret_cast<const h8*>(h + q);
+    float v[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      v[c] = (float)g[c] * 0.125f;
+      v[c] += (float)ad[c];
+    }
+    *reinterpret_cast<h8*>(gf + q) = relu_masked(v, hv);
   }
 }
-// g_coarse = sum of the eight children's g_fine
-__global__ void k_up_back(const _Float16* gf, _Float16* gc, int cnx, int cny, int cnz, int C) {
-  const size_t total = (size_t)cnx * cny * cnz * C;
-  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (size_t)gridDim.x * blockDim.x) {
-    const int c = (int)(q % C);
-    const size_t cell = q / C;
-    const int i = (int)(cell % cnx), j = (int)((cell / cnx) % cny), k = (int)(cell / ((size_t)cnx * cny));
-    const int fnx = 2 * cnx, fny = 2 * cny;
-    float s = 0.f;
-    for (int dz = 0; dz < 2; ++dz)
-      for (int dy = 0; dy < 2; ++dy)
-        for (int dx = 0; dx < 2; ++dx)
-          s += (float)gf[(((size_t)(2 * k + dz) * fny + 2 * j + dy) * fnx + 2 * i + dx) * C + c];
-    gc[q] = (_Float16)s;
+// g_coarse = sum of the eight children's g_fine (in the order dz, dy, dx) where h > 0
+template <int C>
+__global__ void __launch_bounds__(256) k_up_back(const _Float16* gf, const _Float16* h, _Float16* gc, int cnx, int cny,
+                                                 int cnz) {
+  constexpr int G = C / 8;
+  const int t = blockIdx.x * 64 + threadIdx.x;
+  if (t >= cnx * G) return;
+  const int i = t / G, c0 = 8 * (t % G), fnx = 2 * cnx, fny = 2 * cny, rows = cny * cnz;
+  for (int row = blockIdx.y * 4 + threadIdx.y; row < rows; row += gridDim.y * 4) {
+    const int j = row % cny, k = row / cny;
+    h8 f[8];
+#pragma unroll
+    for (int d = 0; d < 8; ++d)
+      f[d] = *reinterpret_cast<const h8*>(
+          gf + (((size_t)(2 * k + (d >> 2)) * fny + 2 * j + ((d >> 1) & 1)) * fnx + 2 * i + (d & 1)) * C + c0);
+    const size_t q = ((size_t)row * cnx + i) * C + c0;
+    const h8 hv = *reinterpret_cast<const h8*>(h + q);
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < 8; ++d)
+#pragma unroll
+      for (int c = 0; c < 8; ++c) v[c] += (float)f[d][c];
+    *reinterpret_cast<h8*>(gc + q) = relu_masked(v, hv);
   }
 }
-// g = g * (h > 0)
-__global__ void k_relu_back(const _Float16* h, _Float16* g, size_t n) {
-  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x)
-    if (!((float)h[q] > 0.f)) g[q] = (_Float16)0.f;
+// Cells with a non-zero flag (16 at a time; the array's unaligned ends byte by byte).
+__global__ void __launch_bounds__(256) k_count_flags(const uint8_t* flags, size_t n, unsigned long long* count) {
+  const size_t head = min(n, (size_t)((16u - ((uintptr_t)flags & 15u)) & 15u));
+  const size_t vecs = (n - head) / 16;
+  const uint4* v = reinterpret_cast<const uint4*>(flags + head);
+  unsigned s = 0;
+  auto word = [&](uint32_t w) {
+    s += ((w & 0xFFu) != 0u) + ((w & 0xFF00u) != 0u) + ((w & 0xFF0000u) != 0u) + ((w & 0xFF000000u) != 0u);
+  };
+  const size_t t0 = (size_t)blockIdx.x * 256 + threadIdx.x, stride = (size_t)gridDim.x * 256;
+  for (size_t q = t0; q < vecs; q += stride) {
+    const uint4 w = v[q];
+    word(w.x); word(w.y); word(w.z); word(w.w);
+  }
+  for (size_t q = t0; q < n - 16 * vecs; q += stride) s += flags[q < head ? q : q + 16 * vecs] != 0;
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
+  if ((threadIdx.x & 63) == 0 && s) atomicAdd(count, (unsigned long long)s);
 }
 // Loss: mean of (y - t)^2 over wet cells; per-block f64 partials; the
 // output gradient scale * 2 (y - t) wet / n_wet as a 4-channel binary16
@@ -877,7 +1069,8 @@ struct fsp_net {
   size_t poff[NL] = {};  // offset of layer l's W in theta (b follows)
   int* bad = nullptr;
   int* hbad = nullptr;
-  double* hloss = nullptr;
+  unsigned long long *nwet = nullptr, *hnwet = nullptr;  // wet cells of the loss in progress
+  hipEvent_t counted = nullptr;                          // hnwet is there
   uint64_t step = 0;
   float gscale = 0.f;
   // activations for one shape
@@ -921,9 +1114,10 @@ void free_shape(fsp_net* N, size_t keep) {
 
 template <int CIN, int COUT, int EPI>
 void conv(hipStream_t st, int nx, int ny, int nz, const _Float16* in, const _Float16* wt, const float* bias,
-          _Float16* out, float* yout, const int32_t* gate = nullptr) {
+          _Float16* out, float* yout, const int32_t* gate = nullptr, const _Float16* relu = nullptr) {
   ConvArgs a{};
   a.gate = gate;
+  a.skip = relu;
   a.nx = nx; a.ny = ny; a.nz = nz;
   a.cnx = nx; a.cny = ny; a.cnz = nz;
   a.in = in; a.wt = wt; a.bias = bias; a.out = out; a.yout = yout;
@@ -947,26 +1141,45 @@ void conv_up(hipStream_t st, int nx, int ny, int nz, const _Float16* in, const _
   k_conv_up<CIN, COUT><<<grid, CTHREADS, 0, st>>>(a);
 }
 
-// dW of layer l (g: gradient at its pre-activation with channel stride gs)
+// Workgroups of a layer's weight gradient on an nx x ny x nz grid: one per
+// brick up to two per CU, or one where a workgroup's staging (over 64 KiB of
+// LDS) or its partial is large.
+template <int CIN, int COUT>
+int wgrad_parts(int nx, int ny, int nz) {
+  using Bk = WgradBrick<CIN, COUT>;
+  const size_t bricks = (size_t)(nx / Bk::BX) * ((ny + Bk::BY - 1) / Bk::BY) * ((nz + Bk::BZ - 1) / Bk::BZ);
+  return (int)std::min<size_t>(bricks, Bk::LDS_BYTES <= 65536 && Bk::ELEMS <= 8192 ? 512 : 256);
+}
+
+// dW and db of layer l (g: gradient at its pre-activation)
 template <int CIN, int COUT, int UP>
-void wgrad(fsp_net* N, int l, int nx, int ny, int nz, const _Float16* g, const _Float16* in, int gs = COUT) {
-  constexpr int MT = npad(COUT) / 16, CH = kpad(CIN) / 16;
-  const size_t segs = (size_t)(nx / 16) * ny * nz;
-  int parts = (int)((8192 + CH * MT - 1) / (CH * MT));
-  if ((size_t)parts > segs) parts = (int)segs;
-  if ((size_t)parts * npad(COUT) * kpad(CIN) > N->partial_floats) parts = (int)(N->partial_floats / (npad(COUT) * kpad(CIN)));
-  if (parts < 1) parts = 1;
+void wgrad(fsp_net* N, int l, int nx, int ny, int nz, const _Float16* g, const _Float16* in) {
+  using Bk = WgradBrick<CIN, COUT>;
   WgradArgs a{};
   a.nx = nx; a.ny = ny; a.nz = nz;
   a.cnx = UP ? nx / 2 : nx; a.cny = UP ? ny / 2 : ny; a.cnz = UP ? nz / 2 : nz;
-  a.g = g; a.gs = gs; a.in = in; a.partial = N->partial; a.parts = parts;
-  const size_t waves = (size_t)CH * MT * parts;
-  k_wgrad<CIN, COUT, UP><<<(unsigned)((waves + WAVES - 1) / WAVES), THREADS, 0, N->cur>>>(a);
-  const float inv = 1.0f / N->gscale;
-  k_wgrad_reduce<<<blocks_for((size_t)COUT * 27 * CIN), 256, 0, N->cur>>>(N->partial, parts, CIN, COUT, inv,
-                                                                             N->grad + N->poff[l], N->bad);
-  k_bgrad<<<COUT, 256, 0, N->cur>>>(g, (size_t)nx * ny * nz, gs, inv, N->grad + N->poff[l] + (size_t)COUT * 27 * CIN,
-                                       N->bad);
+  a.g = g; a.in = in; a.partial = N->partial;
+  const int parts = wgrad_parts<CIN, COUT>(nx, ny, nz);
+  k_wgrad<CIN, COUT, UP><<<(unsigned)parts, 64 * Bk::WV, 0, N->cur>>>(a);
+  k_wgrad_reduce<CIN, COUT><<<(unsigned)((Bk::ELEMS + 63) / 64), 1024, 0, N->cur>>>(
+      N->partial, parts, 1.0f / N->gscale, N->grad + N->poff[l], N->bad);
+}
+
+// Floats of the weight-gradient partials of the largest layer on this shape.
+size_t wgrad_floats(int X0, int Y0, int Z0) {
+  const int X1 = X0 / 2, Y1 = Y0 / 2, Z1 = Z0 / 2, X2 = X0 / 4, Y2 = Y0 / 4, Z2 = Z0 / 4;
+  size_t most = 0;
+  auto layer = [&](int parts, int elems) { most = std::max(most, (size_t)parts * elems); };
+  layer(wgrad_parts<4, 8>(X0, Y0, Z0), WgradBrick<4, 8>::ELEMS);
+  layer(wgrad_parts<8, 8>(X0, Y0, Z0), WgradBrick<8, 8>::ELEMS);
+  layer(wgrad_parts<16, 8>(X0, Y0, Z0), WgradBrick<16, 8>::ELEMS);
+  layer(wgrad_parts<8, 1>(X0, Y0, Z0), WgradBrick<8, 1>::ELEMS);
+  layer(wgrad_parts<8, 16>(X1, Y1, Z1), WgradBrick<8, 16>::ELEMS);
+  layer(wgrad_parts<16, 16>(X1, Y1, Z1), WgradBrick<16, 16>::ELEMS);
+  layer(wgrad_parts<32, 16>(X1, Y1, Z1), WgradBrick<32, 16>::ELEMS);
+  layer(wgrad_parts<16, 32>(X2, Y2, Z2), WgradBrick<16, 32>::ELEMS);
+  layer(wgrad_parts<32, 32>(X2, Y2, Z2), WgradBrick<32, 32>::ELEMS);
+  return most;
 }
 
 int lvl_n(const fsp_net* N, int level, int axis) {
@@ -1023,52 +1236,38 @@ void forward(fsp_net* N, const Acts& A) {
 
 void forward(fsp_net* N) { forward(N, net_acts(N)); }
 
-void relu_back(fsp_net* N, const _Float16* h, _Float16* g, size_t n) {
-  k_relu_back<<<blocks_for(n), 256, 0, N->cur>>>(h, g, n);
-}
-
 // Gradients of the loss (its output gradient already in N->gy) into N->grad.
 void backward(fsp_net* N) {
   hipStream_t st = N->cur;
   const int X0 = N->nx, Y0 = N->ny, Z0 = N->nz;
   const int X1 = X0 / 2, Y1 = Y0 / 2, Z1 = Z0 / 2, X2 = X0 / 4, Y2 = Y0 / 4, Z2 = Z0 / 4;
-  const size_t V0 = N->V[0], V1 = N->V[1], V2 = N->V[2];
   _Float16** g = N->gpre;
+  _Float16** act = N->act;
   // head (gradient gy: 4 channels, channel 0 used)
-  wgrad<8, 1, 0>(N, 10, X0, Y0, Z0, N->gy, N->act[9], 4);
-  conv<4, 8, 2>(st, X0, Y0, Z0, N->gy, N->wb[10], nullptr, g[9], nullptr);
-  relu_back(N, N->act[9], g[9], V0 * 8);
-  wgrad<8, 8, 0>(N, 9, X0, Y0, Z0, g[9], N->act[8]);
-  conv<8, 8, 2>(st, X0, Y0, Z0, g[9], N->wb[9], nullptr, g[8], nullptr);
-  relu_back(N, N->act[8], g[8], V0 * 8);
-  wgrad<16, 8, 1>(N, 8, X0, Y0, Z0, g[8], N->act[7]);
+  wgrad<8, 1, 0>(N, 10, X0, Y0, Z0, N->gy, act[9]);
+  conv<4, 8, 3>(st, X0, Y0, Z0, N->gy, N->wb[10], nullptr, g[9], nullptr, nullptr, act[9]);
+  wgrad<8, 8, 0>(N, 9, X0, Y0, Z0, g[9], act[8]);
+  conv<8, 8, 3>(st, X0, Y0, Z0, g[9], N->wb[9], nullptr, g[8], nullptr, nullptr, act[8]);
+  wgrad<16, 8, 1>(N, 8, X0, Y0, Z0, g[8], act[7]);
   conv<8, 16, 2>(st, X0, Y0, Z0, g[8], N->wb[8], nullptr, N->gf16, nullptr);
-  k_up_back<<<blocks_for(V1 * 16), 256, 0, st>>>(N->gf16, g[7], X1, Y1, Z1, 16);
-  relu_back(N, N->act[7], g[7], V1 * 16);
-  wgrad<16, 16, 0>(N, 7, X1, Y1, Z1, g[7], N->act[6]);
-  conv<16, 16, 2>(st, X1, Y1, Z1, g[7], N->wb[7], nullptr, g[6], nullptr);
-  relu_back(N, N->act[6], g[6], V1 * 16);
-  wgrad<32, 16, 1>(N, 6, X1, Y1, Z1, g[6], N->act[5]);
+  k_up_back<16><<<pool_grid(X1, Y1, Z1, 2), dim3(64, 4), 0, st>>>(N->gf16, act[7], g[7], X1, Y1, Z1);
+  wgrad<16, 16, 0>(N, 7, X1, Y1, Z1, g[7], act[6]);
+  conv<16, 16, 3>(st, X1, Y1, Z1, g[7], N->wb[7], nullptr, g[6], nullptr, nullptr, act[6]);
+  wgrad<32, 16, 1>(N, 6, X1, Y1, Z1, g[6], act[5]);
   conv<16, 32, 2>(st, X1, Y1, Z1, g[6], N->wb[6], nullptr, N->gf32, nullptr);
-  k_up_back<<<blocks_for(V2 * 32), 256, 0, st>>>(N->gf32, g[5], X2, Y2, Z2, 32);
-  relu_back(N, N->act[5], g[5], V2 * 32);
-  wgrad<32, 32, 0>(N, 5, X2, Y2, Z2, g[5], N->act[4]);
-  conv<32, 32, 2>(st, X2, Y2, Z2, g[5], N->wb[5], nullptr, g[4], nullptr);
-  relu_back(N, N->act[4], g[4], V2 * 32);
+  k_up_back<32><<<pool_grid(X2, Y2, Z2, 4), dim3(64, 4), 0, st>>>(N->gf32, act[5], g[5], X2, Y2, Z2);
+  wgrad<32, 32, 0>(N, 5, X2, Y2, Z2, g[5], act[4]);
+  conv<32, 32, 3>(st, X2, Y2, Z2, g[5], N->wb[5], nullptr, g[4], nullptr, nullptr, act[4]);
   wgrad<16, 32, 0>(N, 4, X2, Y2, Z2, g[4], N->p2);
   conv<32, 16, 2>(st, X2, Y2, Z2, g[4], N->wb[4], nullptr, N->gp2, nullptr);
-  k_pool_back<<<blocks_for(V1 * 16), 256, 0, st>>>(N->gp2, g[6], g[3], X1, Y1, Z1, 16);
-  relu_back(N, N->act[3], g[3], V1 * 16);
-  wgrad<16, 16, 0>(N, 3, X1, Y1, Z1, g[3], N->act[2]);
-  conv<16, 16, 2>(st, X1, Y1, Z1, g[3], N->wb[3], nullptr, g[2], nullptr);
-  relu_back(N, N->act[2], g[2], V1 * 16);
+  k_pool_back<16><<<pool_grid(X1, Y1, Z1, 2), dim3(64, 4), 0, st>>>(N->gp2, g[6], act[3], g[3], X1, Y1, Z1);
+  wgrad<16, 16, 0>(N, 3, X1, Y1, Z1, g[3], act[2]);
+  conv<16, 16, 3>(st, X1, Y1, Z1, g[3], N->wb[3], nullptr, g[2], nullptr, nullptr, act[2]);
   wgrad<8, 16, 0>(N, 2, X1, Y1, Z1, g[2], N->p1);
   conv<16, 8, 2>(st, X1, Y1, Z1, g[2], N->wb[2], nullptr, N->gp1, nullptr);
-  k_pool_back<<<blocks_for(V0 * 8), 256, 0, st>>>(N->gp1, g[8], g[1], X0, Y0, Z0, 8);
-  relu_back(N, N->act[1], g[1], V0 * 8);
-  wgrad<8, 8, 0>(N, 1, X0, Y0, Z0, g[1], N->act[0]);
-  conv<8, 8, 2>(st, X0, Y0, Z0, g[1], N->wb[1], nullptr, g[0], nullptr);
-  relu_back(N, N->act[0], g[0], V0 * 8);
+  k_pool_back<8><<<pool_grid(X0, Y0, Z0, 1), dim3(64, 4), 0, st>>>(N->gp1, g[8], act[1], g[1], X0, Y0, Z0);
+  wgrad<8, 8, 0>(N, 1, X0, Y0, Z0, g[1], act[0]);
+  conv<8, 8, 3>(st, X0, Y0, Z0, g[1], N->wb[1], nullptr, g[0], nullptr, nullptr, act[0]);
   wgrad<4, 8, 0>(N, 0, X0, Y0, Z0, g[0], N->x0);
 }
 
@@ -1098,10 +1297,7 @@ fsp_status net_reserve(fsp_net* N, int nx, int ny, int nz) {
     if (l < NL - 1 && (st = nalloc(N, &N->act[l], Vl * LAYERS[l].cout))) return st;
     if ((st = nalloc(N, &N->gpre[l], Vl * gch(LAYERS[l].cout)))) return st;
   }
-  // weight-gradient partials: up to 8192 wavefronts' worth, at least one partition per layer
-  size_t most = 0;
-  for (const LayerDesc& L : LAYERS) most = std::max(most, (size_t)npad(L.cout) * kpad(L.cin));
-  N->partial_floats = std::max(most * 64, (size_t)8192 * 256);
+  N->partial_floats = wgrad_floats(nx, ny, nz);
   if ((st = nalloc(N, &N->partial, N->partial_floats))) return st;
   N->nx = nx; N->ny = ny; N->nz = nz;
   ++N->generation;
@@ -1159,16 +1355,14 @@ fsp_status pack_all(fsp_net* N) {
 fsp_status loss_and_grad(fsp_net* N, const float* target, const uint8_t* wet, double* loss, bool* bad) {
   const size_t V = N->V[0];
   NET_HIP(hipMemsetAsync(N->bad, 0, sizeof(int), N->cur));
+  // wet count for the mean, on its way to the host while the forward pass runs
+  NET_HIP(hipMemsetAsync(N->nwet, 0, sizeof(unsigned long long), N->cur));
+  k_count_flags<<<std::min<unsigned>(256, blocks_for(V / 16 + 1)), 256, 0, N->cur>>>(wet, V, N->nwet);
+  NET_HIP(hipMemcpyAsync(N->hnwet, N->nwet, sizeof(unsigned long long), hipMemcpyDeviceToHost, N->cur));
+  NET_HIP(hipEventRecord(N->counted, N->cur));
   forward(N);
-  // wet count for the mean
-  std::vector<uint8_t> hw;
-  size_t nwet = 0;
-  {
-    hw.resize(V);
-    NET_HIP(hipMemcpyAsync(hw.data(), wet, V, hipMemcpyDeviceToHost, N->cur));
-    NET_HIP(hipStreamSynchronize(N->cur));
-    for (uint8_t b : hw) nwet += b ? 1 : 0;
-  }
+  NET_HIP(hipEventSynchronize(N->counted));
+  size_t nwet = (size_t)*N->hnwet;
   if (nwet == 0) nwet = 1;
   if (N->gscale <= 0.f) N->gscale = std::ldexp(1.0f, (int)std::lround(std::log2((double)nwet)));
   const unsigned blocks = std::min<unsigned>(4096, blocks_for(V));
@@ -1263,7 +1457,7 @@ fsp_status fsp_net_create(int32_t device, fsp_net** out) {
   }
   fsp_status st;
   if ((st = nalloc(N, &N->theta, N->P)) || (st = nalloc(N, &N->m1, N->P)) || (st = nalloc(N, &N->m2, N->P)) ||
-      (st = nalloc(N, &N->grad, N->P)) || (st = nalloc(N, &N->bad, 1)))
+      (st = nalloc(N, &N->grad, N->P)) || (st = nalloc(N, &N->bad, 1)) || (st = nalloc(N, &N->nwet, 1)))
     return fail(st);
   for (int l = 0; l < NL; ++l) {
     const LayerDesc& L = LAYERS[l];
@@ -1273,7 +1467,10 @@ fsp_status fsp_net_create(int32_t device, fsp_net** out) {
       return fail(st);
   }
   N->nparam_allocs = N->allocs.size();
-  if (hipHostMalloc((void**)&N->hbad, sizeof(int), hipHostMallocDefault) != hipSuccess) return fail(FSP_DEVICE);
+  if (hipHostMalloc((void**)&N->hbad, sizeof(int), hipHostMallocDefault) != hipSuccess ||
+      hipHostMalloc((void**)&N->hnwet, sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess ||
+      hipEventCreateWithFlags(&N->counted, hipEventDisableTiming) != hipSuccess)
+    return fail(FSP_DEVICE);
   if (hipStreamSynchronize(N->stream) != hipSuccess) return fail(FSP_DEVICE);
   *out = N;
   return FSP_OK;
@@ -1285,6 +1482,8 @@ void fsp_net_destroy(fsp_net* N) {
   if (N->stream) (void)hipStreamSynchronize(N->stream);
   free_shape(N, 0);
   if (N->hbad) (void)hipHostFree(N->hbad);
+  if (N->hnwet) (void)hipHostFree(N->hnwet);
+  if (N->counted) (void)hipEventDestroy(N->counted);
   if (N->stream) (void)hipStreamDestroy(N->stream);
   delete N;
 }

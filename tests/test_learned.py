@@ -178,6 +178,41 @@ def test_gradients_match_the_reference(net):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(64, 4, 4), (64, 12, 20), (128, 36, 12)])
+def test_gradients_on_partial_bricks_match_the_reference(net, shape):
+    """Every layer's gradient where the weight gradient's bricks (16 x 8 x 8 or
+    4 cells) lie partly outside the grid: a single row and plane at level 2,
+    and more bricks than fit the grid's edges. Each layer within 5e-2 relative
+    L2: binary16 gradients and activations are off by up to 11 layers of
+    2^-11 = 5e-3, and on the smallest grid a ReLU whose input rounds to the
+    other side of zero moves a layer by about 1e-2; a row, plane or tap read
+    from the wrong place is an error of order one."""
+    t = _t()
+    rng = np.random.default_rng(17)
+    th = nr.init(18).astype(np.float32)
+    th[np.arange(th.size) % 5 == 0] += 0.01
+    net.set_params(th)
+    nx, ny, nz = shape
+    x16, wet = random_features(rng, nz, ny, nx)
+    target = (rng.standard_normal((nz, ny, nx)) * wet).astype(np.float32)
+    # flags from an address that is not 16-byte aligned
+    flags = t.zeros(wet.size + 3, dtype=t.uint8, device="cuda")
+    flags[3:] = t.from_numpy(wet.ravel().astype(np.uint8)).cuda()
+    loss, g = net.loss_grad(f16_tensor(x16), t.from_numpy(target.ravel()).cuda(), flags[3:], shape)
+    lr, gr, _ = nr.loss_and_grad(th.astype(np.float64), x16.astype(np.float64), target.astype(np.float64),
+                                 wet.astype(np.float64), round16=True)
+    assert abs(loss - lr) <= 1e-2 * lr
+    off = 0
+    for name, level, ci, co, relu, skip in nr.LAYERS:
+        for part, n in (("W", co * 27 * ci), ("b", co)):
+            a, b = g[off:off + n], gr[off:off + n]
+            err = np.linalg.norm(a - b) / np.linalg.norm(b)
+            print(f"{shape} {name}.{part}: {err:.2e}")
+            assert err <= 5e-2, (name, part)
+            off += n
+
+
+@pytest.mark.gpu
 def test_training_steps_reduce_the_loss(net):
     t = _t()
     rng = np.random.default_rng(9)
