@@ -1644,13 +1644,20 @@ fsp_status fsp_create(const fsp_domain* d, const fsp_options* o, fsp_solver** ou
     return fail(FSP_INVALID);
   if (opt.preconditioner != FSP_PRECOND_JACOBI && quad_vcycle_ok(S->quad, opt) && (st = dalloc(S, &S->precv, S->n)))
     return fail(st);
+  // dynamic LDS a workgroup may have (160 KiB on gfx950)
+  int lds_attr = 0;
+  if (hipDeviceGetAttribute(&lds_attr, hipDeviceAttributeMaxSharedMemoryPerBlock, opt.device) != hipSuccess)
+    return fail(FSP_DEVICE);
+  const size_t lds_limit = std::max<size_t>((size_t)lds_attr, 65536);
   S->tail_first = (int)S->levels.size();
   for (int t = (int)S->levels.size() - 1; t >= 0; --t) {
-    if (S->levels[t].n > 4096 || (int)S->levels.size() - t > TAIL_MAX_LEVELS) break;
+    if (S->levels[t].n > (size_t)TAIL_CELLS || (int)S->levels.size() - t > TAIL_MAX_LEVELS) break;
     const int count = (int)S->levels.size() - t;
     const size_t bytes = gc_tail_ok(opt) ? gc_tail_lds_bytes(&S->levels[t], count)
                                          : tail_lds_bytes(&S->levels[t], count, opt.smoother);
-    if (bytes > TAIL_LDS_FLOATS * sizeof(float)) break;
+    if (bytes > (gc_tail_ok(opt) ? std::min(GC_TAIL_LDS_FLOATS * sizeof(float), lds_limit - TAIL_STATIC_LDS)
+                                 : TAIL_LDS_FLOATS * sizeof(float)))
+      break;
     S->tail_first = t;
     S->tail_lds = bytes;
   }

@@ -590,6 +590,8 @@ struct GcTailLvl {
   int o_x, o_r, o_fx, o_fy, o_fz, o_dd;
 };
 
+constexpr size_t TAIL_STATIC_LDS = 1024;  // reserved beside the tail's dynamic LDS
+
 // Float offset of level l's coupling block in the pack (and in LDS).
 __host__ __device__ inline size_t gct_pack_offset(const TailSet& T, int l) {
   size_t off = 0;
@@ -756,6 +758,70 @@ __device__ __forceinline__ void gct_coarsest_wave(float* lds, const GcTailLvl& L
   __syncthreads();
 }
 
+// The passes of a level with even rows and at most 4096 cells, each thread's
+// cells in registers: two of each colour (pairs q = thread, thread + 1024;
+// a pair holds one cell of each colour), with their couplings, Dirichlet part,
+// diagonal and r loaded once for the whole sequence, so that a pass reads
+// only the six neighbours from LDS. A neighbour index past the level's edge
+// reads another array of the workgroup's LDS (x lies between the couplings
+// and r, both at least a plane long); its coupling is zero and the row
+// leaves it out. Per cell the arithmetic of gct_pass, in the same order.
+template <int ST>
+struct GctCells {
+  using SV = Store<ST>;
+  static constexpr int S = 2;  // pairs per thread
+  float a[2][S][6], dd[2][S], dg[2][S], r[2][S];
+  int c[2][S];  // -1: no cell
+
+  __device__ __forceinline__ void load(const float* lds, const GcTailLvl& L) {
+#pragma clang fp contract(off)
+    const int hx = L.nx >> 1, m = L.n >> 1;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int q = (int)threadIdx.x + s * TAIL_THREADS;
+      const int row = (int)(((float)q + 0.5f) * L.rhx);
+      const int u = q - row * hx;
+      const int k = (int)(((float)row + 0.5f) * L.rny);
+      const int j = row - k * L.ny;
+#pragma unroll
+      for (int col = 0; col < 2; ++col) {
+        const int i = 2 * u + ((col + j + k) & 1);
+        c[col][s] = -1;
+        if (q >= m) continue;
+        const int cc = row * L.nx + i;
+        c[col][s] = cc;
+        gct_faces(lds, L, i, j, k, cc, a[col][s]);
+        dd[col][s] = lds[L.o_dd + cc];
+        r[col][s] = lds[L.o_r + cc];
+        dg[col][s] = gc_diag(a[col][s], dd[col][s], L.inv);
+      }
+    }
+  }
+  // One colour; first: x starts at zero.
+  template <int COL>
+  __device__ __forceinline__ void pass(float* lds, const GcTailLvl& L, bool first) {
+#pragma clang fp contract(off)
+    float* x = lds + L.o_x;
+    const int plane = L.nx * L.ny;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int cc = c[COL][s];
+      if (cc < 0) continue;
+      const float d = dg[COL][s];
+      if (first) {
+        x[cc] = d > 0.f ? SV::rnd(r[COL][s] / d) : 0.f;
+        x[cc ^ 1] = 0.f;  // the pair's other cell (row * nx is even)
+        continue;
+      }
+      if (!(d > 0.f)) continue;
+      const float nb[6] = {x[cc - 1], x[cc + 1], x[cc - L.nx], x[cc + L.nx], x[cc - plane], x[cc + plane]};
+      const float xc = x[cc];
+      x[cc] = SV::rnd(xc + (r[COL][s] - gc_row(a[COL][s], dd[COL][s], L.inv, xc, nb)) / d);
+    }
+    __syncthreads();
+  }
+};
+
 template <int ST>
 __device__ __forceinline__ void gct_sweeps(float* lds, const GcTailLvl& L, int count, bool forward, bool coarsest,
                                            bool from_zero) {
@@ -771,8 +837,37 @@ __device__ __forceinline__ void gct_sweeps(float* lds, const GcTailLvl& L, int c
     gct_coarsest_wave<ST>(lds, L, count, from_zero);
     return;
   }
+  const int half = coarsest ? count / 2 : 0;
+  if ((L.nx & 1) == 0 && L.n <= 2 * GctCells<ST>::S * TAIL_THREADS) {
+    GctCells<ST> cells;
+    cells.load(lds, L);
+    if (coarsest) {
+      for (int s = 0; s < half; ++s) {
+        cells.template pass<0>(lds, L, fz);
+        fz = false;
+        cells.template pass<1>(lds, L, false);
+      }
+      if (count & 1) { cells.template pass<0>(lds, L, fz); fz = false; }
+      for (int s = 0; s < half; ++s) {
+        cells.template pass<1>(lds, L, false);
+        cells.template pass<0>(lds, L, false);
+      }
+    } else if (forward) {
+      for (int s = 0; s < count; ++s) {
+        cells.template pass<0>(lds, L, fz);
+        fz = false;
+        cells.template pass<1>(lds, L, false);
+      }
+    } else {
+      for (int s = 0; s < count; ++s) {
+        cells.template pass<1>(lds, L, fz);
+        fz = false;
+        cells.template pass<0>(lds, L, false);
+      }
+    }
+    return;
+  }
   if (coarsest) {
-    const int half = count / 2;
     for (int s = 0; s < half; ++s) { gct_pass<ST>(lds, L, 0, fz); fz = false; gct_pass<ST>(lds, L, 1, false); }
     if (count & 1) { gct_pass<ST>(lds, L, 0, fz); fz = false; }
     for (int s = 0; s < half; ++s) { gct_pass<ST>(lds, L, 1, fz); fz = false; gct_pass<ST>(lds, L, 0, false); }
@@ -836,6 +931,7 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_gc_tail(TailSet T, Ctl* ctl) {
   if (!ctl->active) return;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   __shared__ GcTailLvl tl[TAIL_MAX_LEVELS];
+  static_assert(sizeof(tl) <= TAIL_STATIC_LDS, "static LDS of the tail");
   int total = 0;  // cells of all tail levels
   for (int l = 0; l < T.count; ++l) total += (int)T.lv[l].n;
   if (threadIdx.x == 0) {
@@ -858,19 +954,20 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_gc_tail(TailSet T, Ctl* ctl) {
   {
     const float4* src = reinterpret_cast<const float4*>(T.pack);
     float4* dst = reinterpret_cast<float4*>(lds);
-    constexpr int MAXQ = (TAIL_LDS_FLOATS / 6 + TAIL_THREADS - 1) / TAIL_THREADS;  // float4s per thread
+    constexpr int MAXQ = (GC_TAIL_LDS_FLOATS / 6 + TAIL_THREADS - 1) / TAIL_THREADS;  // float4s per thread
     float4 v[MAXQ];
 #pragma unroll
     for (int u = 0; u < MAXQ; ++u) {
       const int q = (int)threadIdx.x + u * TAIL_THREADS;
       v[u] = q < total ? src[q] : f4zero();
     }
-    const int c0 = (int)threadIdx.x;
-    const float r0 = c0 < (int)T.lv[0].n ? SV::ld(reinterpret_cast<const typename SV::T*>(T.lv[0].r), c0) : 0.f;
-    const float r1 = c0 + TAIL_THREADS < (int)T.lv[0].n
-                         ? SV::ld(reinterpret_cast<const typename SV::T*>(T.lv[0].r), c0 + TAIL_THREADS) : 0.f;
-    const float r2 = c0 + 2 * TAIL_THREADS < (int)T.lv[0].n
-                         ? SV::ld(reinterpret_cast<const typename SV::T*>(T.lv[0].r), c0 + 2 * TAIL_THREADS) : 0.f;
+    constexpr int RQ = (TAIL_CELLS + TAIL_THREADS - 1) / TAIL_THREADS;
+    float rv[RQ];
+#pragma unroll
+    for (int u = 0; u < RQ; ++u) {
+      const int q = (int)threadIdx.x + u * TAIL_THREADS;
+      rv[u] = q < (int)T.lv[0].n ? SV::ld(reinterpret_cast<const typename SV::T*>(T.lv[0].r), q) : 0.f;
+    }
 #pragma unroll
     for (int u = 0; u < MAXQ; ++u) {
       const int q = (int)threadIdx.x + u * TAIL_THREADS;
@@ -878,9 +975,11 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_gc_tail(TailSet T, Ctl* ctl) {
     }
     __syncthreads();  // tl
     const int orr = tl[0].o_r, n0 = tl[0].n;
-    if (c0 < n0) lds[orr + c0] = r0;
-    if (c0 + TAIL_THREADS < n0) lds[orr + c0 + TAIL_THREADS] = r1;
-    if (c0 + 2 * TAIL_THREADS < n0) lds[orr + c0 + 2 * TAIL_THREADS] = r2;
+#pragma unroll
+    for (int u = 0; u < RQ; ++u) {
+      const int q = (int)threadIdx.x + u * TAIL_THREADS;
+      if (q < n0) lds[orr + q] = rv[u];
+    }
   }
   __syncthreads();
   const int last = T.count - 1;
@@ -908,6 +1007,5 @@ inline size_t gc_tail_lds_bytes(const Level* lv, int count) {
   for (int l = 0; l < count; ++l) floats += 6 * lv[l].n;
   return floats * sizeof(float);
 }
-static_assert(TAIL_LDS_FLOATS / 6 <= 3 * TAIL_THREADS, "the first tail level's r in three loads per thread");
 
 }  // namespace fsp
