@@ -327,14 +327,23 @@ __device__ void full_row(const Fine& G, int i, int j, int k, RowG& R) {
 template <class T>
 __device__ __forceinline__ float ldv(const T* p, size_t i) { return (float)p[i]; }
 
+// The entry of layer k in a column's table of ghost rows. A column's table
+// covers G_SLOTS layers from its lowest ghost row (gk0), so the layer modulo
+// G_SLOTS names the entry without a look at gk0: one round of memory latency
+// less where every ghost row is known to lie in its table.
+__device__ __forceinline__ const float* ghost_entry(const Fine& G, size_t col, int k) {
+  return G.gtab + (col * G_SLOTS + (size_t)(k & (G_SLOTS - 1))) * 8;
+}
+static_assert((G_SLOTS & (G_SLOTS - 1)) == 0, "layer modulo G_SLOTS");
+
 // 1/theta of the six faces of a ghost row, from the per-column table built
 // once per projection (k_ghost_table); false if the row is outside the
 // column's table, in which case the caller derives it from the geometry.
 __device__ __forceinline__ bool ghost_its(const Fine& G, int i, int j, int k, float it[6]) {
   const size_t col = (size_t)j * G.nx + i;
-  const int slot = k - (int)G.gk0[col];
-  if (slot < 0 || slot >= G_SLOTS) return false;
-  const float* e = G.gtab + (col * G_SLOTS + slot) * 8;
+  const int d = k - (int)G.gk0[col];
+  if (d < 0 || d >= G_SLOTS) return false;
+  const float* e = ghost_entry(G, col, k);
   const float4 a = *reinterpret_cast<const float4*>(e);
   const float2 b = *reinterpret_cast<const float2*>(e + 4);
   it[0] = a.x; it[1] = a.y; it[2] = a.z; it[3] = a.w; it[4] = b.x; it[5] = b.y;
@@ -351,17 +360,18 @@ __device__ __forceinline__ bool ghost_its(const Fine& G, int i, int j, int k, fl
 template <bool GEN = true>
 __device__ __forceinline__ void ghost_row(const Fine& G, int i, int j, int k, uint8_t m, uint8_t type[6], float it[6],
                                           float a[6]) {
-  if (!G.frac && !G.phi && ghost_its(G, i, j, k, it)) {
+  if (!GEN) {
+    const float* e = ghost_entry(G, (size_t)j * G.nx + i, k);
+    const float4 lo = *reinterpret_cast<const float4*>(e);
+    const float2 hi = *reinterpret_cast<const float2*>(e + 4);
+    it[0] = lo.x; it[1] = lo.y; it[2] = lo.z; it[3] = lo.w; it[4] = hi.x; it[5] = hi.y;
+  }
+  if (!GEN || (!G.frac && !G.phi && ghost_its(G, i, j, k, it))) {
 #pragma unroll
     for (int f = 0; f < 6; ++f) {
       type[f] = (m & (1u << f)) ? 1 : (it[f] > 0.f ? 2 : 0);
       a[f] = 1.0f;
     }
-    return;
-  }
-  if (!GEN) {
-#pragma unroll
-    for (int f = 0; f < 6; ++f) { type[f] = 0; it[f] = 0.f; a[f] = 0.f; }
     return;
   }
   RowG R;
@@ -604,7 +614,7 @@ __global__ void __launch_bounds__(BLOCK) k_ghost_table(Fine G, uint16_t* gk0, fl
     for (int s = 0; s < G_SLOTS; ++s) ms[s] = k0 + s < G.nz ? G.mask[(size_t)(k0 + s) * plane + col] : 0;
     for (int s = 0; s < G_SLOTS && k0 + s < G.nz; ++s) {
       const int k = k0 + s;
-      float* e = gtab + (col * G_SLOTS + s) * 8;
+      float* e = gtab + (col * G_SLOTS + (size_t)(k & (G_SLOTS - 1))) * 8;
       float it[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       if (ms[s] & M_GHOST) {
         RowG R;

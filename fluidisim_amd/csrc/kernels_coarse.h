@@ -837,47 +837,28 @@ __device__ __forceinline__ void gct_sweeps(float* lds, const GcTailLvl& L, int c
     gct_coarsest_wave<ST>(lds, L, count, from_zero);
     return;
   }
-  const int half = coarsest ? count / 2 : 0;
+  // the colours of the sequence: red-black forward, black-red backward, or on
+  // the coarsest level the palindrome of both halves
+  const int half = coarsest ? count / 2 : 0, odd = coarsest ? count & 1 : 0;
+  const int passes = coarsest ? 4 * half + odd : 2 * count;
+  auto colour = [&](int i) -> int {
+    if (!coarsest) return forward ? (i & 1) : 1 - (i & 1);
+    if (i < 2 * half + odd) return i & 1;
+    return 1 - ((i - 2 * half - odd) & 1);
+  };
   if ((L.nx & 1) == 0 && L.n <= 2 * GctCells<ST>::S * TAIL_THREADS) {
     GctCells<ST> cells;
     cells.load(lds, L);
-    if (coarsest) {
-      for (int s = 0; s < half; ++s) {
-        cells.template pass<0>(lds, L, fz);
-        fz = false;
-        cells.template pass<1>(lds, L, false);
-      }
-      if (count & 1) { cells.template pass<0>(lds, L, fz); fz = false; }
-      for (int s = 0; s < half; ++s) {
-        cells.template pass<1>(lds, L, false);
-        cells.template pass<0>(lds, L, false);
-      }
-    } else if (forward) {
-      for (int s = 0; s < count; ++s) {
-        cells.template pass<0>(lds, L, fz);
-        fz = false;
-        cells.template pass<1>(lds, L, false);
-      }
-    } else {
-      for (int s = 0; s < count; ++s) {
-        cells.template pass<1>(lds, L, fz);
-        fz = false;
-        cells.template pass<0>(lds, L, false);
-      }
+    for (int i = 0; i < passes; ++i) {
+      if (colour(i) == 0) cells.template pass<0>(lds, L, fz);
+      else cells.template pass<1>(lds, L, fz);
+      fz = false;
     }
     return;
   }
-  if (coarsest) {
-    for (int s = 0; s < half; ++s) { gct_pass<ST>(lds, L, 0, fz); fz = false; gct_pass<ST>(lds, L, 1, false); }
-    if (count & 1) { gct_pass<ST>(lds, L, 0, fz); fz = false; }
-    for (int s = 0; s < half; ++s) { gct_pass<ST>(lds, L, 1, fz); fz = false; gct_pass<ST>(lds, L, 0, false); }
-    return;
-  }
-  for (int s = 0; s < count; ++s) {
-    const int c0 = forward ? 0 : 1;
-    gct_pass<ST>(lds, L, c0, fz);
+  for (int i = 0; i < passes; ++i) {
+    gct_pass<ST>(lds, L, colour(i), fz);
     fz = false;
-    gct_pass<ST>(lds, L, 1 - c0, false);
   }
 }
 
@@ -982,20 +963,16 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_gc_tail(TailSet T, Ctl* ctl) {
     }
   }
   __syncthreads();
+  // down to the coarsest level and back up
   const int last = T.count - 1;
-  for (int l = 0; l <= last; ++l) {
+  for (int step = 0; step <= 2 * last; ++step) {
+    const bool down = step <= last;
+    const int l = down ? step : 2 * last - step;
     // level descriptors in registers: the passes do not reload them after each barrier
     const GcTailLvl L = tl[l];
-    gct_sweeps<ST>(lds, L, l == last ? T.coarse : T.pre, true, l == last, true);
-    if (l < last) {
-      const GcTailLvl C = tl[l + 1];
-      gct_restrict<ST>(lds, L, C);
-    }
-  }
-  for (int l = last - 1; l >= 0; --l) {
-    const GcTailLvl L = tl[l], C = tl[l + 1];
-    gct_prolong<ST>(lds, L, C);
-    gct_sweeps<ST>(lds, L, T.post, false, false, false);
+    if (!down) gct_prolong<ST>(lds, L, tl[l + 1]);
+    gct_sweeps<ST>(lds, L, l == last ? T.coarse : down ? T.pre : T.post, down, l == last, down);
+    if (l < last && down) gct_restrict<ST>(lds, L, tl[l + 1]);
   }
   const GcTailLvl L0 = tl[0];
   for (int q = threadIdx.x; q < L0.n; q += TAIL_THREADS)

@@ -98,6 +98,77 @@ __device__ __forceinline__ float row_local(const Fine& G, int i, int j, int k, u
   return acc * G.inv;
 }
 
+// A plain row's sum over its coupled faces (row code m), branch-free.
+__device__ __forceinline__ float plain_sum(uint32_t m, float pc, const float nb[6]) {
+#pragma clang fp contract(off)
+  float acc = 0.f;
+#pragma unroll
+  for (int f = 0; f < 6; ++f) acc = (m & (1u << f)) ? acc + (pc - nb[f]) : acc;
+  return acc;
+}
+// ghost_row_sum from a table entry (binary apertures).
+struct GhostEntry {
+  float4 a;
+  float2 b;
+};
+__device__ __forceinline__ GhostEntry ghost_load(const Fine& G, size_t col, int k) {
+  const float* e = ghost_entry(G, col, k);
+  return {*reinterpret_cast<const float4*>(e), *reinterpret_cast<const float2*>(e + 4)};
+}
+__device__ __forceinline__ float ghost_sum(const GhostEntry& g, uint32_t m, float pc, const float nb[6], float inv,
+                                           float& prec) {
+#pragma clang fp contract(off)
+  const float it[6] = {g.a.x, g.a.y, g.a.z, g.a.w, g.b.x, g.b.y};
+  float acc = 0.f, diag = 0.f;
+#pragma unroll
+  for (int f = 0; f < 6; ++f) {
+    const bool one = (m & (1u << f)) != 0, two = !one && it[f] > 0.f;
+    const float t = one ? pc - nb[f] : pc * it[f], d = one ? 1.0f : it[f];
+    acc = (one || two) ? acc + t : acc;
+    diag = (one || two) ? diag + d : diag;
+  }
+  prec = diag > 0.f ? 1.0f / (diag * inv) : 0.f;
+  return acc;
+}
+
+// The rows (A x)_c of a quad's four cells from values in registers: zc and
+// its x neighbours left and right, ym .. zp the quads around it. The plain
+// rows first, without branches; a quad with free-surface rows then loads the
+// four cells' table entries in one round (a row at a time, each after a look
+// at its column, held a wavefront for up to eight rounds of memory latency,
+// which a small grid has nothing to hide behind).
+template <bool GEN>
+__device__ __forceinline__ void quad_rows(const Fine& G, int x0, int y, int k, uint32_t mq, const float4& zc, float left,
+                                          float right, const float4& ym, const float4& yp, const float4& zm,
+                                          const float4& zp, float row[4]) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t m = (mq >> (8 * e)) & 0xFFu;
+    const float nb[6] = {e == 0 ? left : q_get(zc, e - 1), e == 3 ? right : q_get(zc, e + 1),
+                         q_get(ym, e), q_get(yp, e), q_get(zm, e), q_get(zp, e)};
+    row[e] = (m & M_WET) ? plain_sum(m, q_get(zc, e), nb) * G.inv : 0.f;
+  }
+  const uint32_t ghosts = mq & 0x80808080u;
+  if (!ghosts) return;
+  GhostEntry g[4];
+  if (!GEN) {
+    const size_t col = (size_t)y * G.nx + x0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) g[e] = ghost_load(G, col + e, k);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (!(ghosts & (0x80u << (8 * e)))) continue;
+    const uint32_t m = (mq >> (8 * e)) & 0xFFu;
+    const float pc = q_get(zc, e);
+    const float nb[6] = {e == 0 ? left : q_get(zc, e - 1), e == 3 ? right : q_get(zc, e + 1),
+                         q_get(ym, e), q_get(yp, e), q_get(zm, e), q_get(zp, e)};
+    float prec;
+    row[e] = GEN ? row_local<GEN>(G, x0 + e, y, k, (uint8_t)m, pc, nb, prec) : ghost_sum(g[e], m, pc, nb, G.inv, prec) * G.inv;
+  }
+}
+
 // The four cells' x neighbours: within the quad, from the adjacent lanes, or
 // (at the edge of a lane segment) from memory through `edge`.
 // Every lane takes part in the shuffles; only valid lanes read memory.
@@ -249,19 +320,36 @@ __global__ void __launch_bounds__(QBLOCK, FSP_QGS_MIN_BLOCKS) k_q_gs_first(Fine 
     return first(4 * qx + off, y, k, G.precv[c], r[c]);
   });
   if (!valid) return;
-  float4 out = zc;
+  // the colour-1 cells: x-cells par and par + 2, par = 1 on even rows
+  const bool odd = ((y + k) & 1) == 0;
+  auto sel = [odd](float o, float e) -> float { return odd ? o : e; };
+  const uint32_t m2[2] = {(mq >> (odd ? 8 : 0)) & 0xFFu, (mq >> (odd ? 24 : 16)) & 0xFFu};
+  const float pc2[2] = {sel(zc.y, zc.x), sel(zc.w, zc.z)}, r2[2] = {sel(rq.y, rq.x), sel(rq.w, rq.z)};
+  const float nb2[2][6] = {{sel(zc.x, left), sel(zc.z, zc.y), sel(ym.y, ym.x), sel(yp.y, yp.x), sel(zm.y, zm.x), sel(zp.y, zp.x)},
+                           {sel(zc.z, zc.y), sel(right, zc.w), sel(ym.w, ym.z), sel(yp.w, yp.z), sel(zm.w, zm.z), sel(zp.w, zp.z)}};
+  float v2[2];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    if (((e + y + k) & 1) != 1) continue;
-    const uint8_t m = (uint8_t)(mq >> (8 * e));
-    const float pc = q_get(zc, e);
-    const float xl = e == 0 ? left : q_get(zc, e - 1);
-    const float xr = e == 3 ? right : q_get(zc, e + 1);
-    const float nb[6] = {xl, xr, q_get(ym, e), q_get(yp, e), q_get(zm, e), q_get(zp, e)};
-    float prec;
-    const float az = row_local<GEN>(G, 4 * qx + e, y, k, m, pc, nb, prec);
-    if (prec > 0.f) q_set(out, e, SV::rnd(pc + prec * (q_get(rq, e) - az)));
+  for (int h = 0; h < 2; ++h) {
+    const float prec = (m2[h] & M_WET) ? G.prec_tab[__popc(m2[h] & 0x3Fu)] : 0.f;
+    v2[h] = prec > 0.f ? SV::rnd(pc2[h] + prec * (r2[h] - plain_sum(m2[h], pc2[h], nb2[h]) * G.inv)) : pc2[h];
   }
+  if ((m2[0] | m2[1]) & M_GHOST) {
+    GhostEntry g[2];
+    const size_t col = (size_t)y * G.nx + 4 * qx + (odd ? 1 : 0);
+    if (!GEN) {
+      g[0] = ghost_load(G, col, k);
+      g[1] = ghost_load(G, col + 2, k);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (!(m2[h] & M_GHOST)) continue;
+      float prec, az;
+      if (GEN) az = row_local<GEN>(G, 4 * qx + (odd ? 1 : 0) + 2 * h, y, k, (uint8_t)m2[h], pc2[h], nb2[h], prec);
+      else az = ghost_sum(g[h], m2[h], pc2[h], nb2[h], G.inv, prec) * G.inv;
+      v2[h] = prec > 0.f ? SV::rnd(pc2[h] + prec * (r2[h] - az)) : pc2[h];
+    }
+  }
+  const float4 out = make_float4(sel(zc.x, v2[0]), sel(v2[0], zc.y), sel(zc.z, v2[1]), sel(v2[1], zc.w));
   SV::st4(zout, c0, out);
 }
 
@@ -436,18 +524,38 @@ __global__ void __launch_bounds__(BR_THREADS) k_q_brick(Fine G, BrickGrid B, con
     late = ((ma & M_GHOST) ? (odd ? 2u : 1u) : 0u) | ((mb & M_GHOST) ? (odd ? 8u : 4u) : 0u);
     return make_float4(sel(zc.x, a), sel(a, zc.y), sel(zc.z, b), sel(b, zc.w));
   };
-  // A free-surface cell e of that quad: row_local's ghost form (per-column
-  // table, else the geometry), neighbours from LDS.
-  auto relax_late = [&](int lq, int ly, int lz, int e) -> float {
+  // The free-surface cells of colour col in that quad (up to two, flagged in
+  // `bits` as relax flags them): row_local's ghost form with neighbours from LDS, both
+  // cells' r, row codes and table entries in one round of loads. v: the two
+  // colour cells' values, changed where flagged.
+  auto relax_late = [&](int lq, int ly, int lz, int col, uint32_t bits, float v[2]) {
     const int q = qx0 + lq, y = y0 + ly, k = z0 + lz;
-    const size_t c = ((size_t)k * ny + y) * nx + 4 * (size_t)q + e;
-    const float* sc = zs + ((lz * BR_LY + ly) * BR_LX + 4 * lq + e);
-    const float nb[6] = {(q > 0 || e > 0) ? sc[-1] : 0.f, (q + 1 < nq || e < 3) ? sc[1] : 0.f, sc[-BR_LX],
-                         sc[BR_LX], sc[-BR_LX * BR_LY], sc[BR_LX * BR_LY]};
-    const float pc = sc[0];
-    float prec;
-    const float az = row_local<GEN>(G, 4 * q + e, y, k, G.mask[c], pc, nb, prec);
-    return prec > 0.f ? SV::rnd(pc + prec * (r[c] - az)) : (MODE == 2 ? 0.f : pc);
+    const int par = (col + y + k) & 1;
+    const size_t c = ((size_t)k * ny + y) * nx + 4 * (size_t)q + par;
+    const size_t column = (size_t)y * nx + 4 * (size_t)q + par;
+    uint32_t m2[2];
+    float r2[2];
+    GhostEntry g[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      m2[h] = G.mask[c + 2 * h];
+      r2[h] = r[c + 2 * h];
+      if (!GEN) g[h] = ghost_load(G, column + 2 * h, k);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int e = par + 2 * h;
+      const float* sc = zs + ((lz * BR_LY + ly) * BR_LX + 4 * lq + e);
+      const float pc = sc[0];
+      v[h] = pc;
+      if (!(bits & (1u << e))) continue;
+      const float nb[6] = {(q > 0 || e > 0) ? sc[-1] : 0.f, (q + 1 < nq || e < 3) ? sc[1] : 0.f, sc[-BR_LX],
+                           sc[BR_LX], sc[-BR_LX * BR_LY], sc[BR_LX * BR_LY]};
+      float prec, az;
+      if (GEN) az = row_local<GEN>(G, 4 * q + e, y, k, (uint8_t)m2[h], pc, nb, prec);
+      else az = ghost_sum(g[h], m2[h], pc, nb, G.inv, prec) * G.inv;
+      v[h] = prec > 0.f ? SV::rnd(pc + prec * (r2[h] - az)) : (MODE == 2 ? 0.f : pc);
+    }
   };
   __syncthreads();
   // pass c over the brick and its ring (LDS rows 1..BR_Y+2, planes 1..BR_Z+2, every LDS quad)
@@ -463,11 +571,17 @@ __global__ void __launch_bounds__(BR_THREADS) k_q_brick(Fine G, BrickGrid B, con
       *reinterpret_cast<float4*>(zs + ((lz * BR_LY + ly) * BR_LX + 4 * lq)) = o;
       late |= lt << (4 * m);
     }
-    for (; late; late &= late - 1) {
-      const int bit = __ffs(late) - 1, m = bit >> 2, e = bit & 3;
+    while (late) {
+      const int m = (__ffs(late) - 1) >> 2;
+      const uint32_t bits = (late >> (4 * m)) & 0xFu;
+      late &= ~(0xFu << (4 * m));
       const int idx = tid + BR_THREADS * m;
       const int lq = idx % BR_LQ, rest = idx / BR_LQ, ly = 1 + rest % (BR_Y + 2), lz = 1 + rest / (BR_Y + 2);
-      zs[(lz * BR_LY + ly) * BR_LX + 4 * lq + e] = relax_late(lq, ly, lz, e);
+      float v[2];
+      relax_late(lq, ly, lz, colour, bits, v);
+      float* dst = zs + (lz * BR_LY + ly) * BR_LX + 4 * lq + ((colour + y0 + ly + z0 + lz) & 1);
+      dst[0] = v[0];
+      dst[2] = v[1];
     }
   }
   __syncthreads();
@@ -490,14 +604,22 @@ __global__ void __launch_bounds__(BR_THREADS) k_q_brick(Fine G, BrickGrid B, con
       ob[m] = relax(lq, ly, lz, 1 - colour, rqb[m], mqb[m], lt);
       late |= lt << (4 * m);
     }
-    for (; late; late &= late - 1) {
-      const int bit = __ffs(late) - 1, m = bit >> 2, e = bit & 3;
+    while (late) {
+      const int m = (__ffs(late) - 1) >> 2;
+      const uint32_t bits = (late >> (4 * m)) & 0xFu;
+      late &= ~(0xFu << (4 * m));
       const int idx = tid + BR_THREADS * m;
       const int lq = 1 + idx % BR_QX, rest = idx / BR_QX, ly = 2 + rest % BR_Y, lz = 2 + rest / BR_Y;
-      const float x = relax_late(lq, ly, lz, e);
+      float v[2];
+      relax_late(lq, ly, lz, 1 - colour, bits, v);
 #pragma unroll
-      for (int mm = 0; mm < BR_BITEMS; ++mm)
-        if (mm == m) q_set(ob[mm], e, x);
+      for (int mm = 0; mm < BR_BITEMS; ++mm) {
+        if (mm != m) continue;
+        if (bits & 1u) ob[mm].x = v[0];
+        if (bits & 2u) ob[mm].y = v[0];
+        if (bits & 4u) ob[mm].z = v[1];
+        if (bits & 8u) ob[mm].w = v[1];
+      }
     }
 #pragma unroll
     for (int m = 0; m < BR_BITEMS; ++m) {
@@ -1040,17 +1162,11 @@ __global__ void __launch_bounds__(QBLOCK) k_q_restrict2(Fine G, QuadGrid H, cons
     }
     float left, right;
     x_neighbours(H, valid, qx, zc, left, right, [&](int off) { return SV::ld(z, c0 + off); });
+    // (invalid lanes: mq = 0, every row 0)
+    float row[4];
+    quad_rows<GEN>(G, 4 * qx, y, k, mq, zc, left, right, ym, yp, zm, zp, row);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const uint8_t m = (uint8_t)(mq >> (8 * e));
-      const float pc = q_get(zc, e);
-      const float xl = e == 0 ? left : q_get(zc, e - 1);
-      const float xr = e == 3 ? right : q_get(zc, e + 1);
-      const float nb[6] = {xl, xr, q_get(ym, e), q_get(yp, e), q_get(zm, e), q_get(zp, e)};
-      float prec;
-      const float az = valid ? row_local<GEN>(G, 4 * qx + e, y, k, m, pc, nb, prec) : 0.f;
-      t[dy][e] = q_get(rq, e) - az;
-    }
+    for (int e = 0; e < 4; ++e) t[dy][e] = q_get(rq, e) - row[e];
   }
   float2 sum = make_float2(0.f, 0.f);
   if (dz == 0) {
@@ -1125,17 +1241,9 @@ __global__ void __launch_bounds__(QBLOCK) k_q_spmv_dir(Fine G, QuadGrid Q, const
   });
   double s = 0.0, unused = 0.0;
   if (valid) {
-    float4 qo;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const uint8_t m = (uint8_t)(mq >> (8 * e));
-      const float pc = q_get(dc, e);
-      const float xl = e == 0 ? left : q_get(dc, e - 1);
-      const float xr = e == 3 ? right : q_get(dc, e + 1);
-      const float nb[6] = {xl, xr, q_get(ym, e), q_get(yp, e), q_get(zm, e), q_get(zp, e)};
-      float prec;
-      q_set(qo, e, row_local<GEN>(G, 4 * qx + e, y, k, m, pc, nb, prec));
-    }
+    float row[4];
+    quad_rows<GEN>(G, 4 * qx, y, k, mq, dc, left, right, ym, yp, zm, zp, row);
+    const float4 qo = make_float4(row[0], row[1], row[2], row[3]);
     st4(dnew, c0, dc);
     st4(q, c0, qo);
     s = (double)dc.x * qo.x + (double)dc.y * qo.y + (double)dc.z * qo.z + (double)dc.w * qo.w;
