@@ -59,7 +59,15 @@ struct Ctl {
   double rr_replaced;    // |r|^2 of the last replaced true residual of the pass
   uint32_t wet_cells, ghost_faces;
   int32_t table_miss;    // a ghost row lies past its column's table: the general fine kernels run
-  uint32_t counters[NUM_SLOTS];
+  uint32_t pass;         // number of the pass (Progress)
+};
+
+// Progress of the CG loop, in host memory that the device writes: the host
+// launches iterations by it without stopping the stream. `word` is written
+// last: pass number << 34 | iteration << 2 | non-finite << 1 | active.
+struct Progress {
+  double rr;
+  unsigned long long word;
 };
 
 // Fine-level geometry, passed by value to kernels.

@@ -176,7 +176,7 @@ constexpr int FIN_THREADS = 1024;
 
 template <bool MAX>
 __global__ void __launch_bounds__(FIN_THREADS) k_finish(int op, unsigned nblocks, int gated, Ctl* ctl,
-                                                        double* partials) {
+                                                        double* partials, Progress* progress) {
   if ((gated == 1 && !ctl->active) || (gated == 2 && !ctl->pure_neumann) || (gated == 3 && !replacing(ctl))) return;
   __shared__ double sa[FIN_THREADS / 64], sb[FIN_THREADS / 64];
   const double2* part = reinterpret_cast<const double2*>(partials + (size_t)op * MAX_PARTIALS * 2);
@@ -210,6 +210,14 @@ __global__ void __launch_bounds__(FIN_THREADS) k_finish(int op, unsigned nblocks
   ctl->red[op][0] = a;
   ctl->red[op][1] = b;
   finish(op, ctl, a, b);
+  // an iteration has ended, or the loop has
+  if ((gated == 1 || gated == 3) && (op == OP_RZ || !ctl->active)) {
+    progress->rr = ctl->rr;
+    __hip_atomic_store(&progress->word,
+                       (unsigned long long)ctl->pass << 34 | (unsigned long long)ctl->it << 2 |
+                           (ctl->nonfinite ? 2ull : 0ull) | (ctl->active ? 1ull : 0ull),
+                       __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 // ---------------------------------------------------------------- fine geometry
@@ -1433,7 +1441,7 @@ __global__ void __launch_bounds__(HASH_THREADS) k_hash_combine(const unsigned lo
 
 // Host-side parameters of a CG pass, written on the stream.
 __global__ void k_set_pass(Ctl* ctl, int active, double rr, double tol_b2, double physical_target, uint32_t it,
-                           uint32_t max_iters, uint32_t pass_limit, int flexible, uint32_t replace_every) {
+                           uint32_t max_iters, uint32_t pass_limit, int flexible, uint32_t replace_every, uint32_t pass) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   ctl->active = active;
   ctl->flexible = flexible;
@@ -1448,6 +1456,7 @@ __global__ void k_set_pass(Ctl* ctl, int active, double rr, double tol_b2, doubl
   ctl->pass_limit = pass_limit;
   ctl->stop_dq = 0;
   ctl->nonfinite = 0;
+  ctl->pass = pass;
 }
 
 }  // namespace fsp
