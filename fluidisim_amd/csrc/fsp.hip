@@ -80,6 +80,10 @@ struct fsp_solver {
   float* col_floor = nullptr;  // per column: top of its highest solid cell (0 without one)
   uint16_t* gk0 = nullptr;  // per column: lowest ghost row
   float* gtab = nullptr;    // per column: 1/theta of G_SLOTS ghost rows
+  // ghost-row index of geometries without column tables, reserved by the
+  // first one set (quad grids)
+  uint32_t *gidx = nullptr, *gcells = nullptr, gidx_cap = 0;
+  float* gent = nullptr;
   float* precv = nullptr;   // per cell: row_prec (quad V-cycle)
   float *b = nullptr, *r = nullptr, *p = nullptr, *q = nullptr, *z = nullptr, *zt = nullptr, *d0 = nullptr,
         *d1 = nullptr;
@@ -107,11 +111,11 @@ struct fsp_solver {
   std::vector<void*> allocs;
   // live timing of one kernel (fsp_profile_begin / fsp_profile_end)
   // one CG iteration captured as a graph, replayed per iteration
-  // one CG iteration per (phase, kernel form): [2 * phase + table_only],
+  // one CG iteration per (phase, kernel form): [FORMS * phase + form],
   // phase 0 as configured, 1 the learned phase
-  hipGraph_t iter_graph[4] = {};
-  hipGraphExec_t iter_exec[4] = {};
-  int table_only = 0;                 // 1: the fine kernels' table-only forms (set per projection)
+  hipGraph_t iter_graph[2 * FORMS] = {};
+  hipGraphExec_t iter_exec[2 * FORMS] = {};
+  int form = FORM_GENERAL;            // the fine kernels' form (set per projection)
   fsp_net* net = nullptr;             // learned preconditioner (not owned)
   uint64_t net_gen = 0;               // the network's buffer generation iter_graph[1] captured
   int net_phase = 0;                  // 1 while the current pass uses the network
@@ -164,6 +168,10 @@ struct fsp_solver {
     G.gk0 = gk0;
     G.gtab = gtab;
     G.precv = precv;
+    const bool indexed = (frac || levelset) && gidx;
+    G.gq = indexed ? gidx : nullptr;
+    G.gent = gent;
+    G.gcap = indexed ? gidx_cap : 0u;
     // prec of a plain row with n faces, 1/(n * inv), as rhs_mobile3 computes it
     G.prec_tab[0] = 0.f;
     for (int q = 1; q < 7; ++q) G.prec_tab[q] = 1.0f / ((float)q * G.inv);
@@ -250,13 +258,13 @@ inline bool prof_begin(fsp_solver* S, const char* name, hipStream_t stream, hipE
   FSP_LAUNCH_NBS(S, name, kern, grid, BLOCK, lds, stream, __VA_ARGS__)
 #define FSP_LAUNCH(S, kern, grid, stream, ...) FSP_LAUNCH_N(S, #kern, kern, grid, stream, __VA_ARGS__)
 
-// A fine-level kernel in its table-only form (template argument GEN false:
-// every ghost row of the geometry lies in its column's table, known after
-// the projection's first sync) or its general form.
-#define FSP_LAUNCH_GEN(S, name, KT, KG, grid, block, stream, ...)                             \
-  do {                                                                                     \
-    if ((S)->table_only) FSP_LAUNCH_NBS(S, name, KT, grid, block, 0, stream, __VA_ARGS__); \
-    else FSP_LAUNCH_NBS(S, name, KG, grid, block, 0, stream, __VA_ARGS__);                 \
+// A fine-level kernel in the form the projection's ghost rows allow
+// (FORM_TABLE, FORM_INDEX or FORM_GENERAL, known after its first sync).
+#define FSP_LAUNCH_FORM(S, name, KT, KI, KG, grid, block, stream, ...)                          \
+  do {                                                                                        \
+    if ((S)->form == FORM_TABLE) FSP_LAUNCH_NBS(S, name, KT, grid, block, 0, stream, __VA_ARGS__); \
+    else if ((S)->form == FORM_INDEX) FSP_LAUNCH_NBS(S, name, KI, grid, block, 0, stream, __VA_ARGS__); \
+    else FSP_LAUNCH_NBS(S, name, KG, grid, block, 0, stream, __VA_ARGS__);                     \
   } while (0)
 
 // Kernels templated on the V-cycle storage ST of the enclosing function.
@@ -303,9 +311,10 @@ bool coarsens3(size_t nx, size_t ny, size_t nz) {
 }
 
 __global__ void k_reset(Ctl* ctl, int gauge) {
+  static_assert(sizeof(Ctl) % 4 == 0, "cleared in words");
+  for (int q = (int)threadIdx.x; q < (int)(sizeof(Ctl) / 4); q += (int)blockDim.x) reinterpret_cast<uint32_t*>(ctl)[q] = 0;
+  __syncthreads();
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  unsigned char* bytes = (unsigned char*)ctl;
-  for (size_t q = 0; q < sizeof(Ctl); ++q) bytes[q] = 0;
   ctl->first_dir = 1;
   ctl->physical_target = __longlong_as_double(0x7ff0000000000000ll);
   ctl->gauge = gauge;
@@ -349,6 +358,7 @@ struct Launch {
       // labels and level set: no column structure, no ghost-row table
       FSP_LAUNCH(S, k_mask_ls, g, st, G, S->mask, S->ctl, S->partials);
       FSP_FINISH(S, st, OP_COUNT, g, false, 0);
+      ghost_rows();
       if (S->precv) FSP_LAUNCH(S, k_prec, g, st, G, S->precv);
       return;
     }
@@ -360,10 +370,19 @@ struct Launch {
       FSP_LAUNCH(S, k_mask, g, st, G, S->mask, S->ctl, S->partials);
       FSP_FINISH(S, st, OP_COUNT, g, false, 0);
     }
-    // ghost-row table from the fresh row codes (k_mask's finish does not touch it)
-    Fine Gm = G;
-    FSP_LAUNCH(S, k_ghost_table, dim3(grid_for(S->ncols)), st, Gm, S->gk0, S->gtab, S->ctl);
-    if (S->precv && prec) FSP_LAUNCH(S, k_prec, g, st, Gm, S->precv);
+    // ghost-row table or index from the fresh row codes (k_mask's finish does not touch it)
+    if (S->frac) ghost_rows();
+    else FSP_LAUNCH(S, k_ghost_table, dim3(grid_for(S->ncols)), st, G, S->gk0, S->gtab, S->ctl);
+    if (S->precv && prec) FSP_LAUNCH(S, k_prec, g, st, G, S->precv);
+  }
+
+  // The ghost-row index and its entries (geometries without column tables).
+  void ghost_rows() {
+    if (!G.gq) return;
+    const size_t nquads = G.n / 4;
+    FSP_LAUNCH(S, k_ghost_index, dim3((unsigned)((nquads + BLOCK - 1) / BLOCK)), st, G, nquads, S->gidx, S->gcells, S->ctl);
+    FSP_LAUNCH(S, k_ghost_fill, dim3((unsigned)((S->gidx_cap + BLOCK - 1) / BLOCK)), st, G, (const uint32_t*)S->gcells,
+               S->gent, (const Ctl*)S->ctl);
   }
 
   // A level whose V-cycle kernels read only couplings and Dirichlet parts:
@@ -425,7 +444,7 @@ struct Launch {
     const int gated = replacement ? 1 : 0, fin_gate = replacement ? 3 : 0;
     if (S->quad) {
       const dim3 gq((unsigned)(S->qfine.nbx * S->qfine.nby * S->qfine.planes));
-      FSP_LAUNCH_GEN(S, "k_residual_q", k_residual_q<false>, k_residual_q<true>, gq, QBLOCK, st, G, S->qfine, p64,
+      FSP_LAUNCH_FORM(S, "k_residual_q", k_residual_q<FORM_TABLE>, k_residual_q<FORM_INDEX>, k_residual_q<FORM_GENERAL>, gq, QBLOCK, st, G, S->qfine, p64,
                      S->b, S->r, op, S->ctl, S->partials, gated);
       FSP_FINISH(S, st, op, gq, false, fin_gate);
     } else {
@@ -439,7 +458,8 @@ struct Launch {
   // OP_BACKWARD, in one pass over p64 (quads only).
   void residual_backward(const double* p64) {
     const dim3 gq((unsigned)(S->qfine.nbx * S->qfine.nby * S->qfine.planes));
-    FSP_LAUNCH_GEN(S, "k_residual_q", (k_residual_q<false, true>), (k_residual_q<true, true>), gq, QBLOCK, st, G,
+    FSP_LAUNCH_FORM(S, "k_residual_q", (k_residual_q<FORM_TABLE, true>), (k_residual_q<FORM_INDEX, true>),
+                    (k_residual_q<FORM_GENERAL, true>), gq, QBLOCK, st, G,
                    S->qfine, p64, S->b, S->r, OP_RR, S->ctl, S->partials, 0);
     FSP_FINISH(S, st, OP_RR, gq, false, 0);
     FSP_FINISH(S, st, OP_BACKWARD, gq, true, 0);
@@ -685,7 +705,7 @@ struct Launch {
     const TS<ST>* none = nullptr;
     if (S->brick.bx > 0) return vcycle_fused<ST>(dot_op, from_guess);
     auto pass = [&](TS<ST>* x, int colour, int op) {
-      FSP_LAUNCH_GEN(S, "k_q_gs<0>", (k_q_gs<0, ST, false>), (k_q_gs<0, ST, true>), g, BLOCK, st, G, Q,
+      FSP_LAUNCH_FORM(S, "k_q_gs<0>", (k_q_gs<0, ST, FORM_TABLE>), (k_q_gs<0, ST, FORM_INDEX>), (k_q_gs<0, ST, FORM_GENERAL>), g, BLOCK, st, G, Q,
                      (const TS<ST>*)x, x, S->r, colour, L0, none, op, S->ctl, S->partials);
       if (op >= 0) FSP_FINISH(S, st, op, g, false, 1);
     };
@@ -693,7 +713,7 @@ struct Launch {
       pass(z, 0, -1);
       pass(z, 1, -1);
     } else {
-      FSP_LAUNCH_GEN(S, "k_q_gs_first", (k_q_gs_first<ST, false>), (k_q_gs_first<ST, true>), g, BLOCK, st, G, Q, z,
+      FSP_LAUNCH_FORM(S, "k_q_gs_first", (k_q_gs_first<ST, FORM_TABLE>), (k_q_gs_first<ST, FORM_INDEX>), (k_q_gs_first<ST, FORM_GENERAL>), g, BLOCK, st, G, Q, z,
                      S->r, S->ctl);
     }
     for (int s = 1; s < S->opt.pre_sweeps; ++s) {
@@ -709,11 +729,11 @@ struct Launch {
       H.RY = (QBLOCK / 2) / H.QX;
       H.nby = (H.rows + H.RY - 1) / H.RY;
       const dim3 gr((unsigned)(H.nbx * H.nby * H.planes));
-      FSP_LAUNCH_GEN(S, "k_q_restrict", (k_q_restrict2<ST, false>), (k_q_restrict2<ST, true>), gr, BLOCK, st, G, H,
+      FSP_LAUNCH_FORM(S, "k_q_restrict", (k_q_restrict2<ST, FORM_TABLE>), (k_q_restrict2<ST, FORM_INDEX>), (k_q_restrict2<ST, FORM_GENERAL>), gr, BLOCK, st, G, H,
                      (const TS<ST>*)z, (const float*)S->r, L0, S->ctl);
       const TS<ST>* x0 = coarse_cycle<ST>();
       const int op = passes == 1 ? dot_op : -1;
-      FSP_LAUNCH_GEN(S, "k_q_gs<2>", (k_q_gs<2, ST, false>), (k_q_gs<2, ST, true>), g, BLOCK, st, G, Q,
+      FSP_LAUNCH_FORM(S, "k_q_gs<2>", (k_q_gs<2, ST, FORM_TABLE>), (k_q_gs<2, ST, FORM_INDEX>), (k_q_gs<2, ST, FORM_GENERAL>), g, BLOCK, st, G, Q,
                      (const TS<ST>*)z, zt, S->r, 1, L0, x0, op, S->ctl, S->partials);
       if (op >= 0) FSP_FINISH(S, st, op, g, false, 1);
       out = zt;
@@ -740,17 +760,17 @@ struct Launch {
     const TS<ST>* none = nullptr;
     auto sweep = [&](int colour, const TS<ST>* xc, int op) {
       if (xc)
-        FSP_LAUNCH_GEN(S, "k_q_brick<2>", (k_q_brick<2, ST, false>), (k_q_brick<2, ST, true>), gb, BR_THREADS, st, G,
+        FSP_LAUNCH_FORM(S, "k_q_brick<2>", (k_q_brick<2, ST, FORM_TABLE>), (k_q_brick<2, ST, FORM_INDEX>), (k_q_brick<2, ST, FORM_GENERAL>), gb, BR_THREADS, st, G,
                        S->brick, (const TS<ST>*)a, b, S->r, colour, L0, xc, op, S->ctl, S->partials);
       else
-        FSP_LAUNCH_GEN(S, "k_q_brick<0>", (k_q_brick<0, ST, false>), (k_q_brick<0, ST, true>), gb, BR_THREADS, st, G,
+        FSP_LAUNCH_FORM(S, "k_q_brick<0>", (k_q_brick<0, ST, FORM_TABLE>), (k_q_brick<0, ST, FORM_INDEX>), (k_q_brick<0, ST, FORM_GENERAL>), gb, BR_THREADS, st, G,
                        S->brick, (const TS<ST>*)a, b, S->r, colour, L0, none, op, S->ctl, S->partials);
       if (op >= 0) FSP_FINISH(S, st, op, gb, false, 1);
       std::swap(a, b);
     };
     if (from_guess) sweep(0, none, -1);
     else
-      FSP_LAUNCH_GEN(S, "k_q_gs_first", (k_q_gs_first<ST, false>), (k_q_gs_first<ST, true>), g, BLOCK, st, G, Q, a,
+      FSP_LAUNCH_FORM(S, "k_q_gs_first", (k_q_gs_first<ST, FORM_TABLE>), (k_q_gs_first<ST, FORM_INDEX>), (k_q_gs_first<ST, FORM_GENERAL>), g, BLOCK, st, G, Q, a,
                      S->r, S->ctl);
     for (int s = 1; s < S->opt.pre_sweeps; ++s) sweep(0, none, -1);
     const TS<ST>* x0 = none;
@@ -759,7 +779,7 @@ struct Launch {
       H.RY = (QBLOCK / 2) / H.QX;
       H.nby = (H.rows + H.RY - 1) / H.RY;
       const dim3 gr((unsigned)(H.nbx * H.nby * H.planes));
-      FSP_LAUNCH_GEN(S, "k_q_restrict", (k_q_restrict2<ST, false>), (k_q_restrict2<ST, true>), gr, BLOCK, st, G, H,
+      FSP_LAUNCH_FORM(S, "k_q_restrict", (k_q_restrict2<ST, FORM_TABLE>), (k_q_restrict2<ST, FORM_INDEX>), (k_q_restrict2<ST, FORM_GENERAL>), gr, BLOCK, st, G, H,
                      (const TS<ST>*)a, (const float*)S->r, L0, S->ctl);
       x0 = coarse_cycle<ST>();
     }
@@ -787,7 +807,7 @@ struct Launch {
         const float* none = nullptr;
         for (int s = 0; s < S->opt.learned_smooth; ++s)
           for (int c = 0; c < 2; ++c)
-            FSP_LAUNCH_GEN(S, "k_q_gs<0>", (k_q_gs<0, ST_F32, false>), (k_q_gs<0, ST_F32, true>), g, BLOCK, st,
+            FSP_LAUNCH_FORM(S, "k_q_gs<0>", (k_q_gs<0, ST_F32, FORM_TABLE>), (k_q_gs<0, ST_F32, FORM_INDEX>), (k_q_gs<0, ST_F32, FORM_GENERAL>), g, BLOCK, st,
                            G, Q, (const float*)S->z, S->z, S->r, c, none_l, none, -1, S->ctl, S->partials);
       }
       FSP_LAUNCH(S, k_dot_rz_qz, dim3(grid_for(G.n)), st, G.n, (const float*)S->r, (const float*)zout,
@@ -832,7 +852,7 @@ struct Launch {
                                                                                            : FSP_STORE_F32;
       with_storage(storage, [&](auto c) {
         constexpr int ST = decltype(c)::value;
-        FSP_LAUNCH_GEN(S, "k_q_spmv_dir", (k_q_spmv_dir<ST, false>), (k_q_spmv_dir<ST, true>), g, BLOCK, st, G, Q,
+        FSP_LAUNCH_FORM(S, "k_q_spmv_dir", (k_q_spmv_dir<ST, FORM_TABLE>), (k_q_spmv_dir<ST, FORM_INDEX>), (k_q_spmv_dir<ST, FORM_GENERAL>), g, BLOCK, st, G, Q,
                        (const TS<ST>*)S->zres, S->d0, S->d1, S->q, S->ctl, S->partials);
         return 0;
       });
@@ -901,7 +921,7 @@ fsp_status sync_ctl(fsp_solver* S) {
 }
 
 void cleanup(fsp_solver* S) {
-  for (int g = 0; g < 4; ++g) {
+  for (int g = 0; g < 2 * FORMS; ++g) {
     if (S->iter_exec[g]) (void)hipGraphExecDestroy(S->iter_exec[g]);
     if (S->iter_graph[g]) (void)hipGraphDestroy(S->iter_graph[g]);
     S->iter_exec[g] = nullptr;
@@ -983,7 +1003,7 @@ void launch_backward(fsp_solver* S, const double* p) {
   Launch K(S);
   if (S->quad) {
     const dim3 gq((unsigned)(S->qfine.nbx * S->qfine.nby * S->qfine.planes));
-    FSP_LAUNCH_GEN(S, "k_backward_q", k_backward_q<false>, k_backward_q<true>, gq, QBLOCK, K.st, K.G, S->qfine,
+    FSP_LAUNCH_FORM(S, "k_backward_q", k_backward_q<FORM_TABLE>, k_backward_q<FORM_INDEX>, k_backward_q<FORM_GENERAL>, gq, QBLOCK, K.st, K.G, S->qfine,
                    (const double*)p, S->b, S->r, S->ctl, S->partials);
     FSP_FINISH(S, K.st, OP_BACKWARD, gq, true, 0);
   } else {
@@ -1014,8 +1034,15 @@ fsp_status fingerprint(fsp_solver* S, const double* p, uint64_t& h) {
 // Captures one CG iteration (every kernel reads its scalars from the device
 // control block and every buffer is the solver's own, so the graph stays
 // valid for the solver's lifetime) and instantiates it once.
+// The kernel form of the geometry in place when every ghost row is where the
+// form looks for it.
+int fast_form(const fsp_solver* S) {
+  if (!S->frac && !S->levelset) return FORM_TABLE;
+  return S->gidx ? FORM_INDEX : FORM_GENERAL;
+}
+
 fsp_status capture_iteration(fsp_solver* S) {
-  const int slot = 2 * S->net_phase + S->table_only;
+  const int slot = FORMS * S->net_phase + S->form;
   if (S->iter_exec[slot]) return FSP_OK;
   const bool prof = S->prof_on;
   S->prof_on = false;
@@ -1040,10 +1067,10 @@ fsp_status capture_iteration(fsp_solver* S) {
   return FSP_OK;
 }
 
-// Drops both kernel forms' graphs of phase `phase`.
+// Drops every kernel form's graph of phase `phase`.
 void drop_graph(fsp_solver* S, int phase) {
-  for (int t = 0; t < 2; ++t) {
-    const int slot = 2 * phase + t;
+  for (int t = 0; t < FORMS; ++t) {
+    const int slot = FORMS * phase + t;
     if (S->iter_exec[slot]) (void)hipGraphExecDestroy(S->iter_exec[slot]);
     if (S->iter_graph[slot]) (void)hipGraphDestroy(S->iter_graph[slot]);
     S->iter_exec[slot] = nullptr;
@@ -1056,12 +1083,13 @@ void drop_graph(fsp_solver* S, int phase) {
 // projection allocates nothing (the reference reserves every buffer before
 // seal(), delta3d.rs:225-241). A throwaway capture of the prime first sets
 // which buffer holds M^-1 r, as the prime of a projection does before its
-// first iteration. Both kernel forms (general and table-only) are captured;
-// each projection replays the one its geometry allows.
+// first iteration. The general form and the one the kind of geometry may
+// allow are captured; each projection replays the one its rows allow.
 fsp_status prepare_graph(fsp_solver* S, int phase) {
-  if (!S->opt.graph || (S->iter_exec[2 * phase] && S->iter_exec[2 * phase + 1])) return FSP_OK;
+  const int forms[2] = {FORM_GENERAL, fast_form(S)};
+  if (!S->opt.graph || (S->iter_exec[FORMS * phase + forms[0]] && S->iter_exec[FORMS * phase + forms[1]])) return FSP_OK;
   if (phase == 1 && !S->net) return FSP_OK;
-  const int saved = S->net_phase, saved_table = S->table_only;
+  const int saved = S->net_phase, saved_form = S->form;
   const bool prof = S->prof_on;
   S->net_phase = phase;
   S->prof_on = false;
@@ -1078,13 +1106,34 @@ fsp_status prepare_graph(fsp_solver* S, int phase) {
   S->prof_on = prof;
   fsp_status st = e == hipSuccess ? FSP_OK : FSP_DEVICE;
   for (int t = 0; t < 2 && st == FSP_OK; ++t) {
-    S->table_only = t;
+    S->form = forms[t];
     st = capture_iteration(S);
   }
-  S->table_only = saved_table;
+  S->form = saved_form;
   S->net_phase = saved;
   if (e != hipSuccess) std::fprintf(stderr, "fsp: prime capture failed: %s\n", hipGetErrorString(e));
   return st;
+}
+
+// Reserves the ghost-row index (configuration calls of geometries without
+// column tables): entries for a quarter of the cells, 14 bytes a cell in all. Without
+// the memory the general kernels run.
+void reserve_index(fsp_solver* S) {
+  if (!S->quad || S->gidx) return;
+  const size_t cap = std::max<size_t>(S->n / 4, 64);
+  void* mem[3] = {};
+  const size_t bytes[3] = {S->n, cap * sizeof(uint32_t), cap * GE_FLOATS * sizeof(float)};
+  for (int a = 0; a < 3; ++a)
+    if (hipMalloc(&mem[a], bytes[a]) != hipSuccess) {
+      (void)hipGetLastError();
+      for (int q = 0; q < a; ++q) (void)hipFree(mem[q]);
+      return;
+    }
+  for (void* m : mem) S->allocs.push_back(m);
+  S->gcells = (uint32_t*)mem[1];
+  S->gent = (float*)mem[2];
+  S->gidx_cap = (uint32_t)cap;
+  S->gidx = (uint32_t*)mem[0];
 }
 
 // The iteration graphs hold the fine geometry's kernel arguments: after a
@@ -1291,12 +1340,12 @@ fsp_status run(fsp_solver* S, const float* us, const float* vs, const float* ws,
   if (!S->geom) return FSP_DOMAIN;
   // the graded column takes the projection (delta3d_mobile.rs:473-475)
   if (!S->gnodes.empty()) return run_graded(S, us, vs, ws, p, warm, u, v, w, scale, k1, rel_tol, max_iters, rep);
-  // the table-only kernel forms hold for this projection only
+  // the table and index forms hold for this projection only
   struct TableGuard {
     fsp_solver* S;
-    ~TableGuard() { S->table_only = 0; }
+    ~TableGuard() { S->form = FORM_GENERAL; }
   } table_guard{S};
-  S->table_only = 0;
+  S->form = FORM_GENERAL;
   S->net_phase = 0;
   if (S->opt.preconditioner == FSP_PRECOND_LEARNED) {
     if (!S->net) return FSP_INVALID;
@@ -1304,7 +1353,7 @@ fsp_status run(fsp_solver* S, const float* us, const float* vs, const float* ws,
     if (ns) return ns;
     // the network's buffers moved since the learned graph was captured (a
     // forward pass or another solver at another shape): capture it again
-    if (S->iter_exec[2] && S->net_gen != net_generation(S->net)) {
+    if (S->iter_exec[FORMS + FORM_GENERAL] && S->net_gen != net_generation(S->net)) {
       drop_graph(S, 1);
       if (const fsp_status gs = prepare_graph(S, 1)) return gs;
     }
@@ -1350,9 +1399,9 @@ fsp_status run(fsp_solver* S, const float* us, const float* vs, const float* ws,
   fsp_status st = sync_ctl(S);
   if (st) return st;
   if (S->hctl->nonfinite) return FSP_NOT_FINITE;
-  // every ghost row in its column's table (binary apertures, column
-  // geometry): the fine kernels' table-only forms
-  S->table_only = (!S->frac && !S->levelset && !S->hctl->table_miss) ? 1 : 0;
+  // every ghost row in its column's table or in the index: the fine kernels'
+  // forms that read nothing else
+  S->form = S->hctl->table_miss ? FORM_GENERAL : fast_form(S);
   // the correction's gauge runs only for a pure-Neumann problem (known now)
   const bool gauge_now = S->opt.gauge && S->hctl->pure_neumann;
 
@@ -1395,7 +1444,7 @@ fsp_status run(fsp_solver* S, const float* us, const float* vs, const float* ws,
       // times a projection: 2.10 against 1.87 ms at 128^3, 4.50 against 4.08 at
       // 256x256x128.)
       if (S->opt.graph && !S->prof_on && (st = capture_iteration(S))) return st;
-      const hipGraphExec_t gx = S->prof_on ? nullptr : S->iter_exec[2 * S->net_phase + S->table_only];
+      const hipGraphExec_t gx = S->prof_on ? nullptr : S->iter_exec[FORMS * S->net_phase + S->form];
       const double goal = std::min(tol_b2, physical_target);
       PassState done{it, true, false, rr};
       double rate = 1.0;  // |r|^2 per iteration, observed
@@ -1840,6 +1889,7 @@ fsp_status fsp_set_geometry(fsp_solver* S, const fsp_surface* surf, const float*
       fsp_status as;
       if ((as = dalloc(S, &S->au, S->nu)) || (as = dalloc(S, &S->av, S->nv)) || (as = dalloc(S, &S->aw, S->nw)))
         return as;
+      reserve_index(S);
     }
     float* dst[3] = {S->au, S->av, S->aw};
     for (int a = 0; a < 3; ++a) {
@@ -1904,6 +1954,7 @@ fsp_status fsp_set_level_set(fsp_solver* S, const uint8_t* labels, size_t n_labe
   if (!S->water) {
     fsp_status as;
     if ((as = dalloc(S, &S->water, S->n)) || (as = dalloc(S, &S->phi, S->n))) return as;
+    reserve_index(S);
   }
   FSP_HIP(hipMemcpyAsync(S->solid, hs.data(), S->n, hipMemcpyHostToDevice, S->stream));
   FSP_HIP(hipMemcpyAsync(S->water, hwat.data(), S->n, hipMemcpyHostToDevice, S->stream));
@@ -2198,14 +2249,13 @@ fsp_status fsp_precondition_device(fsp_solver* S, const float* d_r, float* d_z) 
   if (!S->geom) return FSP_DOMAIN;
   FSP_HIP(hipSetDevice(S->opt.device));
   build_geometry(S, true);
-  // the fine kernels' form a projection on this geometry takes (the
-  // table-only one when every ghost row lies in its column's table)
+  // the fine kernels' form a projection on this geometry takes
   if (const fsp_status st = sync_ctl(S)) return st;
   struct TableGuard {
     fsp_solver* S;
-    ~TableGuard() { S->table_only = 0; }
+    ~TableGuard() { S->form = FORM_GENERAL; }
   } table_guard{S};
-  S->table_only = (!S->frac && !S->levelset && !S->hctl->table_miss) ? 1 : 0;
+  S->form = S->hctl->table_miss ? FORM_GENERAL : fast_form(S);
   Launch K(S);
   FSP_HIP(hipMemcpyAsync(S->r, d_r, S->n * 4, hipMemcpyDeviceToDevice, S->stream));
   K.set_pass(1, 0.0, 0.0, 0.0, 0, 1);

@@ -20,6 +20,12 @@ constexpr int MAX_BLOCKS = 2048;  // grid cap of grid-stride kernels (8 per CU)
 constexpr int NUM_SLOTS = 16;     // reduction slots
 constexpr int MAX_PARTIALS = 65536;  // blocks a reducing kernel may have
 constexpr int G_SLOTS = 8;        // ghost rows tabulated per column
+constexpr int GE_FLOATS = 12;     // floats of an indexed ghost row's entry
+
+// Where the fine kernels' ghost rows come from: the column's table alone, the
+// geometry itself (any row; the tables where they hold it), or the entries of
+// the ghost-row index alone.
+enum : int { FORM_TABLE = 0, FORM_GENERAL = 1, FORM_INDEX = 2, FORMS = 3 };
 
 // Reduction slots / finish operations.
 enum Op : int {
@@ -58,7 +64,8 @@ struct Ctl {
   int32_t stalled;       // a replaced true residual did not fall below the previous one: the pass ends
   double rr_replaced;    // |r|^2 of the last replaced true residual of the pass
   uint32_t wet_cells, ghost_faces;
-  int32_t table_miss;    // a ghost row lies past its column's table: the general fine kernels run
+  int32_t table_miss;    // a ghost row lies past its column's table or the index: the general fine kernels run
+  uint32_t ghost_rows;   // rows in the ghost-row index
   uint32_t pass;         // number of the pass (Progress)
 };
 
@@ -88,6 +95,14 @@ struct Fine {
   const uint16_t* gk0;   // columns: lowest ghost row (0xFFFF: none)
   const float* gtab;     // columns x G_SLOTS x 8: 1/theta of the ghost faces
   const float* precv;    // cells: row_prec of every row (k_prec)
+  // Ghost rows of a geometry without column tables (fractional apertures, a
+  // level set), on grids of quads: gq[quad] is the entry of the quad's first
+  // ghost row, the others follow; GE_FLOATS floats an entry (1/theta of the
+  // six faces, then their apertures), the first gcap entries exist (null:
+  // no index)
+  const uint32_t* gq;
+  const float* gent;
+  uint32_t gcap;
   // Fractional apertures (the reference's cut geometry): the u8 face arrays
   // hold 0 closed, 1 open, 2 fractional, and a code-2 face's aperture is in
   // au/av/aw (null and frac == 0 when every aperture is 0 or 1).

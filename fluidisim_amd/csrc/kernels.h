@@ -358,23 +358,43 @@ __device__ __forceinline__ bool ghost_its(const Fine& G, int i, int j, int k, fl
   return true;
 }
 
+// The index entry of the ghost row of x-cell e in a quad with row codes mq
+// whose first ghost row has entry `first`.
+__device__ __forceinline__ uint32_t ghost_index(const Fine& G, uint32_t mq, uint32_t first, int e) {
+  return first + (uint32_t)__popc(mq & 0x80808080u & ((1u << (8 * e)) - 1u));
+}
+
 // Per-face coefficients of a row with ghost faces or fractional apertures:
 // type 1 neighbour, 2 ghost, with the face's aperture a (1 with binary
 // apertures). With fractional apertures every such row comes from the
 // geometry (the ghost table holds binary rows only).
-// GEN false: the table only (the host runs these forms when every ghost row
-// of a binary column geometry lies in its column's table; the geometry's
-// arithmetic, which sets a kernel's register count, is then not compiled).
-template <bool GEN = true>
+// FORM_TABLE, FORM_INDEX: the host runs these forms when every ghost row is
+// in its column's table or in the index; the geometry's arithmetic, which sets
+// a kernel's register count, is then not compiled.
+template <int FORM = FORM_GENERAL>
 __device__ __forceinline__ void ghost_row(const Fine& G, int i, int j, int k, uint8_t m, uint8_t type[6], float it[6],
                                           float a[6]) {
-  if (!GEN) {
+  if (FORM == FORM_INDEX || (FORM == FORM_GENERAL && G.gq)) {
+    const size_t c = cidx(G, i, j, k);
+    const uint32_t n = ghost_index(G, *reinterpret_cast<const uint32_t*>(G.mask + (c & ~(size_t)3)), G.gq[c >> 2],
+                                   (int)(c & 3));
+    if (FORM == FORM_INDEX || n < G.gcap) {
+      const float4* e = reinterpret_cast<const float4*>(G.gent + (size_t)n * GE_FLOATS);
+      const float4 x = e[0], y = e[1], z = e[2];
+      it[0] = x.x; it[1] = x.y; it[2] = x.z; it[3] = x.w; it[4] = y.x; it[5] = y.y;
+      a[0] = y.z; a[1] = y.w; a[2] = z.x; a[3] = z.y; a[4] = z.z; a[5] = z.w;
+#pragma unroll
+      for (int f = 0; f < 6; ++f) type[f] = (m & (1u << f)) ? 1 : (it[f] > 0.f ? 2 : 0);
+      return;
+    }
+  }
+  if (FORM == FORM_TABLE) {
     const float* e = ghost_entry(G, (size_t)j * G.nx + i, k);
     const float4 lo = *reinterpret_cast<const float4*>(e);
     const float2 hi = *reinterpret_cast<const float2*>(e + 4);
     it[0] = lo.x; it[1] = lo.y; it[2] = lo.z; it[3] = lo.w; it[4] = hi.x; it[5] = hi.y;
   }
-  if (!GEN || (!G.frac && !G.phi && ghost_its(G, i, j, k, it))) {
+  if (FORM == FORM_TABLE || (FORM == FORM_GENERAL && !G.frac && !G.phi && ghost_its(G, i, j, k, it))) {
 #pragma unroll
     for (int f = 0; f < 6; ++f) {
       type[f] = (m & (1u << f)) ? 1 : (it[f] > 0.f ? 2 : 0);
@@ -644,6 +664,49 @@ __global__ void __launch_bounds__(BLOCK) k_ghost_table(Fine G, uint16_t* gk0, fl
     }
     if (miss) ctl->table_miss = 1;
   }
+}
+
+// The ghost-row index of a quad grid from the row codes: entries are dealt out
+// a wavefront at a time (their order differs from run to run, the rows' values
+// do not depend on it), cells[entry] is the row's cell.
+__global__ void __launch_bounds__(BLOCK) k_ghost_index(Fine G, size_t nquads, uint32_t* gq, uint32_t* cells, Ctl* ctl) {
+  const size_t q = (size_t)blockIdx.x * BLOCK + threadIdx.x;
+  const int lane = (int)(threadIdx.x & 63u);
+  const uint32_t ghosts = q < nquads ? *reinterpret_cast<const uint32_t*>(G.mask + 4 * q) & 0x80808080u : 0u;
+  const uint32_t count = (uint32_t)__popc(ghosts);
+  uint32_t upto = count;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t v = __shfl_up(upto, o, 64);
+    if (lane >= o) upto += v;
+  }
+  uint32_t first = 0;
+  if (lane == 63 && upto) first = atomicAdd(&ctl->ghost_rows, upto);
+  first = __shfl(first, 63, 64) + upto - count;
+  if (!count) return;
+  gq[q] = first;
+  for (int e = 0; e < 4; ++e) {
+    if (!(ghosts & (0x80u << (8 * e)))) continue;
+    if (first < G.gcap) cells[first] = (uint32_t)(4 * q) + e;
+    ++first;
+  }
+  if (first > G.gcap) ctl->table_miss = 1;
+}
+// The entries: full_row of each listed cell, once per projection instead of
+// at every pass over the row.
+__global__ void __launch_bounds__(BLOCK) k_ghost_fill(Fine G, const uint32_t* cells, float* gent, const Ctl* ctl) {
+  const uint32_t n = (uint32_t)blockIdx.x * BLOCK + threadIdx.x;
+  if (n >= ctl->ghost_rows || n >= G.gcap) return;
+  int i, j, k;
+  decode(G, cells[n], i, j, k);
+  RowG R;
+  full_row(G, i, j, k, R);
+  float4* e = reinterpret_cast<float4*>(gent + (size_t)n * GE_FLOATS);
+  float it[6];
+#pragma unroll
+  for (int f = 0; f < 6; ++f) it[f] = R.type[f] == 2 ? R.it[f] : 0.f;
+  e[0] = make_float4(it[0], it[1], it[2], it[3]);
+  e[1] = make_float4(it[4], it[5], R.a[0], R.a[1]);
+  e[2] = make_float4(R.a[2], R.a[3], R.a[4], R.a[5]);
 }
 
 // b = scale*div + ghost terms; prec (optional). div from faces or given.

@@ -60,14 +60,14 @@ __device__ __forceinline__ float4 ld4(const float* p, size_t c) { return *reinte
 __device__ __forceinline__ void st4(float* p, size_t c, const float4& v) { *reinterpret_cast<float4*>(p + c) = v; }
 __device__ __forceinline__ float4 f4zero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
 
-// The sum of a free-surface row (about one row in a hundred); GEN as ghost_row.
-template <bool GEN = true>
+// The sum of a free-surface row (about one row in a hundred); FORM as ghost_row.
+template <int FORM = FORM_GENERAL>
 __device__ __forceinline__ float ghost_row_sum(const Fine& G, int i, int j, int k, uint8_t m, float pc, const float nb[6],
                                             float& prec) {
 #pragma clang fp contract(off)
   uint8_t type[6];
   float it[6], a[6];
-  ghost_row<GEN>(G, i, j, k, m, type, it, a);
+  ghost_row<FORM>(G, i, j, k, m, type, it, a);
   float acc = 0.f, diag = 0.f;
 #pragma unroll
   for (int f = 0; f < 6; ++f) {
@@ -79,8 +79,8 @@ __device__ __forceinline__ float ghost_row_sum(const Fine& G, int i, int j, int 
 }
 
 // Row of the fine operator from neighbour values already in registers, in the
-// reference's face order; prec as rhs_mobile3 computes it (GEN as ghost_row).
-template <bool GEN = true>
+// reference's face order; prec as rhs_mobile3 computes it (FORM as ghost_row).
+template <int FORM = FORM_GENERAL>
 __device__ __forceinline__ float row_local(const Fine& G, int i, int j, int k, uint8_t m, float pc, const float nb[6],
                                           float& prec) {
 #pragma clang fp contract(off)
@@ -93,7 +93,7 @@ __device__ __forceinline__ float row_local(const Fine& G, int i, int j, int k, u
       if (m & (1u << f)) acc += pc - nb[f];
     prec = G.prec_tab[__popc(m & 0x3Fu)];
   } else {
-    acc = ghost_row_sum<GEN>(G, i, j, k, m, pc, nb, prec);
+    acc = ghost_row_sum<FORM>(G, i, j, k, m, pc, nb, prec);
   }
   return acc * G.inv;
 }
@@ -106,24 +106,38 @@ __device__ __forceinline__ float plain_sum(uint32_t m, float pc, const float nb[
   for (int f = 0; f < 6; ++f) acc = (m & (1u << f)) ? acc + (pc - nb[f]) : acc;
   return acc;
 }
-// ghost_row_sum from a table entry (binary apertures).
+// ghost_row_sum from a ghost row's entry: of its column's table (column col,
+// layer k; apertures 1) or of the index (entry n).
 struct GhostEntry {
-  float4 a;
-  float2 b;
+  float it[6], a[6];
 };
-__device__ __forceinline__ GhostEntry ghost_load(const Fine& G, size_t col, int k) {
-  const float* e = ghost_entry(G, col, k);
-  return {*reinterpret_cast<const float4*>(e), *reinterpret_cast<const float2*>(e + 4)};
+template <int FORM>
+__device__ __forceinline__ GhostEntry ghost_load(const Fine& G, size_t col, int k, uint32_t n) {
+  GhostEntry g;
+  const float4* e = reinterpret_cast<const float4*>(FORM == FORM_INDEX ? G.gent + (size_t)n * GE_FLOATS
+                                                                       : ghost_entry(G, col, k));
+  const float4 x = e[0];
+  g.it[0] = x.x; g.it[1] = x.y; g.it[2] = x.z; g.it[3] = x.w;
+  if (FORM == FORM_INDEX) {
+    const float4 y = e[1], z = e[2];
+    g.it[4] = y.x; g.it[5] = y.y;
+    g.a[0] = y.z; g.a[1] = y.w; g.a[2] = z.x; g.a[3] = z.y; g.a[4] = z.z; g.a[5] = z.w;
+  } else {
+    const float2 y = *reinterpret_cast<const float2*>(e + 1);
+    g.it[4] = y.x; g.it[5] = y.y;
+#pragma unroll
+    for (int f = 0; f < 6; ++f) g.a[f] = 1.0f;
+  }
+  return g;
 }
 __device__ __forceinline__ float ghost_sum(const GhostEntry& g, uint32_t m, float pc, const float nb[6], float inv,
                                            float& prec) {
 #pragma clang fp contract(off)
-  const float it[6] = {g.a.x, g.a.y, g.a.z, g.a.w, g.b.x, g.b.y};
   float acc = 0.f, diag = 0.f;
 #pragma unroll
   for (int f = 0; f < 6; ++f) {
-    const bool one = (m & (1u << f)) != 0, two = !one && it[f] > 0.f;
-    const float t = one ? pc - nb[f] : pc * it[f], d = one ? 1.0f : it[f];
+    const bool one = (m & (1u << f)) != 0, two = !one && g.it[f] > 0.f;
+    const float t = one ? g.a[f] * (pc - nb[f]) : g.a[f] * pc * g.it[f], d = one ? g.a[f] : g.a[f] * g.it[f];
     acc = (one || two) ? acc + t : acc;
     diag = (one || two) ? diag + d : diag;
   }
@@ -137,7 +151,7 @@ __device__ __forceinline__ float ghost_sum(const GhostEntry& g, uint32_t m, floa
 // four cells' table entries in one round (a row at a time, each after a look
 // at its column, held a wavefront for up to eight rounds of memory latency,
 // which a small grid has nothing to hide behind).
-template <bool GEN>
+template <int FORM>
 __device__ __forceinline__ void quad_rows(const Fine& G, int x0, int y, int k, uint32_t mq, const float4& zc, float left,
                                           float right, const float4& ym, const float4& yp, const float4& zm,
                                           const float4& zp, float row[4]) {
@@ -151,21 +165,30 @@ __device__ __forceinline__ void quad_rows(const Fine& G, int x0, int y, int k, u
   }
   const uint32_t ghosts = mq & 0x80808080u;
   if (!ghosts) return;
-  GhostEntry g[4];
-  if (!GEN) {
-    const size_t col = (size_t)y * G.nx + x0;
+  // (index entries hold apertures too: two cells at a time keep the registers)
+  constexpr int W = FORM == FORM_INDEX ? 2 : 4;
+  const size_t col = (size_t)y * G.nx + x0;
+  const uint32_t first = FORM == FORM_INDEX ? G.gq[((size_t)k * G.nx * G.ny + col) >> 2] : 0u;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) g[e] = ghost_load(G, col + e, k);
-  }
+  for (int e0 = 0; e0 < 4; e0 += W) {
+    GhostEntry g[W];
+    if (FORM != FORM_GENERAL)
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    if (!(ghosts & (0x80u << (8 * e)))) continue;
-    const uint32_t m = (mq >> (8 * e)) & 0xFFu;
-    const float pc = q_get(zc, e);
-    const float nb[6] = {e == 0 ? left : q_get(zc, e - 1), e == 3 ? right : q_get(zc, e + 1),
-                         q_get(ym, e), q_get(yp, e), q_get(zm, e), q_get(zp, e)};
-    float prec;
-    row[e] = GEN ? row_local<GEN>(G, x0 + e, y, k, (uint8_t)m, pc, nb, prec) : ghost_sum(g[e], m, pc, nb, G.inv, prec) * G.inv;
+      for (int w = 0; w < W; ++w)
+        if (FORM == FORM_TABLE || (ghosts & (0x80u << (8 * (e0 + w)))))
+          g[w] = ghost_load<FORM>(G, col + e0 + w, k, ghost_index(G, mq, first, e0 + w));
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const int e = e0 + w;
+      if (!(ghosts & (0x80u << (8 * e)))) continue;
+      const uint32_t m = (mq >> (8 * e)) & 0xFFu;
+      const float pc = q_get(zc, e);
+      const float nb[6] = {e == 0 ? left : q_get(zc, e - 1), e == 3 ? right : q_get(zc, e + 1),
+                           q_get(ym, e), q_get(yp, e), q_get(zm, e), q_get(zp, e)};
+      float prec;
+      row[e] = FORM == FORM_GENERAL ? row_local<FORM>(G, x0 + e, y, k, (uint8_t)m, pc, nb, prec)
+                                    : ghost_sum(g[w], m, pc, nb, G.inv, prec) * G.inv;
+    }
   }
 }
 
@@ -195,7 +218,7 @@ __device__ __forceinline__ void x_neighbours(const QuadGrid& Q, bool valid, int 
 // dot_op >= 0: also reduce <r, z> over every cell into that slot.
 // z, zout and the parents xc are held in storage ST (r is the f32 CG
 // residual); every value entering the arithmetic is a stored value.
-template <int MODE, int ST, bool GEN = true>
+template <int MODE, int ST, int FORM = FORM_GENERAL>
 __global__ void __launch_bounds__(QBLOCK, FSP_QGS_MIN_BLOCKS) k_q_gs(Fine G, QuadGrid Q, const typename Store<ST>::T* z,
                                                  typename Store<ST>::T* zout, const float* r, int colour, Level L0,
                                                  const typename Store<ST>::T* xc, int dot_op, Ctl* ctl,
@@ -257,7 +280,7 @@ __global__ void __launch_bounds__(QBLOCK, FSP_QGS_MIN_BLOCKS) k_q_gs(Fine G, Qua
       const float xr = e == 3 ? right : q_get(zc, e + 1);
       const float nb[6] = {xl, xr, q_get(ym, e), q_get(yp, e), q_get(zm, e), q_get(zp, e)};
       float prec;
-      const float az = row_local<GEN>(G, 4 * qx + e, y, k, m, pc, nb, prec);
+      const float az = row_local<FORM>(G, 4 * qx + e, y, k, m, pc, nb, prec);
       if (prec > 0.f) q_set(out, e, SV::rnd(pc + prec * (q_get(rq, e) - az)));
     }
     SV::st4(zout, c0, out);
@@ -273,7 +296,7 @@ __global__ void __launch_bounds__(QBLOCK, FSP_QGS_MIN_BLOCKS) k_q_gs(Fine G, Qua
 // Every value is the one the two single passes store, so the result is
 // theirs bit for bit, for one pass's traffic plus the row_prec reads (a
 // variant deriving plain rows' factor from the row code ran slower).
-template <int ST, bool GEN = true>
+template <int ST, int FORM = FORM_GENERAL>
 __global__ void __launch_bounds__(QBLOCK, FSP_QGS_MIN_BLOCKS) k_q_gs_first(Fine G, QuadGrid Q,
                                                                          typename Store<ST>::T* zout, const float* r,
                                                                          Ctl* ctl) {
@@ -336,15 +359,18 @@ __global__ void __launch_bounds__(QBLOCK, FSP_QGS_MIN_BLOCKS) k_q_gs_first(Fine 
   if ((m2[0] | m2[1]) & M_GHOST) {
     GhostEntry g[2];
     const size_t col = (size_t)y * G.nx + 4 * qx + (odd ? 1 : 0);
-    if (!GEN) {
-      g[0] = ghost_load(G, col, k);
-      g[1] = ghost_load(G, col + 2, k);
-    }
+    const uint32_t first = FORM == FORM_INDEX ? G.gq[c0 >> 2] : 0u;
+    if (FORM != FORM_GENERAL)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (FORM == FORM_TABLE || (m2[h] & M_GHOST))
+          g[h] = ghost_load<FORM>(G, col + 2 * h, k, ghost_index(G, mq, first, (odd ? 1 : 0) + 2 * h));
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       if (!(m2[h] & M_GHOST)) continue;
       float prec, az;
-      if (GEN) az = row_local<GEN>(G, 4 * qx + (odd ? 1 : 0) + 2 * h, y, k, (uint8_t)m2[h], pc2[h], nb2[h], prec);
+      if (FORM == FORM_GENERAL)
+        az = row_local<FORM>(G, 4 * qx + (odd ? 1 : 0) + 2 * h, y, k, (uint8_t)m2[h], pc2[h], nb2[h], prec);
       else az = ghost_sum(g[h], m2[h], pc2[h], nb2[h], G.inv, prec) * G.inv;
       v2[h] = prec > 0.f ? SV::rnd(pc2[h] + prec * (r2[h] - az)) : pc2[h];
     }
@@ -404,7 +430,7 @@ struct BrickGrid {
 };
 
 
-template <int MODE, int ST, bool GEN = true>
+template <int MODE, int ST, int FORM = FORM_GENERAL>
 __global__ void __launch_bounds__(BR_THREADS) k_q_brick(Fine G, BrickGrid B, const typename Store<ST>::T* zin,
                                                         typename Store<ST>::T* zout, const float* r, int colour,
                                                         Level L0, const typename Store<ST>::T* xc, int dot_op,
@@ -536,11 +562,14 @@ __global__ void __launch_bounds__(BR_THREADS) k_q_brick(Fine G, BrickGrid B, con
     uint32_t m2[2];
     float r2[2];
     GhostEntry g[2];
+    const uint32_t mq = *reinterpret_cast<const uint32_t*>(G.mask + (c - par));
+    const uint32_t first = FORM == FORM_INDEX ? G.gq[c >> 2] : 0u;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      m2[h] = G.mask[c + 2 * h];
+      m2[h] = (mq >> (8 * (par + 2 * h))) & 0xFFu;
       r2[h] = r[c + 2 * h];
-      if (!GEN) g[h] = ghost_load(G, column + 2 * h, k);
+      if (FORM == FORM_TABLE || (FORM == FORM_INDEX && (bits & (1u << (par + 2 * h)))))
+        g[h] = ghost_load<FORM>(G, column + 2 * h, k, ghost_index(G, mq, first, par + 2 * h));
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -552,7 +581,7 @@ __global__ void __launch_bounds__(BR_THREADS) k_q_brick(Fine G, BrickGrid B, con
       const float nb[6] = {(q > 0 || e > 0) ? sc[-1] : 0.f, (q + 1 < nq || e < 3) ? sc[1] : 0.f, sc[-BR_LX],
                            sc[BR_LX], sc[-BR_LX * BR_LY], sc[BR_LX * BR_LY]};
       float prec, az;
-      if (GEN) az = row_local<GEN>(G, 4 * q + e, y, k, (uint8_t)m2[h], pc, nb, prec);
+      if (FORM == FORM_GENERAL) az = row_local<FORM>(G, 4 * q + e, y, k, (uint8_t)m2[h], pc, nb, prec);
       else az = ghost_sum(g[h], m2[h], pc, nb, G.inv, prec) * G.inv;
       v[h] = prec > 0.f ? SV::rnd(pc + prec * (r2[h] - az)) : (MODE == 2 ? 0.f : pc);
     }
@@ -698,7 +727,7 @@ __global__ void __launch_bounds__(QBLOCK) k_mask_q(Fine G, QuadGrid Q, uint8_t* 
 // BACKWARD: the same pass also folds the backward error of the r it stores
 // into OP_BACKWARD, k_backward_q's arithmetic from the same pressures (|A||p|
 // beside A p), so that the wrap-up reads p once for both.
-template <bool GEN = true, bool BACKWARD = false>
+template <int FORM = FORM_GENERAL, bool BACKWARD = false>
 __global__ void __launch_bounds__(QBLOCK) k_residual_q(Fine G, QuadGrid Q, const double* p, const float* b, float* r,
                                                        int op, Ctl* ctl, double* partials, int gated) {
 #pragma clang fp contract(off)
@@ -740,7 +769,7 @@ __global__ void __launch_bounds__(QBLOCK) k_residual_q(Fine G, QuadGrid Q, const
         } else {
           uint8_t type[6];
           float it[6], a[6];
-          ghost_row<GEN>(G, 4 * qx + e, y, k, m, type, it, a);
+          ghost_row<FORM>(G, 4 * qx + e, y, k, m, type, it, a);
 #pragma unroll
           for (int f = 0; f < 6; ++f) {
             if (type[f] == 1) {
@@ -1050,7 +1079,7 @@ __global__ void __launch_bounds__(QBLOCK) k_divmetric_q(Fine G, QuadGrid Q, cons
 // Oettli-Prager backward error on quads (k_backward with four x-cells per
 // thread, the pressures of the quad and of its y and z neighbours as 32-byte
 // loads with indices clamped into the grid; k_backward's arithmetic per cell).
-template <bool GEN = true>
+template <int FORM = FORM_GENERAL>
 __global__ void __launch_bounds__(QBLOCK) k_backward_q(Fine G, QuadGrid Q, const double* p, const float* b,
                                                        const float* r, Ctl* ctl, double* partials) {
 #pragma clang fp contract(off)
@@ -1086,7 +1115,7 @@ __global__ void __launch_bounds__(QBLOCK) k_backward_q(Fine G, QuadGrid Q, const
       } else {
         uint8_t type[6];
         float it[6], a[6];
-        ghost_row<GEN>(G, 4 * qx + e, y, k, m, type, it, a);
+        ghost_row<FORM>(G, 4 * qx + e, y, k, m, type, it, a);
         for (int f = 0; f < 6; ++f) {
           if (type[f] == 1) acc += (double)a[f] * (pe + fabs(pn[f]));
           else if (type[f] == 2) acc += (double)a[f] * pe * (double)it[f];
@@ -1128,7 +1157,7 @@ __global__ void __launch_bounds__(QBLOCK) k_start_cold(size_t nquads, const floa
 // and so the coarse r, is the one-thread sum bit for bit, with twice the
 // waves in flight to overlap the loads with the arithmetic (38 -> 28 us at
 // 256x256x128). H: the restriction's quad grid for 128-thread halves.
-template <int ST, bool GEN = true>
+template <int ST, int FORM = FORM_GENERAL>
 __global__ void __launch_bounds__(QBLOCK) k_q_restrict2(Fine G, QuadGrid H, const typename Store<ST>::T* z,
                                                         const float* r, Level L0, Ctl* ctl) {
 #pragma clang fp contract(off)
@@ -1164,7 +1193,7 @@ __global__ void __launch_bounds__(QBLOCK) k_q_restrict2(Fine G, QuadGrid H, cons
     x_neighbours(H, valid, qx, zc, left, right, [&](int off) { return SV::ld(z, c0 + off); });
     // (invalid lanes: mq = 0, every row 0)
     float row[4];
-    quad_rows<GEN>(G, 4 * qx, y, k, mq, zc, left, right, ym, yp, zm, zp, row);
+    quad_rows<FORM>(G, 4 * qx, y, k, mq, zc, left, right, ym, yp, zm, zp, row);
 #pragma unroll
     for (int e = 0; e < 4; ++e) t[dy][e] = q_get(rq, e) - row[e];
   }
@@ -1202,7 +1231,7 @@ __global__ void __launch_bounds__(BLOCK) k_unpack(size_t n, const typename Store
 // ---------------------------------------------------------------- CG steps on quads
 // d = z (first) or z + beta d_old, q = A d, <d, q> (delta3d_mobile.rs:520-523, :460-465).
 // z is held in storage ST.
-template <int ST, bool GEN = true>
+template <int ST, int FORM = FORM_GENERAL>
 __global__ void __launch_bounds__(QBLOCK) k_q_spmv_dir(Fine G, QuadGrid Q, const typename Store<ST>::T* z, float* d0,
                                                        float* d1, float* q, Ctl* ctl, double* partials) {
 #pragma clang fp contract(off)
@@ -1242,7 +1271,7 @@ __global__ void __launch_bounds__(QBLOCK) k_q_spmv_dir(Fine G, QuadGrid Q, const
   double s = 0.0, unused = 0.0;
   if (valid) {
     float row[4];
-    quad_rows<GEN>(G, 4 * qx, y, k, mq, dc, left, right, ym, yp, zm, zp, row);
+    quad_rows<FORM>(G, 4 * qx, y, k, mq, dc, left, right, ym, yp, zm, zp, row);
     const float4 qo = make_float4(row[0], row[1], row[2], row[3]);
     st4(dnew, c0, dc);
     st4(q, c0, qo);
