@@ -30,6 +30,7 @@
 #include "kernels.h"
 #include "kernels_fast.h"
 #include "kernels_coarse.h"
+#include "kernels_rows.h"
 #include "kernels_step.h"
 #include "kernels_graded.h"
 #include "learned_internal.h"
@@ -268,8 +269,6 @@ inline bool prof_begin(fsp_solver* S, const char* name, hipStream_t stream, hipE
   } while (0)
 
 // Kernels templated on the V-cycle storage ST of the enclosing function.
-#define K_CGS (k_cgs<ST>)
-#define K_CRESTRICT (k_crestrict<ST>)
 #define K_CPROLONG (k_cprolong<ST>)
 #define K_GCGS(M) (k_gc_gs<M, ST>)
 template <int ST> using TS = typename Store<ST>::T;
@@ -344,6 +343,12 @@ bool quad_vcycle_ok(bool quad, const fsp_options& o) {
   return quad && o.smoother == FSP_SMOOTH_RBGS && o.pre_sweeps >= 1 && o.post_sweeps >= 1;
 }
 
+// The same with damped Jacobi (at least two pre-sweeps and one post-sweep: other
+// counts, which no configuration here uses, run a thread per cell).
+bool quad_jacobi_ok(bool quad, const fsp_options& o) {
+  return quad && o.smoother == FSP_SMOOTH_JACOBI && o.pre_sweeps >= 2 && o.post_sweeps >= 1;
+}
+
 struct Launch {
   fsp_solver* S;
   hipStream_t st;
@@ -400,7 +405,7 @@ struct Launch {
       if (!kindless(l)) last_generic = l;
     for (size_t l = 0; l < S->levels.size(); ++l) {
       Level& L = S->levels[l];
-      const bool kinds = (int)l <= last_generic, diag = !kindless((int)l);
+      const bool kinds = (int)l <= last_generic;
       const size_t nf = (size_t)(L.nx + 1) * L.ny * L.nz + (size_t)L.nx * (L.ny + 1) * L.nz +
                         (size_t)L.nx * L.ny * (L.nz + 1);
       if (l == 0) {
@@ -416,7 +421,7 @@ struct Launch {
         if (L.galerkin) FSP_LAUNCH(S, k_cgal, dim3(grid_for(std::max(nf, L.n))), st, S->levels[l - 1], L);
         else FSP_LAUNCH(S, k_cfaces, dim3(grid_for(nf)), st, S->levels[l - 1], L);
       }
-      if (diag) FSP_LAUNCH(S, k_cdiag, dim3(grid_for(L.n)), st, L);
+      if (L.c6) FSP_LAUNCH(S, k_r6_build, dim3(grid_for(L.n)), st, L);
       if (L.compact) FSP_LAUNCH(S, k_gc_build, dim3(grid_for(L.n)), st, L);
     }
     if (S->tail_pack) {
@@ -469,46 +474,54 @@ struct Launch {
     FSP_LAUNCH(S, k_fill_gated, dim3(grid_for(n)), st, x, n, v, S->ctl);
   }
 
-  // Sweeps on coarse level l; `x` is the current iterate (nullptr = zero),
-  // returns the buffer holding the result. Jacobi sweeps exist in f32 only.
+  // Sweeps from zero on coarse level l (row coefficients); returns the buffer
+  // holding the result. Jacobi sweeps exist in f32 only.
   template <int ST>
-  TS<ST>* coarse_sweeps(int l, TS<ST>* x, int count, bool forward, bool coarsest) {
+  TS<ST>* r6_down(int l, int count, bool coarsest) {
     Level& L = S->levels[l];
     TS<ST>* lx = reinterpret_cast<TS<ST>*>(L.x);
-    const int smoother = S->opt.smoother;
-    if (count == 0) {
-      if (!x) { fill_gated(L.x, L.n, 0.f); return lx; }
-      return x;
-    }
+    if (count == 0) { fill_gated(L.x, L.n, 0.f); return lx; }
     if constexpr (ST == ST_F32) {
-      if (smoother == FSP_SMOOTH_JACOBI) {
-        float* cur = x;
-        for (int s = 0; s < count; ++s) {
-          float* out = (cur == L.x) ? L.t : L.x;
-          FSP_LAUNCH(S, k_cjacobi, dim3(grid_for(L.n)), st, L, cur, out, S->ctl);
-          cur = out;
-        }
-        return cur;
-      }
-      if (x && x != L.x) FSP_LAUNCH(S, k_copy_gated, dim3(grid_for(L.n)), st, x, L.x, L.n, S->ctl);
-    }
-    // red-black Gauss-Seidel, in place on L.x
-    int first = x ? 0 : 1;
-    auto colour = [&](int c) {
-      FSP_LAUNCH_N(S, "k_cgs", K_CGS, dim3(grid_for(L.n)), st, L, lx, c, first, S->ctl);
-      first = 0;
-    };
-    if (coarsest) {
-      const int half = count / 2;
-      for (int s = 0; s < half; ++s) { colour(0); colour(1); }
-      if (count & 1) colour(0);
-      for (int s = 0; s < half; ++s) { colour(1); colour(0); }
-    } else {
-      for (int s = 0; s < count; ++s) {
-        if (forward) { colour(0); colour(1); } else { colour(1); colour(0); }
+      if (S->opt.smoother == FSP_SMOOTH_JACOBI) {
+        if (count == 1) FSP_LAUNCH(S, k_r6_zero, dim3(grid_for(L.n)), st, L, L.x, S->ctl);
+        else FSP_LAUNCH(S, k_r6_first, dim3(grid_for(L.n)), st, L, L.x, S->ctl);
+        return r6_jacobi(L, L.x, count - 2);
       }
     }
+    for (int p = 0; p < sweep_passes(coarsest, count); ++p) r6_gs<ST>(L, sweep_colour(coarsest, true, count, p), p == 0);
     return lx;
+  }
+  // Prolongation of the coarser level's xp onto x and `count` sweeps.
+  template <int ST>
+  TS<ST>* r6_up(int l, TS<ST>* x, const TS<ST>* xp, int count) {
+    Level& L = S->levels[l];
+    Level& C = S->levels[l + 1];
+    if constexpr (ST == ST_F32) {
+      if (S->opt.smoother == FSP_SMOOTH_JACOBI && count > 0) {
+        float* out = x == L.x ? L.t : L.x;
+        FSP_LAUNCH(S, k_r6_jacobi<true>, dim3(grid_for(L.n)), st, L, C, xp, (const float*)x, out, S->ctl);
+        return r6_jacobi(L, out, count - 1);
+      }
+    }
+    FSP_LAUNCH_N(S, "k_cprolong", K_CPROLONG, dim3(grid_for(L.n)), st, L, C, xp, x, S->ctl);
+    if (S->opt.smoother != FSP_SMOOTH_JACOBI)
+      for (int p = 0; p < sweep_passes(false, count); ++p) r6_gs<ST>(L, sweep_colour(false, false, count, p), false);
+    return x;
+  }
+  float* r6_jacobi(Level& L, float* cur, int count) {
+    for (int s = 0; s < count; ++s) {
+      float* out = cur == L.x ? L.t : L.x;
+      FSP_LAUNCH(S, k_r6_jacobi<false>, dim3(grid_for(L.n)), st, L, L, (const float*)nullptr, (const float*)cur, out,
+                 S->ctl);
+      cur = out;
+    }
+    return cur;
+  }
+  // red-black Gauss-Seidel, in place on L.x
+  template <int ST>
+  void r6_gs(Level& L, int colour, bool first) {
+    FSP_LAUNCH_N(S, "k_r6_gs", (k_r6_gs<ST>), dim3(grid_for(L.n)), st, L, reinterpret_cast<TS<ST>*>(L.x), colour,
+                 first ? 1 : 0, S->ctl);
   }
 
   // The tail levels in one workgroup: level tail_first's r is restricted;
@@ -517,7 +530,7 @@ struct Launch {
   void tail() {
     const TailSet T = tail_set();
     if (gc_tail_ok(S->opt)) k_gc_tail<ST><<<dim3(1), dim3(TAIL_THREADS), S->tail_lds, st>>>(T, S->ctl);
-    else k_tail<ST><<<dim3(1), dim3(TAIL_THREADS), S->tail_lds, st>>>(T, S->ctl);
+    else k_r6_tail<ST><<<dim3(1), dim3(TAIL_THREADS), S->tail_lds, st>>>(T, S->ctl);
   }
 
   static dim3 qgrid(const QuadGrid& Q) { return dim3((unsigned)(Q.nbx * Q.nby * Q.planes)); }
@@ -600,7 +613,7 @@ struct Launch {
       }
       const int sweeps = (l == last) ? S->opt.coarse_sweeps : S->opt.pre_sweeps;
       if (L.compact) xcur[l] = gc_sweeps<ST>(l, sweeps, l == last);
-      else xcur[l] = coarse_sweeps<ST>(l, nullptr, sweeps, true, l == last);
+      else xcur[l] = r6_down<ST>(l, sweeps, l == last);
       if (l < last) {
         Level& C = S->levels[l + 1];
         if (L.compact) {
@@ -611,7 +624,8 @@ struct Launch {
           FSP_LAUNCH_N(S, "k_gc_restrict", (k_gc_restrict2<ST>), qgrid(H), st, L, H, (const TS<ST>*)xcur[l], C,
                        S->ctl);
         } else {
-          FSP_LAUNCH_N(S, "k_crestrict", K_CRESTRICT, dim3(grid_for(C.n)), st, L, C, (const TS<ST>*)xcur[l], S->ctl);
+          FSP_LAUNCH_N(S, "k_r6_restrict", (k_r6_restrict<ST>), dim3(grid_for(8 * C.n)), st, L, C,
+                       (const TS<ST>*)xcur[l], S->ctl);
         }
       }
     }
@@ -637,9 +651,7 @@ struct Launch {
         xcur[l] = gc_ascend<ST>(l, xcur[l + 1]);
         continue;
       }
-      FSP_LAUNCH_N(S, "k_cprolong", K_CPROLONG, dim3(grid_for(L.n)), st, L, C, (const TS<ST>*)xcur[l + 1], xcur[l],
-                   S->ctl);
-      xcur[l] = coarse_sweeps<ST>(l, xcur[l], S->opt.post_sweeps, false, false);
+      xcur[l] = r6_up<ST>(l, xcur[l], xcur[l + 1], S->opt.post_sweeps);
     }
     return xcur[0];
   }
@@ -689,6 +701,48 @@ struct Launch {
     }
   }
 
+  // The same V-cycle with damped-Jacobi sweeps on quads (k_q_jacobi): the
+  // first two pre-sweeps in one launch, the prolongation within the first
+  // post-sweep. Returns the buffer holding z.
+  float* vcycle_quad_jacobi() {
+    const QuadGrid& Q = S->qfine;
+    const dim3 g((unsigned)(Q.nbx * Q.nby * Q.planes));
+    const Level L0 = S->levels.empty() ? Level{} : S->levels[0];
+    const float* none = nullptr;
+    float *a = S->z, *b = S->zt;
+    auto sweep = [&]() {
+      FSP_LAUNCH_FORM(S, "k_q_jacobi<0>", (k_q_jacobi<0, FORM_TABLE>), (k_q_jacobi<0, FORM_INDEX>),
+                      (k_q_jacobi<0, FORM_GENERAL>), g, QBLOCK, st, G, Q, (const float*)a, b, S->r, L0, none, S->ctl);
+      std::swap(a, b);
+    };
+    FSP_LAUNCH_FORM(S, "k_q_jacobi<1>", (k_q_jacobi<1, FORM_TABLE>), (k_q_jacobi<1, FORM_INDEX>),
+                    (k_q_jacobi<1, FORM_GENERAL>), g, QBLOCK, st, G, Q, none, a, S->r, L0, none, S->ctl);
+    for (int s = 2; s < S->opt.pre_sweeps; ++s) sweep();
+    int done = 0;
+    if (!S->levels.empty()) {
+      restrict_quads<ST_F32>(a, L0);
+      const float* x0 = coarse_cycle<ST_F32>();
+      FSP_LAUNCH_FORM(S, "k_q_jacobi<2>", (k_q_jacobi<2, FORM_TABLE>), (k_q_jacobi<2, FORM_INDEX>),
+                      (k_q_jacobi<2, FORM_GENERAL>), g, QBLOCK, st, G, Q, (const float*)a, b, S->r, L0, x0, S->ctl);
+      std::swap(a, b);
+      done = 1;
+    }
+    for (int s = done; s < S->opt.post_sweeps; ++s) sweep();
+    return a;
+  }
+
+  // The residual of z on quads restricted to the first coarse level (k_q_restrict2).
+  template <int ST>
+  void restrict_quads(const TS<ST>* z, const Level& L0) {
+    // the restriction's grid for 128-thread halves
+    QuadGrid H = S->qrestr;
+    H.RY = (QBLOCK / 2) / H.QX;
+    H.nby = (H.rows + H.RY - 1) / H.RY;
+    const dim3 gr((unsigned)(H.nbx * H.nby * H.planes));
+    FSP_LAUNCH_FORM(S, "k_q_restrict", (k_q_restrict2<ST, FORM_TABLE>), (k_q_restrict2<ST, FORM_INDEX>),
+                    (k_q_restrict2<ST, FORM_GENERAL>), gr, BLOCK, st, G, H, z, (const float*)S->r, L0, S->ctl);
+  }
+
   bool quad_vcycle() const { return quad_vcycle_ok(S->quad, S->opt); }
 
   // The V-cycle on quads with red-black smoothing: first pass from zero (or,
@@ -724,13 +778,7 @@ struct Launch {
     int passes = 2 * S->opt.post_sweeps;
     int done = 0;
     if (!S->levels.empty()) {
-      // the restriction's grid for 128-thread halves (k_q_restrict2)
-      QuadGrid H = S->qrestr;
-      H.RY = (QBLOCK / 2) / H.QX;
-      H.nby = (H.rows + H.RY - 1) / H.RY;
-      const dim3 gr((unsigned)(H.nbx * H.nby * H.planes));
-      FSP_LAUNCH_FORM(S, "k_q_restrict", (k_q_restrict2<ST, FORM_TABLE>), (k_q_restrict2<ST, FORM_INDEX>), (k_q_restrict2<ST, FORM_GENERAL>), gr, BLOCK, st, G, H,
-                     (const TS<ST>*)z, (const float*)S->r, L0, S->ctl);
+      restrict_quads<ST>(z, L0);
       const TS<ST>* x0 = coarse_cycle<ST>();
       const int op = passes == 1 ? dot_op : -1;
       FSP_LAUNCH_FORM(S, "k_q_gs<2>", (k_q_gs<2, ST, FORM_TABLE>), (k_q_gs<2, ST, FORM_INDEX>), (k_q_gs<2, ST, FORM_GENERAL>), g, BLOCK, st, G, Q,
@@ -775,12 +823,7 @@ struct Launch {
     for (int s = 1; s < S->opt.pre_sweeps; ++s) sweep(0, none, -1);
     const TS<ST>* x0 = none;
     if (!S->levels.empty()) {
-      QuadGrid H = S->qrestr;
-      H.RY = (QBLOCK / 2) / H.QX;
-      H.nby = (H.rows + H.RY - 1) / H.RY;
-      const dim3 gr((unsigned)(H.nbx * H.nby * H.planes));
-      FSP_LAUNCH_FORM(S, "k_q_restrict", (k_q_restrict2<ST, FORM_TABLE>), (k_q_restrict2<ST, FORM_INDEX>), (k_q_restrict2<ST, FORM_GENERAL>), gr, BLOCK, st, G, H,
-                     (const TS<ST>*)a, (const float*)S->r, L0, S->ctl);
+      restrict_quads<ST>(a, L0);
       x0 = coarse_cycle<ST>();
     }
     for (int s = 0; s < S->opt.post_sweeps; ++s)
@@ -829,10 +872,11 @@ struct Launch {
       });
       return;
     }
-    vcycle();
-    FSP_LAUNCH(S, k_dot, dim3(grid_for(G.n)), st, G.n, S->r, S->z, op, 1, S->ctl, S->partials);
-    FSP_FINISH(S, st, op, dim3(grid_for(G.n)), false, 1);
     S->zres = S->z;
+    if (quad_jacobi_ok(S->quad, S->opt)) S->zres = vcycle_quad_jacobi();
+    else vcycle();
+    FSP_LAUNCH(S, k_dot, dim3(grid_for(G.n)), st, G.n, S->r, S->zres, op, 1, S->ctl, S->partials);
+    FSP_FINISH(S, st, op, dim3(grid_for(G.n)), false, 1);
   }
 
   // The preconditioned vector in f32 (tests and the device entry point).
@@ -1738,7 +1782,8 @@ fsp_status fsp_create(const fsp_domain* d, const fsp_options* o, fsp_solver** ou
   }
   if (opt.preconditioner == FSP_PRECOND_LEARNED && opt.learned_vcycle && !quad_vcycle_ok(S->quad, opt))
     return fail(FSP_INVALID);
-  if (opt.preconditioner != FSP_PRECOND_JACOBI && quad_vcycle_ok(S->quad, opt) && (st = dalloc(S, &S->precv, S->n)))
+  if (opt.preconditioner != FSP_PRECOND_JACOBI && (quad_vcycle_ok(S->quad, opt) || quad_jacobi_ok(S->quad, opt)) &&
+      (st = dalloc(S, &S->precv, S->n)))
     return fail(st);
   // dynamic LDS a workgroup may have (160 KiB on gfx950)
   int lds_attr = 0;
@@ -1749,11 +1794,9 @@ fsp_status fsp_create(const fsp_domain* d, const fsp_options* o, fsp_solver** ou
   for (int t = (int)S->levels.size() - 1; t >= 0; --t) {
     if (S->levels[t].n > (size_t)TAIL_CELLS || (int)S->levels.size() - t > TAIL_MAX_LEVELS) break;
     const int count = (int)S->levels.size() - t;
-    const size_t bytes = gc_tail_ok(opt) ? gc_tail_lds_bytes(&S->levels[t], count)
-                                         : tail_lds_bytes(&S->levels[t], count, opt.smoother);
-    if (bytes > (gc_tail_ok(opt) ? std::min(GC_TAIL_LDS_FLOATS * sizeof(float), lds_limit - TAIL_STATIC_LDS)
-                                 : TAIL_LDS_FLOATS * sizeof(float)))
-      break;
+    const bool gc = gc_tail_ok(opt);
+    const size_t bytes = gc ? gc_tail_lds_bytes(&S->levels[t], count) : r6_tail_lds_bytes(&S->levels[t], count);
+    if (bytes > std::min(GC_TAIL_LDS_FLOATS * sizeof(float), lds_limit - TAIL_STATIC_LDS)) break;
     S->tail_first = t;
     S->tail_lds = bytes;
   }
@@ -1782,6 +1825,11 @@ fsp_status fsp_create(const fsp_domain* d, const fsp_options* o, fsp_solver** ou
       if (l + 1 < (int)S->levels.size()) S->cqr[l] = make_q(L.nx / 4, L.ny / 2, L.nz / 2);
     }
   }
+  // every other level above the compact tail: row coefficients
+  for (int l = 0; l < (int)S->levels.size(); ++l)
+    if (!S->levels[l].compact && !(gc_tail_ok(opt) && l >= S->tail_first) &&
+        (st = dalloc(S, &S->levels[l].c6, 6 * S->levels[l].n)))
+      return fail(st);
   // 16-bit V-cycle storage exists on the red-black quad path only
   if (opt.vcycle_storage != FSP_STORE_F32 &&
       !(opt.preconditioner != FSP_PRECOND_JACOBI && quad_vcycle_ok(S->quad, opt)))

@@ -145,6 +145,7 @@ struct Level {
   float* r;
   float* t;
   float* dd;             // Galerkin levels: Dirichlet part of the diagonal (units of inv)
+  float* c6;             // row coefficients (kernels_rows.h): 6 x n, null on compact levels and the compact tail
   int galerkin;          // 1: P^T A P / 16 coarse operator, 0: re-discretised
   int compact;           // 1: smoothed by the compact quad kernels (Galerkin, binary16 couplings)
   uint16_t* cx;          // compact levels: binary16 coupling of each cell's x- face

@@ -975,39 +975,6 @@ __device__ __forceinline__ void ldecode(const Level& L, size_t c, int& i, int& j
   j = (int)(t - (uint32_t)k * ny);
 }
 
-// row_sums (delta3d_multigrid.rs:216-255); x == nullptr gives the diagonal.
-// x is held in storage ST.
-template <int ST = ST_F32>
-__device__ __forceinline__ float coarse_row(const Level& L, int i, int j, int k, size_t c,
-                                            const typename Store<ST>::T* x) {
-#pragma clang fp contract(off)
-  using SV = Store<ST>;
-  if (L.kind[c] <= 0) return 0.f;
-  const float pc = x ? SV::ld(x, c) : 0.f;
-  float acc = 0.f;
-  const int nx = L.nx, ny = L.ny, nz = L.nz;
-  const size_t plane = (size_t)nx * ny;
-  const bool gal = L.galerkin != 0;
-  auto face = [&](float a, bool has, size_t n, bool top) {
-    if (a == 0.f) return;
-    if (has) {
-      const int8_t kn = L.kind[n];
-      if (kn > 0) acc += x ? a * (pc - SV::ld(x, n)) : a;
-      else if (!gal && kn < 0) acc += 2.0f * a * (x ? pc : 1.0f);
-    } else if (!gal && top) {
-      acc += 2.0f * a * (x ? pc : 1.0f);
-    }
-  };
-  face(L.ou[((size_t)k * ny + j) * (nx + 1) + i], i > 0, c - 1, false);
-  face(L.ou[((size_t)k * ny + j) * (nx + 1) + i + 1], i + 1 < nx, c + 1, false);
-  face(L.ov[((size_t)k * (ny + 1) + j) * nx + i], j > 0, c - nx, false);
-  face(L.ov[((size_t)k * (ny + 1) + j + 1) * nx + i], j + 1 < ny, c + nx, false);
-  face(L.ow[((size_t)k * ny + j) * nx + i], k > 0, c - plane, false);
-  face(L.ow[((size_t)(k + 1) * ny + j) * nx + i], k + 1 < nz, c + plane, true);
-  if (gal) acc += x ? L.dd[c] * pc : L.dd[c];
-  return acc * L.inv;
-}
-
 // kind of the first coarse level from the fine cells (delta3d_multigrid.rs:153-169, :357-367)
 __global__ void __launch_bounds__(BLOCK) k_ckind_fine(Fine G, Level L) {
   FSP_FOR(c, L.n) {
@@ -1184,56 +1151,6 @@ __global__ void __launch_bounds__(BLOCK) k_cgal(Level F, Level L) {
   }
 }
 
-__global__ void __launch_bounds__(BLOCK) k_cdiag(Level L) {
-  FSP_FOR(c, L.n) {
-    int i, j, k;
-    ldecode(L, c, i, j, k);
-    L.diag[c] = coarse_row<ST_F32>(L, i, j, k, c, nullptr);
-  }
-}
-
-// Damped Jacobi on a coarse level (delta3d_multigrid.rs:290-299): xout = xin +
-// w (r - L xin)/diag; xin == nullptr means xin = 0.
-__global__ void __launch_bounds__(BLOCK) k_cjacobi(Level L, const float* xin, float* xout, Ctl* ctl) {
-#pragma clang fp contract(off)
-  if (!ctl->active) return;
-  const float omega = 6.0f / 7.0f;
-  FSP_FOR(c, L.n) {
-    int i, j, k;
-    ldecode(L, c, i, j, k);
-    const float t = xin ? coarse_row(L, i, j, k, c, xin) : 0.f;
-    float xc = xin ? xin[c] : 0.f;
-    const float dg = L.diag[c];
-    if (dg > 0.f) xc += omega * (L.r[c] - t) / dg;
-    xout[c] = xc;
-  }
-}
-// One colour of red-black Gauss-Seidel on a coarse level, in place; x and
-// L.r are held in storage ST.
-template <int ST>
-__global__ void __launch_bounds__(BLOCK) k_cgs(Level L, typename Store<ST>::T* x, int colour, int first, Ctl* ctl) {
-#pragma clang fp contract(off)
-  using SV = Store<ST>;
-  if (!ctl->active) return;
-  const typename SV::T* lr = reinterpret_cast<const typename SV::T*>(L.r);
-  FSP_FOR(c, L.n) {
-    int i, j, k;
-    ldecode(L, c, i, j, k);
-    const int col = (i + j + k) & 1;
-    const float dg = L.diag[c];
-    if (first) {
-      if (col != colour) { SV::st(x, c, 0.f); continue; }
-      SV::st(x, c, dg > 0.f ? SV::ld(lr, c) / dg : 0.f);
-      continue;
-    }
-    if (col != colour) continue;
-    if (dg > 0.f) {
-      const float t = coarse_row<ST>(L, i, j, k, c, x);
-      SV::st(x, c, SV::ld(x, c) + (SV::ld(lr, c) - t) / dg);
-    }
-  }
-}
-
 // Residual of the fine level restricted to the first coarse level
 // (delta3d_multigrid.rs:406-411, restrict3 :258-272).
 __global__ void __launch_bounds__(BLOCK) k_restrict_fine(Fine G, Level L, const float* z, const float* r, Ctl* ctl) {
@@ -1249,26 +1166,6 @@ __global__ void __launch_bounds__(BLOCK) k_restrict_fine(Fine G, Level L, const 
       s += r[f] - apply_row(G, fi, fj, fk, f, G.mask[f], z);
     }
     L.r[c] = 0.125f * s;
-  }
-}
-// Coarse residual restricted one level down (delta3d_multigrid.rs:312-321).
-template <int ST>
-__global__ void __launch_bounds__(BLOCK) k_crestrict(Level F, Level L, const typename Store<ST>::T* xf, Ctl* ctl) {
-#pragma clang fp contract(off)
-  using SV = Store<ST>;
-  if (!ctl->active) return;
-  const typename SV::T* fr = reinterpret_cast<const typename SV::T*>(F.r);
-  typename SV::T* lr = reinterpret_cast<typename SV::T*>(L.r);
-  FSP_FOR(c, L.n) {
-    int i, j, k;
-    ldecode(L, c, i, j, k);
-    float s = 0.f;
-    for (int ch = 0; ch < 8; ++ch) {
-      const int fi = 2 * i + (ch & 1), fj = 2 * j + ((ch >> 1) & 1), fk = 2 * k + ((ch >> 2) & 1);
-      const size_t f = lidx(F, fi, fj, fk);
-      s += SV::ld(fr, f) - coarse_row<ST>(F, fi, fj, fk, f, xf);
-    }
-    SV::st(lr, c, 0.125f * s);
   }
 }
 // Prolongation by injection (delta3d_multigrid.rs:275-287); on the fine

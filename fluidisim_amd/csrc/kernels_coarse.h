@@ -837,27 +837,19 @@ __device__ __forceinline__ void gct_sweeps(float* lds, const GcTailLvl& L, int c
     gct_coarsest_wave<ST>(lds, L, count, from_zero);
     return;
   }
-  // the colours of the sequence: red-black forward, black-red backward, or on
-  // the coarsest level the palindrome of both halves
-  const int half = coarsest ? count / 2 : 0, odd = coarsest ? count & 1 : 0;
-  const int passes = coarsest ? 4 * half + odd : 2 * count;
-  auto colour = [&](int i) -> int {
-    if (!coarsest) return forward ? (i & 1) : 1 - (i & 1);
-    if (i < 2 * half + odd) return i & 1;
-    return 1 - ((i - 2 * half - odd) & 1);
-  };
+  const int passes = sweep_passes(coarsest, count);
   if ((L.nx & 1) == 0 && L.n <= 2 * GctCells<ST>::S * TAIL_THREADS) {
     GctCells<ST> cells;
     cells.load(lds, L);
     for (int i = 0; i < passes; ++i) {
-      if (colour(i) == 0) cells.template pass<0>(lds, L, fz);
+      if (sweep_colour(coarsest, forward, count, i) == 0) cells.template pass<0>(lds, L, fz);
       else cells.template pass<1>(lds, L, fz);
       fz = false;
     }
     return;
   }
   for (int i = 0; i < passes; ++i) {
-    gct_pass<ST>(lds, L, colour(i), fz);
+    gct_pass<ST>(lds, L, sweep_colour(coarsest, forward, count, i), fz);
     fz = false;
   }
 }

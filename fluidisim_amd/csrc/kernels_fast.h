@@ -1146,6 +1146,73 @@ __global__ void __launch_bounds__(QBLOCK) k_start_cold(size_t nquads, const floa
   reduce_finish<false>(s, unused, op, ctl, partials);
 }
 
+// ---------------------------------------------------------------- damped Jacobi
+// Sweeps of the fine level on quads (k_fjacobi's arithmetic,
+// delta3d_multigrid.rs:398-405; the rows' factors from G.precv): zout = zin + w prec (r - A zin). MODE 2:
+// zin is first prolonged from the first coarse level (k_prolong_fine's arithmetic) on the fly. MODE 1: the
+// first two sweeps from zero; the first is local (w prec r), so its neighbours'
+// values are formed from their r and factors. At 128x64x96 with a cut bottom
+// a sweep takes 6.6 us against 10.9 with a thread per cell, the first two 8.0 against 21.8.
+template <int MODE, int FORM>
+__global__ void __launch_bounds__(QBLOCK) k_q_jacobi(Fine G, QuadGrid Q, const float* zin, float* zout, const float* r,
+                                                     Level L0, const float* xc, Ctl* ctl) {
+#pragma clang fp contract(off)
+  if (!ctl->active) return;
+  const float omega = 6.0f / 7.0f;
+  int qx, y, k;
+  const bool valid = quad_coords(Q, qx, y, k);
+  const size_t plane = (size_t)G.nx * G.ny;
+  const size_t c0 = valid ? ((size_t)k * G.ny + y) * G.nx + 4 * (size_t)qx : 0;
+  auto first = [&](float prec, float rv) { return prec > 0.f ? omega * prec * rv : 0.f; };
+  // the iterate of quad c in row yy, plane kk (MODE 2: prolonged; rows that the
+  // prolongation zeroes have no coupling and no factor)
+  auto iterate = [&](size_t c, int yy, int kk) {
+    if (MODE == 1) {
+      const float4 p = ld4(G.precv, c), v = ld4(r, c);
+      return make_float4(first(p.x, v.x), first(p.y, v.y), first(p.z, v.z), first(p.w, v.w));
+    }
+    float4 v = ld4(zin, c);
+    if (MODE == 2) {
+      const float2 a = *reinterpret_cast<const float2*>(xc + lidx(L0, 2 * qx, yy >> 1, kk >> 1));
+      v.x = v.x + a.x; v.y = v.y + a.x; v.z = v.z + a.y; v.w = v.w + a.y;
+    }
+    return v;
+  };
+  float4 zc = f4zero(), ym = f4zero(), yp = f4zero(), zm = f4zero(), zp = f4zero(), rq = f4zero(), pq = f4zero();
+  uint32_t mq = 0;
+  if (valid) {
+    mq = *reinterpret_cast<const uint32_t*>(G.mask + c0);
+    rq = ld4(r, c0);
+    pq = ld4(G.precv, c0);
+    zc = iterate(c0, y, k);
+    if (y > 0) ym = iterate(c0 - G.nx, y - 1, k);
+    if (y + 1 < G.ny) yp = iterate(c0 + G.nx, y + 1, k);
+    if (k > 0) zm = iterate(c0 - plane, y, k - 1);
+    if (k + 1 < G.nz) zp = iterate(c0 + plane, y, k + 1);
+  }
+  float left, right;
+  x_neighbours(Q, valid, qx, zc, left, right, [&](int off) {
+    const size_t c = c0 + off;
+    if (MODE == 1) return first(G.precv[c], r[c]);
+    float v = zin[c];
+    if (MODE == 2) v = v + xc[lidx(L0, (4 * qx + off) >> 1, y >> 1, k >> 1)];
+    return v;
+  });
+  if (!valid) return;
+  float row[4];
+  quad_rows<FORM>(G, 4 * qx, y, k, mq, zc, left, right, ym, yp, zm, zp, row);
+  float4 out = zc;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float prec = q_get(pq, e);
+    float z = q_get(zc, e);
+    if (MODE == 2 && !prec_positive((uint8_t)(mq >> (8 * e)))) z = 0.f;
+    if (prec > 0.f) z += omega * prec * (q_get(rq, e) - row[e]);
+    q_set(out, e, z);
+  }
+  st4(zout, c0, out);
+}
+
 // ---------------------------------------------------------------- residual + restriction
 // The residual t = r - A z of the 16 fine cells of (fine quad column qx,
 // coarse row J, coarse plane K), summed per coarse cell in the reference's
@@ -1310,7 +1377,6 @@ __global__ void __launch_bounds__(QBLOCK) k_q_update(size_t nquads, double* p, f
 constexpr int TAIL_THREADS = 1024;
 constexpr int TAIL_MAX_LEVELS = 8;
 constexpr int TAIL_CELLS = 4096;                // largest first level of the tail
-constexpr int TAIL_LDS_FLOATS = 64 * 1024 / 4;  // LDS of the tail workgroup
 // LDS of the compact tail workgroup: the levels from one of TAIL_CELLS cells
 // down (4096 + 512 + ... = 4681 cells of 6 floats, 110 KiB). A closed box of
 // 64^3 with its coarsest level of 16^3 ran that level's 16 colour passes as
@@ -1325,220 +1391,16 @@ struct TailSet {
   int pre, post, coarse;
 };
 
-// A tail level inside LDS: sizes and float offsets of its arrays.
-struct TailLvl {
-  int nx, ny, nz, n;
-  float inv;
-  int o_kind, o_ou, o_ov, o_ow, o_diag, o_x, o_r, o_t, o_dd;
-  int galerkin;
-};
-
-__device__ __forceinline__ void tail_decode(const TailLvl& L, int c, int& i, int& j, int& k) {
-  const int t = c / L.nx;
-  i = c - t * L.nx;
-  k = t / L.ny;
-  j = t - k * L.ny;
+// The colours of a level's red-black sweeps: red-black on the way down,
+// black-red on the way up, and on the coarsest level the palindrome of both halves
+// (count passes of each colour in all).
+__host__ __device__ inline int sweep_passes(bool coarsest, int count) {
+  return coarsest ? 4 * (count / 2) + (count & 1) : 2 * count;
 }
-
-// row_sums (delta3d_multigrid.rs:216-255) on LDS arrays; x at offset xo.
-__device__ __forceinline__ float tail_row(const float* lds, const TailLvl& L, int i, int j, int k, int c, int xo) {
-#pragma clang fp contract(off)
-  const int8_t* kind = reinterpret_cast<const int8_t*>(lds + L.o_kind);
-  if (kind[c] <= 0) return 0.f;
-  const float* x = lds + xo;
-  const float* ou = lds + L.o_ou;
-  const float* ov = lds + L.o_ov;
-  const float* ow = lds + L.o_ow;
-  const float pc = x[c];
-  float acc = 0.f;
-  const int nx = L.nx, ny = L.ny, nz = L.nz, plane = nx * ny;
-  const bool gal = L.galerkin != 0;
-  auto face = [&](float a, bool has, int n, bool top) {
-    if (a == 0.f) return;
-    if (has) {
-      const int8_t kn = kind[n];
-      if (kn > 0) acc += a * (pc - x[n]);
-      else if (!gal && kn < 0) acc += 2.0f * a * pc;
-    } else if (!gal && top) {
-      acc += 2.0f * a * pc;
-    }
-  };
-  face(ou[(k * ny + j) * (nx + 1) + i], i > 0, c - 1, false);
-  face(ou[(k * ny + j) * (nx + 1) + i + 1], i + 1 < nx, c + 1, false);
-  face(ov[(k * (ny + 1) + j) * nx + i], j > 0, c - nx, false);
-  face(ov[(k * (ny + 1) + j + 1) * nx + i], j + 1 < ny, c + nx, false);
-  face(ow[(k * ny + j) * nx + i], k > 0, c - plane, false);
-  face(ow[((k + 1) * ny + j) * nx + i], k + 1 < nz, c + plane, true);
-  if (gal) acc += lds[L.o_dd + c] * pc;
-  return acc * L.inv;
-}
-
-// One smoothing pass on tail level l. RBGS: colour `col` in place (first: x
-// starts at zero). Jacobi: t = x + w(r - Lx)/diag, then x = t. Stored values
-// are rounded to storage ST.
-template <int ST>
-__device__ __forceinline__ void tail_pass(float* lds, const TailLvl& L, int smoother, int col, bool first) {
-#pragma clang fp contract(off)
-  using SV = Store<ST>;
-  float* x = lds + L.o_x;
-  const float* r = lds + L.o_r;
-  const float* diag = lds + L.o_diag;
-  if (smoother == 0) {
-    float* t = lds + L.o_t;
-    const float omega = 6.0f / 7.0f;
-    for (int c = threadIdx.x; c < L.n; c += TAIL_THREADS) {
-      int i, j, k;
-      tail_decode(L, c, i, j, k);
-      const float row = first ? 0.f : tail_row(lds, L, i, j, k, c, L.o_x);
-      float xc = first ? 0.f : x[c];
-      const float dg = diag[c];
-      if (dg > 0.f) xc = SV::rnd(xc + omega * (r[c] - row) / dg);
-      t[c] = xc;
-    }
-    __syncthreads();
-    for (int c = threadIdx.x; c < L.n; c += TAIL_THREADS) x[c] = t[c];
-    __syncthreads();
-    return;
-  }
-  for (int c = threadIdx.x; c < L.n; c += TAIL_THREADS) {
-    int i, j, k;
-    tail_decode(L, c, i, j, k);
-    const float dg = diag[c];
-    if (((i + j + k) & 1) != col) {
-      if (first) x[c] = 0.f;
-      continue;
-    }
-    if (first) { x[c] = dg > 0.f ? SV::rnd(r[c] / dg) : 0.f; continue; }
-    if (dg > 0.f) x[c] = SV::rnd(x[c] + (r[c] - tail_row(lds, L, i, j, k, c, L.o_x)) / dg);
-  }
-  __syncthreads();
-}
-
-template <int ST>
-__device__ __forceinline__ void tail_sweeps(float* lds, const TailLvl& L, int smoother, int count, bool forward,
-                                            bool coarsest, bool from_zero) {
-  if (count == 0) {
-    if (from_zero) {
-      for (int c = threadIdx.x; c < L.n; c += TAIL_THREADS) lds[L.o_x + c] = 0.f;
-      __syncthreads();
-    }
-    return;
-  }
-  bool fz = from_zero;
-  if (smoother == 0) {
-    for (int s = 0; s < count; ++s) { tail_pass<ST>(lds, L, 0, 0, fz); fz = false; }
-    return;
-  }
-  if (coarsest) {
-    const int half = count / 2;
-    for (int s = 0; s < half; ++s) { tail_pass<ST>(lds, L, 1, 0, fz); fz = false; tail_pass<ST>(lds, L, 1, 1, false); }
-    if (count & 1) { tail_pass<ST>(lds, L, 1, 0, fz); fz = false; }
-    for (int s = 0; s < half; ++s) { tail_pass<ST>(lds, L, 1, 1, fz); fz = false; tail_pass<ST>(lds, L, 1, 0, false); }
-    return;
-  }
-  for (int s = 0; s < count; ++s) {
-    const int c0 = forward ? 0 : 1;
-    tail_pass<ST>(lds, L, 1, c0, fz);
-    fz = false;
-    tail_pass<ST>(lds, L, 1, 1 - c0, false);
-  }
-}
-
-// Descends and ascends every tail level in LDS (coarse_cycle3,
-// delta3d_multigrid.rs:303-332), starting from the first tail level whose r
-// is already restricted; writes that level's x back to global.
-// Level vectors x and r are held in storage ST, in global memory and (as
-// rounded f32 values) in LDS.
-template <int ST>
-__global__ void __launch_bounds__(TAIL_THREADS) k_tail(TailSet T, Ctl* ctl) {
-#pragma clang fp contract(off)
-  using SV = Store<ST>;
-  if (!ctl->active) return;
-  extern __shared__ float lds[];
-  __shared__ TailLvl tl[TAIL_MAX_LEVELS];
-  if (threadIdx.x == 0) {
-    int off = 0;
-    for (int l = 0; l < T.count; ++l) {
-      const Level& g = T.lv[l];
-      TailLvl& L = tl[l];
-      L.nx = g.nx; L.ny = g.ny; L.nz = g.nz; L.n = (int)g.n; L.inv = g.inv;
-      L.o_kind = off; off += (L.n + 3) / 4;
-      L.o_ou = off; off += (g.nx + 1) * g.ny * g.nz;
-      L.o_ov = off; off += g.nx * (g.ny + 1) * g.nz;
-      L.o_ow = off; off += g.nx * g.ny * (g.nz + 1);
-      L.o_diag = off; off += L.n;
-      L.o_x = off; off += L.n;
-      L.o_r = off; off += L.n;
-      if (T.smoother == 0) { L.o_t = off; off += L.n; } else { L.o_t = L.o_x; }
-      L.galerkin = g.galerkin;
-      if (g.galerkin) { L.o_dd = off; off += L.n; } else { L.o_dd = L.o_diag; }
-    }
-  }
-  __syncthreads();
-  for (int l = 0; l < T.count; ++l) {
-    const Level& g = T.lv[l];
-    const TailLvl L = tl[l];
-    int8_t* kind = reinterpret_cast<int8_t*>(lds + L.o_kind);
-    const int nu = (g.nx + 1) * g.ny * g.nz, nv = g.nx * (g.ny + 1) * g.nz, nw = g.nx * g.ny * (g.nz + 1);
-    for (int q = threadIdx.x; q < L.n; q += TAIL_THREADS) {
-      kind[q] = g.kind[q];
-      lds[L.o_diag + q] = g.diag[q];
-      if (L.galerkin) lds[L.o_dd + q] = g.dd[q];
-    }
-    for (int q = threadIdx.x; q < nu; q += TAIL_THREADS) lds[L.o_ou + q] = g.ou[q];
-    for (int q = threadIdx.x; q < nv; q += TAIL_THREADS) lds[L.o_ov + q] = g.ov[q];
-    for (int q = threadIdx.x; q < nw; q += TAIL_THREADS) lds[L.o_ow + q] = g.ow[q];
-    if (l == 0)
-      for (int q = threadIdx.x; q < L.n; q += TAIL_THREADS)
-        lds[L.o_r + q] = SV::ld(reinterpret_cast<const typename SV::T*>(g.r), q);
-  }
-  __syncthreads();
-  const int last = T.count - 1;
-  for (int l = 0; l <= last; ++l) {
-    const TailLvl L = tl[l];
-    tail_sweeps<ST>(lds, L, T.smoother, l == last ? T.coarse : T.pre, true, l == last, true);
-    if (l < last) {
-      const TailLvl C = tl[l + 1];
-      for (int c = threadIdx.x; c < C.n; c += TAIL_THREADS) {
-        int i, j, k;
-        tail_decode(C, c, i, j, k);
-        float s = 0.f;
-        for (int ch = 0; ch < 8; ++ch) {
-          const int fi = 2 * i + (ch & 1), fj = 2 * j + ((ch >> 1) & 1), fk = 2 * k + ((ch >> 2) & 1);
-          const int f = (fk * L.ny + fj) * L.nx + fi;
-          s += lds[L.o_r + f] - tail_row(lds, L, fi, fj, fk, f, L.o_x);
-        }
-        lds[C.o_r + c] = SV::rnd(0.125f * s);
-      }
-      __syncthreads();
-    }
-  }
-  for (int l = last - 1; l >= 0; --l) {
-    const TailLvl L = tl[l];
-    const TailLvl C = tl[l + 1];
-    for (int c = threadIdx.x; c < L.n; c += TAIL_THREADS) {
-      int i, j, k;
-      tail_decode(L, c, i, j, k);
-      lds[L.o_x + c] = SV::rnd(lds[L.o_x + c] + lds[C.o_x + ((k >> 1) * C.ny + (j >> 1)) * C.nx + (i >> 1)]);
-    }
-    __syncthreads();
-    tail_sweeps<ST>(lds, L, T.smoother, T.post, false, false, false);
-  }
-  const TailLvl L0 = tl[0];
-  for (int q = threadIdx.x; q < L0.n; q += TAIL_THREADS)
-    SV::st(reinterpret_cast<typename SV::T*>(T.lv[0].x), q, lds[L0.o_x + q]);
-}
-
-// LDS bytes k_tail needs for the given levels.
-inline size_t tail_lds_bytes(const Level* lv, int count, int smoother) {
-  size_t floats = 0;
-  for (int l = 0; l < count; ++l) {
-    const Level& g = lv[l];
-    const size_t nu = (size_t)(g.nx + 1) * g.ny * g.nz, nv = (size_t)g.nx * (g.ny + 1) * g.nz,
-                 nw = (size_t)g.nx * g.ny * (g.nz + 1);
-    floats += (g.n + 3) / 4 + nu + nv + nw + (smoother == 0 ? 4 : 3) * g.n + (g.galerkin ? g.n : 0);
-  }
-  return floats * sizeof(float);
+__host__ __device__ inline int sweep_colour(bool coarsest, bool forward, int count, int p) {
+  if (!coarsest) return forward ? (p & 1) : 1 - (p & 1);
+  const int mid = 2 * (count / 2) + (count & 1);
+  return p < mid ? (p & 1) : 1 - ((p - mid) & 1);
 }
 
 }  // namespace fsp

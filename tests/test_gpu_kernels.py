@@ -116,3 +116,23 @@ def test_scattered_water_matches_the_f64_oracle(share):
     # the oracle stops at a relative residual of 1e-6 on a system whose smallest
     # theta (0.11) keeps its condition below 100
     assert np.linalg.norm(p[m] - p64[m]) <= 1e-4 * np.linalg.norm(p64[m])
+
+
+@pytest.mark.parametrize("size,levels,sweeps", [
+    ((48, 32, 32), -1, (2, 2, 8)),   # 24 x 16 x 16 above the tail
+    ((48, 32, 32), -1, (3, 1, 5)),   # an odd number of sweeps: the other buffer
+    ((48, 32, 32), -1, (1, 2, 1)),   # one pre-sweep: the fine level a thread per cell
+    ((48, 32, 32), -1, (2, 0, 0)),   # no post-sweep, no coarsest sweep
+    ((32, 32, 32), 1, (2, 2, 8)),    # 16^3: the tail's largest level
+    ((52, 36, 40), 2, (2, 3, 2)),    # 26 x 20 x 18 over 13 x 10 x 9: odd rows
+    ((34, 32, 32), -1, (2, 2, 3)),   # rows that do not split into quads
+    ((36, 34, 38), 1, (4, 2, 3)),    # 18 x 19 x 17 as the coarsest level above the tail
+], ids=str)
+@pytest.mark.parametrize("smoother", [_lib.SMOOTH_JACOBI, _lib.SMOOTH_RBGS])
+@pytest.mark.parametrize("coarse_operator", [_lib.COARSE_REDISCRETISED, _lib.COARSE_GALERKIN])
+def test_levels_of_row_coefficients_match_the_oracle(size, levels, sweeps, smoother, coarse_operator):
+    if smoother == _lib.SMOOTH_RBGS and 0 in sweeps:
+        sweeps = (1, 1, 3)
+    wl = W.tank(*size, seed=51)
+    assert_vcycle_is_the_oracles(wl, max_levels=levels, pre_sweeps=sweeps[0], post_sweeps=sweeps[1],
+                                 coarse_sweeps=sweeps[2], smoother=smoother, coarse_operator=coarse_operator)
