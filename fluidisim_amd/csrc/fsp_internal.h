@@ -77,6 +77,17 @@ struct Progress {
   unsigned long long word;
 };
 
+// Arrays whose rows change their length (k_rows): row r of a[q] (from[q] floats)
+// to row r of b[q] (to[q] floats), cut off or filled with zeros.
+constexpr int ROW_ARRAYS = 10;
+struct RowSet {
+  const float* a[ROW_ARRAYS];
+  float* b[ROW_ARRAYS];
+  int from[ROW_ARRAYS], to[ROW_ARRAYS];
+  size_t rows[ROW_ARRAYS];
+  int count;
+};
+
 // Fine-level geometry, passed by value to kernels.
 struct Fine {
   int nx, ny, nz;

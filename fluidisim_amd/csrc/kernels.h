@@ -783,6 +783,27 @@ __global__ void __launch_bounds__(BLOCK) k_store_p(size_t n, const double* p, fl
   FSP_FOR(c, n) pout[c] = (float)p[c];
 }
 
+// The grid's row y takes array y.
+__global__ void __launch_bounds__(BLOCK) k_rows(RowSet R) {
+  const int y = (int)blockIdx.y, from = R.from[y], to = R.to[y];
+  const float* a = R.a[y];
+  float* b = R.b[y];
+  const size_t total = R.rows[y] * (size_t)to;
+  for (size_t q = (size_t)blockIdx.x * BLOCK + threadIdx.x; q < total; q += (size_t)gridDim.x * BLOCK) {
+    const uint32_t row = (uint32_t)q / (uint32_t)to;
+    const int i = (int)((uint32_t)q - row * (uint32_t)to);
+    b[q] = i < from ? a[(size_t)row * from + i] : 0.f;
+  }
+}
+__global__ void __launch_bounds__(BLOCK) k_rows_u8(const uint8_t* a, uint8_t* b, int from, int to, size_t rows,
+                                                   uint8_t fill) {
+  FSP_FOR(q, rows * (size_t)to) {
+    const uint32_t row = (uint32_t)q / (uint32_t)to;
+    const int i = (int)((uint32_t)q - row * (uint32_t)to);
+    b[q] = i < from ? a[(size_t)row * from + i] : fill;
+  }
+}
+
 __global__ void __launch_bounds__(BLOCK) k_fill(float* x, size_t n, float value) {
   FSP_FOR(c, n) x[c] = value;
 }
