@@ -136,3 +136,14 @@ def test_levels_of_row_coefficients_match_the_oracle(size, levels, sweeps, smoot
     wl = W.tank(*size, seed=51)
     assert_vcycle_is_the_oracles(wl, max_levels=levels, pre_sweeps=sweeps[0], post_sweeps=sweeps[1],
                                  coarse_sweeps=sweeps[2], smoother=smoother, coarse_operator=coarse_operator)
+
+
+@pytest.mark.parametrize("sweeps", [0, 1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("size", [
+    (40, 36, 32),   # 20 x 18 x 16: tiles cut by the level's edge in x and y
+    (48, 34, 42),   # 24 x 17 x 21: odd rows and planes
+    (80, 16, 56),   # 40 x 8 x 28
+], ids=str)
+def test_a_coarsest_level_above_the_tail_matches_the_oracle(size, sweeps):
+    """1 to 16 colour passes, up to five to a launch."""
+    assert_vcycle_is_the_oracles(W.tank(size[0], size[2], size[1], seed=71), max_levels=1, coarse_sweeps=sweeps)

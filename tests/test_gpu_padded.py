@@ -54,7 +54,7 @@ def compare(vol, faces, what, rel_tol=1e-10):
 
 
 @pytest.mark.parametrize("size", [(34, 20, 24), (18, 12, 16), (7, 6, 5), (33, 16, 12), (30, 1, 16), (90, 14, 10),
-                                  (5, 8, 8), (6, 6, 6)], ids=str)
+                                  (50, 36, 30), (5, 8, 8), (6, 6, 6)], ids=str)
 @pytest.mark.parametrize("options", [
     dict(smoother=_lib.SMOOTH_RBGS, coarse_operator=_lib.COARSE_GALERKIN),
     dict(smoother=_lib.SMOOTH_RBGS, coarse_operator=_lib.COARSE_REDISCRETISED),
