@@ -52,6 +52,7 @@ struct fsp_solver {
   // padded with solid cells in x to rows that do: its solver (null: none), on
   // this solver's stream. This solver keeps the caller's arrays and geometry.
   fsp_solver* inner = nullptr;
+  FinishSet fins{};  // folds put off to the next launch of k_finish
   bool shares_stream = false;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   size_t n = 0, nu = 0, nv = 0, nw = 0, ncols = 0;
@@ -288,15 +289,34 @@ auto with_storage(int storage, F&& f) {
   }
 }
 
-// Fold the per-block partials of a reducing kernel (k_finish) right after it.
-void launch_finish(fsp_solver* S, hipStream_t st, int op, unsigned nblocks, bool is_max, int gated) {
-  if (is_max)
-    hipLaunchKernelGGL(k_finish<true>, dim3(1), dim3(FIN_THREADS), 0, st, op, nblocks, gated, S->ctl, S->partials,
-                       S->progress);
-  else
-    hipLaunchKernelGGL(k_finish<false>, dim3(1), dim3(FIN_THREADS), 0, st, op, nblocks, gated, S->ctl, S->partials,
-                       S->progress);
+// The fold (k_finish) of a reducing kernel's partials put off to the next
+// launch_finish, where no kernel in between reads its result.
+void defer_finish(fsp_solver* S, int op, unsigned nblocks, bool is_max, int gated) {
+  FinishSet& F = S->fins;
+  F.op[F.count] = op;
+  F.nblocks[F.count] = nblocks;
+  F.is_max[F.count] = is_max;
+  F.gated[F.count] = gated;
+  ++F.count;
 }
+void flush_finish(fsp_solver* S, hipStream_t st) {
+  const FinishSet& F = S->fins;
+  const dim3 one(1), threads(FIN_THREADS);
+  switch (F.count) {
+    case 0: break;
+    case 1: k_finish<1><<<one, threads, 0, st>>>(F, S->ctl, S->partials, S->progress); break;
+    case 2: k_finish<2><<<one, threads, 0, st>>>(F, S->ctl, S->partials, S->progress); break;
+    case 3: k_finish<3><<<one, threads, 0, st>>>(F, S->ctl, S->partials, S->progress); break;
+    default: k_finish<4><<<one, threads, 0, st>>>(F, S->ctl, S->partials, S->progress); break;
+  }
+  S->fins.count = 0;
+}
+// Folds the partials of a reducing kernel right after it, with the ones put off.
+void launch_finish(fsp_solver* S, hipStream_t st, int op, unsigned nblocks, bool is_max, int gated) {
+  defer_finish(S, op, nblocks, is_max, gated);
+  flush_finish(S, st);
+}
+#define FSP_DEFER(S, op, grid, is_max, gated) defer_finish(S, op, (grid).x, is_max, gated)
 #define FSP_FINISH(S, stream, op, grid, is_max, gated) launch_finish(S, stream, op, (grid).x, is_max, gated)
 
 template <class T>
@@ -456,12 +476,13 @@ struct Launch {
       const dim3 gq((unsigned)(S->qfine.nbx * S->qfine.nby * S->qfine.planes));
       FSP_LAUNCH_FORM(S, "k_residual_q", k_residual_q<FORM_TABLE>, k_residual_q<FORM_INDEX>, k_residual_q<FORM_GENERAL>, gq, QBLOCK, st, G, S->qfine, p64,
                      S->b, S->r, op, S->ctl, S->partials, gated);
-      FSP_FINISH(S, st, op, gq, false, fin_gate);
+      FSP_DEFER(S, op, gq, false, fin_gate);
     } else {
       const dim3 g(grid_for(G.n));
       FSP_LAUNCH(S, k_residual, g, st, G, p64, S->b, S->r, op, S->ctl, S->partials, gated);
-      FSP_FINISH(S, st, op, g, false, fin_gate);
+      FSP_DEFER(S, op, g, false, fin_gate);
     }
+    if (!replacement) flush_finish(S, st);
   }
 
   // The true residual into OP_RR with the backward error of the same r into
@@ -931,23 +952,26 @@ struct Launch {
                        (const TS<ST>*)S->zres, S->d0, S->d1, S->q, S->ctl, S->partials);
         return 0;
       });
-      FSP_FINISH(S, st, OP_DQ, g, false, 1);
+      const unsigned folded = g.x <= (unsigned)FSP_FOLD_PARTIALS ? g.x : 0u;
+      if (folded) FSP_DEFER(S, OP_DQ, g, false, 1);
+      else FSP_FINISH(S, st, OP_DQ, g, false, 1);
       const size_t nquads = G.n / 4;
       const dim3 gu((unsigned)((nquads + QBLOCK - 1) / QBLOCK));
       FSP_LAUNCH(S, k_q_update, gu, st, nquads, S->p64, S->r, (const float*)S->d0, (const float*)S->d1,
-                 (const float*)S->q, S->ctl, S->partials);
-      FSP_FINISH(S, st, OP_RN, gu, false, 1);
+                 (const float*)S->q, S->ctl, S->partials, folded);
+      FSP_DEFER(S, OP_RN, gu, false, 1);
     } else {
       FSP_LAUNCH(S, k_spmv_dir, dim3(grid_for(G.n)), st, G, S->zres, S->d0, S->d1, S->q, S->ctl, S->partials);
       FSP_FINISH(S, st, OP_DQ, dim3(grid_for(G.n)), false, 1);
       FSP_LAUNCH(S, k_update, dim3(grid_for(G.n)), st, G.n, S->p64, S->r, S->d0, S->d1, S->q, S->ctl,
                  S->partials);
-      FSP_FINISH(S, st, OP_RN, dim3(grid_for(G.n)), false, 1);
+      FSP_DEFER(S, OP_RN, dim3(grid_for(G.n)), false, 1);
     }
     // true-residual replacement: every replace_every-th iteration r (and
     // |r|^2, which the loop test reads) becomes b - A p64 formed in f64; the
     // preconditioned residual, beta and the direction then follow from it
     if (S->opt.replace_every > 0) residual(S->p64, OP_RN_TRUE, true);
+    if (S->net_phase) flush_finish(S, st);  // the network's scale is |r|^2
     precondition(OP_RZ);
   }
 
@@ -969,23 +993,26 @@ struct PassState {
   double rr;
 };
 bool wait_pass(fsp_solver* S, uint32_t it, PassState& state) {
+  bool drained = false;
   for (uint32_t spins = 1;; ++spins) {
     const unsigned long long w = __atomic_load_n(&S->progress->word, __ATOMIC_ACQUIRE);
     if ((uint32_t)(w >> 34) == (S->pass & 0x3FFFFFFFu)) {
       state.it = (uint32_t)(w >> 2);
       state.active = (w & 1ull) != 0;
       state.nonfinite = (w & 2ull) != 0;
-      if (!state.active || state.it >= it) {
-        state.rr = S->progress->rr;
+      const unsigned long long rate = __atomic_load_n(&S->progress->rate, __ATOMIC_ACQUIRE);
+      if ((!state.active || state.it >= it) && (uint32_t)rate == progress_tag(w)) {
+        const uint32_t bits = (uint32_t)(rate >> 32);
+        float rr;
+        std::memcpy(&rr, &bits, sizeof rr);
+        state.rr = rr;
         return true;
       }
     }
+    if (drained) return false;
     __builtin_ia32_pause();
-    // every so often: is the stream still at work?
-    if ((spins & 0x3FFFu) == 0 && hipStreamQuery(S->stream) != hipErrorNotReady) {
-      const unsigned long long last = __atomic_load_n(&S->progress->word, __ATOMIC_ACQUIRE);
-      if (last == w) return false;
-    }
+    // every so often: is the stream still at work? (if not, what it left is read once more)
+    if ((spins & 0x3FFFu) == 0) drained = hipStreamQuery(S->stream) != hipErrorNotReady;
   }
 }
 
@@ -1894,7 +1921,7 @@ fsp_status create_solver(const fsp_domain* d, const fsp_options* o, fsp_solver* 
   S->hctl = &S->host->ctl;
   S->hhash = &S->host->hash;
   S->progress = &S->host->progress;
-  S->progress->word = 0;
+  S->progress->word = S->progress->rate = 0;
   if (opt.preconditioner != FSP_PRECOND_JACOBI) {  // the learned preconditioner falls back to the V-cycle
     size_t x = nx, y = ny, z = nz;
     float h = d->dx;

@@ -70,11 +70,25 @@ struct Ctl {
 };
 
 // Progress of the CG loop, in host memory that the device writes: the host
-// launches iterations by it without stopping the stream. `word` is written
-// last: pass number << 34 | iteration << 2 | non-finite << 1 | active.
+// launches iterations by it without stopping the stream. `word` is pass number
+// << 34 | iteration << 2 | non-finite << 1 | active; `rate` is |r|^2 (f32)
+// << 32 | the tag of the word it belongs to, so that the two need no order
+// (a store that releases writes the whole L2 back: 3 us an iteration).
 struct Progress {
-  double rr;
-  unsigned long long word;
+  unsigned long long word, rate;
+};
+__host__ __device__ inline unsigned progress_tag(unsigned long long word) {
+  return (unsigned)(word >> 34) * 0x9E3779B1u + (unsigned)(word >> 2);
+}
+
+// The reductions that one k_finish folds: `nblocks` partials of each operation's
+// slot, sums or maxima, and its gate (k_finish).
+constexpr int FIN_ENTRIES = 4;
+struct FinishSet {
+  int op[FIN_ENTRIES];
+  unsigned nblocks[FIN_ENTRIES];
+  int gated[FIN_ENTRIES], is_max[FIN_ENTRIES];
+  int count;
 };
 
 // Arrays whose rows change their length (k_rows): row r of a[q] (from[q] floats)

@@ -52,13 +52,37 @@ __device__ __forceinline__ void decode(const Fine& G, size_t c, int& i, int& j, 
 }
 
 // ---------------------------------------------------------------- reductions
+// v of the lane N above, where the sums below read it (lane 0's tree; other
+// lanes hold no total): a row of 16 lanes shifts by DPP, the rows and halves of
+// the wavefront swap, a few cycles each where a shuffle through LDS costs a
+// hundred; the values meet in the order of a tree of __shfl_down.
+template <int N>
+__device__ __forceinline__ unsigned lane_above(unsigned v) {
+  if constexpr (N == 32) return __builtin_amdgcn_permlane32_swap(v, v, false, false)[1];
+  else if constexpr (N == 16) return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
+  else return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x100 + N, 0xF, 0xF, true);  // row_shl
+}
+template <int N>
+__device__ __forceinline__ double lane_above(double v) {
+  const unsigned long long w = __double_as_longlong(v);
+  const unsigned lo = lane_above<N>((unsigned)w), hi = lane_above<N>((unsigned)(w >> 32));
+  return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
 __device__ __forceinline__ double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  return v;
+  v += lane_above<32>(v);
+  v += lane_above<16>(v);
+  v += lane_above<8>(v);
+  v += lane_above<4>(v);
+  v += lane_above<2>(v);
+  return v + lane_above<1>(v);
 }
 __device__ __forceinline__ double wave_max(double v) {
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_down(v, o, 64));
-  return v;
+  v = fmax(v, lane_above<32>(v));
+  v = fmax(v, lane_above<16>(v));
+  v = fmax(v, lane_above<8>(v));
+  v = fmax(v, lane_above<4>(v));
+  v = fmax(v, lane_above<2>(v));
+  return fmax(v, lane_above<1>(v));
 }
 
 // Block-level reduction of two values into this block's slot of `partials`.
@@ -166,58 +190,110 @@ __device__ __forceinline__ void reduce_finish(double a, double b, int op, Ctl* c
   block_partial<MAX>(a, b, op, partials);
 }
 
-// Folds the partials of `nblocks` blocks in block order and applies the
-// finish operation. `gated`: 1, skipped like its producer once the loop
-// stopped; 2, skipped like the gauge kernels unless the problem is pure
-// Neumann.
+// Folds the partials of N kernels, each in block order, and applies the finish
+// operations one after the other on a copy of the control block in LDS (on
+// the block itself each read what the one before had written, 1 us through
+// memory: three operations 7.5 us, now 4.7). `gated`: 1, skipped like its producer once the loop stopped,
+// be it by the operation before; 2, skipped like the gauge kernels unless the
+// problem is pure Neumann; 3, only in an iteration that replaces the residual.
 // FIN_THREADS threads with eight loads each fold 8192 partials (the fine
 // kernels' grid) in one round of memory latency.
 constexpr int FIN_THREADS = 1024;
 
-template <bool MAX>
-__global__ void __launch_bounds__(FIN_THREADS) k_finish(int op, unsigned nblocks, int gated, Ctl* ctl,
-                                                        double* partials, Progress* progress) {
-  if ((gated == 1 && !ctl->active) || (gated == 2 && !ctl->pure_neumann) || (gated == 3 && !replacing(ctl))) return;
-  __shared__ double sa[FIN_THREADS / 64], sb[FIN_THREADS / 64];
-  const double2* part = reinterpret_cast<const double2*>(partials + (size_t)op * MAX_PARTIALS * 2);
-  // eight independent loads in flight per step, folded in a fixed order
-  double a = 0.0, b = 0.0;
-  for (unsigned base = threadIdx.x; base < nblocks; base += 8 * FIN_THREADS) {
-    double2 v[8];
+template <int N>
+__global__ void __launch_bounds__(FIN_THREADS) k_finish(FinishSet F, Ctl* ctl, const double* partials,
+                                                        Progress* progress) {
+  constexpr int WAVES = FIN_THREADS / 64;
+  constexpr int WORDS = sizeof(Ctl) / 4;
+  static_assert(WORDS <= FIN_THREADS, "a word per thread");
+  __shared__ double sums[2 * N][WAVES], totals[2 * N];
+  __shared__ Ctl block;
+  const bool active = ctl->active != 0, replaced = replacing(ctl), pure = ctl->pure_neumann != 0;
+  if (F.gated[N - 1] == 1 && !active) return;  // (the last of an iteration's)
+  bool on[N];
+  unsigned most = 0;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const unsigned q = base + (unsigned)u * FIN_THREADS;
-      v[u] = q < nblocks ? part[q] : make_double2(0.0, 0.0);
+  for (int n = 0; n < N; ++n) {
+    const int g = F.gated[n];
+    on[n] = !((g == 1 && !active) || (g == 2 && !pure) || (g == 3 && !replaced));
+    if (on[n]) most = F.nblocks[n] > most ? F.nblocks[n] : most;
+  }
+  if (most == 0) return;
+  uint32_t* words = reinterpret_cast<uint32_t*>(&block);
+  if (threadIdx.x < WORDS) words[threadIdx.x] = reinterpret_cast<const uint32_t*>(ctl)[threadIdx.x];
+  double a[N], b[N];
+  auto slot = [&](int n) { return reinterpret_cast<const double2*>(partials + (size_t)F.op[n] * MAX_PARTIALS * 2); };
+  if (most <= FIN_THREADS) {  // every operation's loads at once
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const double2 v = on[n] && threadIdx.x < F.nblocks[n] ? slot(n)[threadIdx.x] : make_double2(0.0, 0.0);
+      a[n] = v.x;
+      b[n] = v.y;
     }
+  } else {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      a = MAX ? fmax(a, v[u].x) : a + v[u].x;
-      b = MAX ? fmax(b, v[u].y) : b + v[u].y;
+    for (int n = 0; n < N; ++n) {
+      a[n] = b[n] = 0.0;
+      if (!on[n]) continue;
+      const double2* part = slot(n);
+      const unsigned nblocks = F.nblocks[n];
+      // eight independent loads in flight per step, folded in a fixed order
+      for (unsigned base = threadIdx.x; base < nblocks; base += 8 * FIN_THREADS) {
+        double2 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const unsigned q = base + (unsigned)u * FIN_THREADS;
+          v[u] = q < nblocks ? part[q] : make_double2(0.0, 0.0);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          a[n] = F.is_max[n] ? fmax(a[n], v[u].x) : a[n] + v[u].x;
+          b[n] = F.is_max[n] ? fmax(b[n], v[u].y) : b[n] + v[u].y;
+        }
+      }
     }
   }
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  a = MAX ? wave_max(a) : wave_sum(a);
-  b = MAX ? wave_max(b) : wave_sum(b);
-  if (lane == 0) { sa[wid] = a; sb[wid] = b; }
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    a[n] = F.is_max[n] ? wave_max(a[n]) : wave_sum(a[n]);
+    b[n] = F.is_max[n] ? wave_max(b[n]) : wave_sum(b[n]);
+    if (lane == 0) { sums[2 * n][wid] = a[n]; sums[2 * n + 1][wid] = b[n]; }
+  }
   __syncthreads();
-  if (threadIdx.x != 0) return;
-  a = sa[0];
-  b = sb[0];
-  for (int w = 1; w < FIN_THREADS / 64; ++w) {
-    a = MAX ? fmax(a, sa[w]) : a + sa[w];
-    b = MAX ? fmax(b, sb[w]) : b + sb[w];
+  if (threadIdx.x < 2 * N) {
+    const bool mx = F.is_max[threadIdx.x / 2] != 0;
+    double t = sums[threadIdx.x][0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) t = mx ? fmax(t, sums[threadIdx.x][w]) : t + sums[threadIdx.x][w];
+    totals[threadIdx.x] = t;
   }
-  ctl->red[op][0] = a;
-  ctl->red[op][1] = b;
-  finish(op, ctl, a, b);
-  // an iteration has ended, or the loop has
-  if ((gated == 1 || gated == 3) && (op == OP_RZ || !ctl->active)) {
-    progress->rr = ctl->rr;
-    __hip_atomic_store(&progress->word,
-                       (unsigned long long)ctl->pass << 34 | (unsigned long long)ctl->it << 2 |
-                           (ctl->nonfinite ? 2ull : 0ull) | (ctl->active ? 1ull : 0ull),
-                       __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    Ctl* c = &block;
+    bool loop = false;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const int g = F.gated[n];
+      loop |= g == 1 || g == 3;
+      if ((g == 2 && !c->pure_neumann) || (g == 3 && !replaced) || ((g == 1 || g == 3) && !c->active)) continue;
+      const int op = F.op[n];
+      c->red[op][0] = totals[2 * n];
+      c->red[op][1] = totals[2 * n + 1];
+      finish(op, c, totals[2 * n], totals[2 * n + 1]);
+    }
+    // an iteration has ended, or the loop has
+    if (loop && (F.op[N - 1] == OP_RZ || !c->active)) {
+      const unsigned long long word = (unsigned long long)c->pass << 34 | (unsigned long long)c->it << 2 |
+                                      (c->nonfinite ? 2ull : 0ull) | (c->active ? 1ull : 0ull);
+      const unsigned long long rate =
+          (unsigned long long)__float_as_uint((float)c->rr) << 32 | progress_tag(word);
+      __hip_atomic_store(&progress->rate, rate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(&progress->word, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
   }
+  __syncthreads();
+  if (threadIdx.x < WORDS) reinterpret_cast<uint32_t*>(ctl)[threadIdx.x] = words[threadIdx.x];
 }
 
 // ---------------------------------------------------------------- fine geometry

@@ -1347,21 +1347,67 @@ __global__ void __launch_bounds__(QBLOCK) k_q_spmv_dir(Fine G, QuadGrid Q, const
   reduce_finish<false>(s, unused, OP_DQ, ctl, partials);
 }
 
-// p += alpha d (f64), r -= alpha q, |r|^2; four cells per thread.
+// Largest number of partials that k_q_update folds itself.
+#ifndef FSP_FOLD_PARTIALS
+#define FSP_FOLD_PARTIALS 2048
+#endif
+
+// Sum of the first components of `count` partials by a whole workgroup of
+// QBLOCK threads, in k_finish's order, for every thread.
+__device__ __forceinline__ double fold_partials(const double* partials, int slot, unsigned count) {
+  constexpr int WAVES = FIN_THREADS / 64, PER = WAVES / (QBLOCK / 64);
+  __shared__ double sums[WAVES];
+  const double* part = partials + (size_t)slot * MAX_PARTIALS * 2;
+  const int lane = threadIdx.x & 63, first = (int)(threadIdx.x >> 6) * PER;
+  double a[PER];
+#pragma unroll
+  for (int u = 0; u < PER; ++u) a[u] = 0.0;
+  for (unsigned base = 0; base < count; base += FIN_THREADS) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const unsigned q = base + (unsigned)((first + u) * 64 + lane);
+      a[u] += q < count ? part[2 * (size_t)q] : 0.0;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    a[u] = wave_sum(a[u]);
+    if (lane == 0) sums[first + u] = a[u];
+  }
+  __syncthreads();
+  double t = sums[0];
+  for (int w = 1; w < WAVES; ++w) t += sums[w];
+  return t;
+}
+
+// p += alpha d (f64), r -= alpha q, |r|^2; four cells per thread. dq_parts: the
+// number of partials of <d, q> that every workgroup folds itself (the
+// iteration's k_finish records the sum, the step and the buffer switch), or 0
+// where k_finish has run in between (above FSP_FOLD_PARTIALS the folds read
+// more than that launch costs: 2048 partials take 128^3 cells from 1.923 to 1.911
+// ms, 1024 leave it there).
 __global__ void __launch_bounds__(QBLOCK) k_q_update(size_t nquads, double* p, float* r, const float* d0,
-                                                     const float* d1, const float* q, Ctl* ctl, double* partials) {
+                                                     const float* d1, const float* q, Ctl* ctl, double* partials,
+                                                     unsigned dq_parts) {
   if (!ctl->active) return;
-  const double alpha64 = ctl->alpha;
-  const float alpha = (float)alpha64;
-  const float* d = ctl->dsel ? d1 : d0;
-  double s = 0.0, unused = 0.0;
+  double alpha64 = ctl->alpha;
+  int sel = ctl->dsel;
   const size_t t = (size_t)blockIdx.x * QBLOCK + threadIdx.x;
-  if (t < nquads) {
-    const size_t c = 4 * t;
-    const float4 dv = ld4(d, c), qv = ld4(q, c);
-    float4 rv = ld4(r, c);
-    double2* pp = reinterpret_cast<double2*>(p + c);
-    double2 p0 = pp[0], p1 = pp[1];
+  const bool valid = t < nquads;
+  const size_t c = valid ? 4 * t : 0;
+  if (dq_parts) sel ^= 1;
+  const float4 dv = ld4(sel ? d1 : d0, c), qv = ld4(q, c);
+  float4 rv = ld4(r, c);
+  double2* pp = reinterpret_cast<double2*>(p + c);
+  double2 p0 = pp[0], p1 = pp[1];
+  if (dq_parts) {
+    const double dq = fold_partials(partials, OP_DQ, dq_parts);
+    if (!(dq > 0.0)) return;
+    alpha64 = ctl->rz / dq;
+  }
+  const float alpha = (float)alpha64;
+  double s = 0.0, unused = 0.0;
+  if (valid) {
     p0.x += alpha64 * (double)dv.x; p0.y += alpha64 * (double)dv.y;
     p1.x += alpha64 * (double)dv.z; p1.y += alpha64 * (double)dv.w;
     pp[0] = p0;
