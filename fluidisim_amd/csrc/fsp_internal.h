@@ -69,6 +69,16 @@ struct Ctl {
   uint32_t pass;         // number of the pass (Progress)
 };
 
+// The plain-row acceptance metric of the corrected faces (delta3d_mobile.rs:422-432,
+// f32 arithmetic), normalised as the reference.
+__host__ __device__ inline float divergence_ratio(const Ctl& c, float dx) {
+  const float mx = (float)c.red[OP_UMAX][0];
+  return mx > 0.f ? dx / (mx > 1e-4f ? mx : 1e-4f) : 0.f;
+}
+__host__ __device__ inline double plain_divergence(const Ctl& c, float dx) {
+  return (double)((float)c.red[OP_DIVMAX][1] * divergence_ratio(c, dx));
+}
+
 // Progress of the CG loop, in host memory that the device writes: the host
 // launches iterations by it without stopping the stream. `word` is pass number
 // << 34 | iteration << 2 | non-finite << 1 | active; `rate` is |r|^2 (f32)

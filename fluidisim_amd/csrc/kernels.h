@@ -193,16 +193,18 @@ __device__ __forceinline__ void reduce_finish(double a, double b, int op, Ctl* c
 // Folds the partials of N kernels, each in block order, and applies the finish
 // operations one after the other on a copy of the control block in LDS (on
 // the block itself each read what the one before had written, 1 us through
-// memory: three operations 7.5 us, now 4.7). `gated`: 1, skipped like its producer once the loop stopped,
-// be it by the operation before; 2, skipped like the gauge kernels unless the
-// problem is pure Neumann; 3, only in an iteration that replaces the residual.
+// memory: three operations 7.5 us, now 4.7). `gated`: 1, skipped like its
+// producer once the loop stopped, be it by the operation before; 2, skipped
+// like the gauge kernels unless the problem is pure Neumann; 3, only in an
+// iteration that replaces the residual. host: where the host reads the block
+// after the stream's next stop, or null.
 // FIN_THREADS threads with eight loads each fold 8192 partials (the fine
 // kernels' grid) in one round of memory latency.
 constexpr int FIN_THREADS = 1024;
 
 template <int N>
 __global__ void __launch_bounds__(FIN_THREADS) k_finish(FinishSet F, Ctl* ctl, const double* partials,
-                                                        Progress* progress) {
+                                                        Progress* progress, Ctl* host) {
   constexpr int WAVES = FIN_THREADS / 64;
   constexpr int WORDS = sizeof(Ctl) / 4;
   static_assert(WORDS <= FIN_THREADS, "a word per thread");
@@ -293,7 +295,10 @@ __global__ void __launch_bounds__(FIN_THREADS) k_finish(FinishSet F, Ctl* ctl, c
     }
   }
   __syncthreads();
-  if (threadIdx.x < WORDS) reinterpret_cast<uint32_t*>(ctl)[threadIdx.x] = words[threadIdx.x];
+  if (threadIdx.x < WORDS) {
+    reinterpret_cast<uint32_t*>(ctl)[threadIdx.x] = words[threadIdx.x];
+    if (host) reinterpret_cast<uint32_t*>(host)[threadIdx.x] = words[threadIdx.x];
+  }
 }
 
 // ---------------------------------------------------------------- fine geometry
@@ -790,7 +795,7 @@ __global__ void __launch_bounds__(BLOCK) k_assemble(Fine G, const float* us, con
                                                     const float* div_in, float scale, float* b, float* prec_out,
                                                     Ctl* ctl, double* partials) {
 #pragma clang fp contract(off)
-  double s2 = 0.0, unused = 0.0;
+  double s2 = 0.0, unused = 0.0, sum = 0.0, active = 0.0;
   FSP_FOR(c, G.n) {
     int i, j, k;
     decode(G, c, i, j, k);
@@ -818,14 +823,17 @@ __global__ void __launch_bounds__(BLOCK) k_assemble(Fine G, const float* us, con
     b[c] = bb;
     if (prec_out) prec_out[c] = pr;
     s2 += (double)bb * (double)bb;
+    if (prec_positive(m)) { sum += (double)bb; active += 1.0; }
   }
   reduce_finish<false>(s2, unused, OP_B2, ctl, partials);
+  if (!ctl->gauge) return;  // whether the gauge applies is known after OP_COUNT's fold
+  __syncthreads();
+  reduce_finish<false>(sum, active, OP_MEAN_B, ctl, partials);
 }
 
-// Sum of x and count over rows with prec > 0 (gauge of a pure-Neumann problem).
+// Sum of p and count over rows with prec > 0 (gauge of a pure-Neumann problem).
 // Skipped (with its fold, k_finish gated == 2) unless the problem is pure Neumann.
-template <class T>
-__global__ void __launch_bounds__(BLOCK) k_sum_active(Fine G, const T* x, int op, Ctl* ctl, double* partials) {
+__global__ void __launch_bounds__(BLOCK) k_sum_active(Fine G, const double* x, int op, Ctl* ctl, double* partials) {
   if (!ctl->pure_neumann) return;
   double s = 0.0, n = 0.0;
   FSP_FOR(c, G.n) {
@@ -834,28 +842,43 @@ __global__ void __launch_bounds__(BLOCK) k_sum_active(Fine G, const T* x, int op
   reduce_finish<false>(s, n, op, ctl, partials);
 }
 
-// x -= mean on active rows when the problem is pure Neumann; for b also
-// recompute |b|^2 (otherwise x and |b|^2 stand: skipped, with its fold).
-template <class T>
-__global__ void __launch_bounds__(BLOCK) k_sub_mean(Fine G, T* x, int which, int op, Ctl* ctl, double* partials) {
-  const int pure = ctl->pure_neumann;
-  if (!pure) return;
-  const T mean = (T)(which == 0 ? ctl->mean_b : ctl->mean_p);
-  double s2 = 0.0, unused = 0.0;
-  FSP_FOR(c, G.n) {
-    T val = x[c];
-    if (pure && prec_positive(G.mask[c])) { val = val - mean; x[c] = val; }
-    s2 += (double)val * (double)val;
-  }
-  if (op >= 0) reduce_finish<false>(s2, unused, op, ctl, partials);
+// p -= mean on active rows when the problem is pure Neumann.
+__global__ void __launch_bounds__(BLOCK) k_sub_mean(Fine G, double* p, Ctl* ctl) {
+  if (!ctl->pure_neumann) return;
+  const double mean = ctl->mean_p;
+  FSP_FOR(c, G.n)
+    if (prec_positive(G.mask[c])) p[c] = p[c] - mean;
 }
 
 // Warm start (delta3d_mobile.rs:486-496): p from the caller, 0 on dry cells;
-// cold start: p = 0.
-__global__ void __launch_bounds__(BLOCK) k_load_p(Fine G, const float* pin, double* p, int warm) {
-  FSP_FOR(c, G.n) p[c] = (warm && (G.mask[c] & M_WET)) ? (double)pin[c] : 0.0;
+// cold start: p = 0. With a pure-Neumann problem b -= mean on active rows and
+// |b|^2 again.
+__global__ void __launch_bounds__(BLOCK) k_load_p(Fine G, const float* pin, double* p, int warm, float* b, Ctl* ctl,
+                                                  double* partials) {
+  const bool pure = ctl->pure_neumann != 0;
+  const float mean = (float)ctl->mean_b;
+  double s2 = 0.0, unused = 0.0;
+  FSP_FOR(c, G.n) {
+    const uint8_t m = G.mask[c];
+    p[c] = (warm && (m & M_WET)) ? (double)pin[c] : 0.0;
+    if (pure) {
+      float val = b[c];
+      if (prec_positive(m)) { val = val - mean; b[c] = val; }
+      s2 += (double)val * (double)val;
+    }
+  }
+  if (pure) reduce_finish<false>(s2, unused, OP_B2, ctl, partials);
 }
-__global__ void __launch_bounds__(BLOCK) k_store_p(size_t n, const double* p, float* pout) {
+
+// p in f32 to the caller. accepted: only if the residual and the plain-row
+// divergence of the control block (the host's own test, in its arithmetic)
+// end the projection; then *stored is set.
+__global__ void __launch_bounds__(BLOCK) k_store_p(size_t n, const double* p, float* pout, int accepted, double tol_b2,
+                                                   float dx, const Ctl* ctl, int* stored) {
+  if (accepted) {
+    if (ctl->nonfinite || !(ctl->actual <= tol_b2) || !(plain_divergence(*ctl, dx) <= 1e-5)) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *stored = 1;
+  }
   FSP_FOR(c, n) pout[c] = (float)p[c];
 }
 

@@ -825,7 +825,7 @@ __global__ void __launch_bounds__(QBLOCK) k_assemble_q(Fine G, QuadGrid Q, const
                                                        const float* ws, const float* div_in, float scale, float* b,
                                                        float* prec_out, Ctl* ctl, double* partials) {
 #pragma clang fp contract(off)
-  double s2 = 0.0, unused = 0.0;
+  double s2 = 0.0, unused = 0.0, sum = 0.0, active = 0.0;
   int qx, j, k;
   const bool valid = quad_coords(Q, qx, j, k);
   if (valid) {
@@ -884,11 +884,15 @@ __global__ void __launch_bounds__(QBLOCK) k_assemble_q(Fine G, QuadGrid Q, const
       }
       q_set(out, e, bb);
       s2 += (double)bb * (double)bb;
+      if (prec_positive(m)) { sum += (double)bb; active += 1.0; }
     }
     st4(b, c0, out);
     if (prec_out) st4(prec_out, c0, pout);
   }
   reduce_finish<false>(s2, unused, OP_B2, ctl, partials);
+  if (!ctl->gauge) return;
+  __syncthreads();
+  reduce_finish<false>(sum, active, OP_MEAN_B, ctl, partials);
 }
 
 // Velocity correction on quads (k_correct with four x-cells per thread: the
@@ -1129,14 +1133,24 @@ __global__ void __launch_bounds__(QBLOCK) k_backward_q(Fine G, QuadGrid Q, const
 }
 
 // Cold start, p = 0: p64 = 0, r = b - A 0 = b exactly, |r|^2 into `op`
-// (k_load_p and k_residual in one pass over b).
-__global__ void __launch_bounds__(QBLOCK) k_start_cold(size_t nquads, const float* b, double* p, float* r, int op,
-                                                       Ctl* ctl, double* partials) {
+// (k_load_p and k_residual in one pass over b), b without its mean first where
+// the problem is pure Neumann.
+__global__ void __launch_bounds__(QBLOCK) k_start_cold(size_t nquads, const uint8_t* mask, float* b, double* p, float* r,
+                                                       int op, Ctl* ctl, double* partials) {
+  const bool pure = ctl->pure_neumann != 0;
+  const float mean = (float)ctl->mean_b;
   double s = 0.0, unused = 0.0;
   const size_t t = (size_t)blockIdx.x * QBLOCK + threadIdx.x;
   if (t < nquads) {
     const size_t c = 4 * t;
-    const float4 bq = ld4(b, c);
+    float4 bq = ld4(b, c);
+    if (pure) {
+      const uint32_t mq = *reinterpret_cast<const uint32_t*>(mask + c);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (prec_positive((uint8_t)(mq >> (8 * e)))) q_set(bq, e, q_get(bq, e) - mean);
+      st4(b, c, bq);
+    }
     double2* pp = reinterpret_cast<double2*>(p + c);
     pp[0] = make_double2(0.0, 0.0);
     pp[1] = make_double2(0.0, 0.0);
@@ -1144,6 +1158,9 @@ __global__ void __launch_bounds__(QBLOCK) k_start_cold(size_t nquads, const floa
     s = (double)bq.x * bq.x + (double)bq.y * bq.y + (double)bq.z * bq.z + (double)bq.w * bq.w;
   }
   reduce_finish<false>(s, unused, op, ctl, partials);
+  if (!pure) return;
+  __syncthreads();
+  reduce_finish<false>(s, unused, OP_B2, ctl, partials);
 }
 
 // ---------------------------------------------------------------- damped Jacobi
