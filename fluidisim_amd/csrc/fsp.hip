@@ -559,7 +559,9 @@ struct Launch {
   template <int ST>
   void tail() {
     const TailSet T = tail_set();
-    if (gc_tail_ok(S->opt)) k_gc_tail<ST><<<dim3(1), dim3(TAIL_THREADS), S->tail_lds, st>>>(T, S->ctl);
+    if (gc_tail_ok(S->opt) && gc_tail_top(T.lv))
+      k_gc_tail<ST, true><<<dim3(1), dim3(TAIL_THREADS), S->tail_lds, st>>>(T, S->ctl);
+    else if (gc_tail_ok(S->opt)) k_gc_tail<ST, false><<<dim3(1), dim3(TAIL_THREADS), S->tail_lds, st>>>(T, S->ctl);
     else k_r6_tail<ST><<<dim3(1), dim3(TAIL_THREADS), S->tail_lds, st>>>(T, S->ctl);
   }
 
@@ -1995,7 +1997,7 @@ fsp_status create_solver(const fsp_domain* d, const fsp_options* o, fsp_solver* 
     const int count = (int)S->levels.size() - t;
     const bool gc = gc_tail_ok(opt);
     const size_t bytes = gc ? gc_tail_lds_bytes(&S->levels[t], count) : r6_tail_lds_bytes(&S->levels[t], count);
-    if (bytes > std::min(GC_TAIL_LDS_FLOATS * sizeof(float), lds_limit - TAIL_STATIC_LDS)) break;
+    if (bytes > std::min(TAIL_LDS_FLOATS * sizeof(float), lds_limit - TAIL_STATIC_LDS)) break;
     S->tail_first = t;
     S->tail_lds = bytes;
   }

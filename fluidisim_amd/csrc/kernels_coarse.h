@@ -606,8 +606,8 @@ inline unsigned gb_blocks(const Level& L) {
 namespace fsp {
 
 // ---------------------------------------------------------------- compact tail
-// Every Galerkin level below the compact ones in one workgroup, in LDS:
-// per cell the x-, y-, z- couplings in f32 and dd, then x and r (values
+// Every Galerkin level below the compact ones in one workgroup, the first in
+// registers (GctTop), the others in LDS: per cell the x-, y-, z- couplings in f32 and dd, then x and r (values
 // rounded to storage ST): 6 floats. Same arithmetic as k_gc_gs /
 // k_gc_restrict2. The couplings of all levels lie first, level after level
 // ([fx, fy, fz, dd] blocks of n floats each), exactly as k_gct_pack lays
@@ -735,71 +735,125 @@ __device__ __forceinline__ void gct_pass(float* lds, const GcTailLvl& L, int col
   __syncthreads();
 }
 
-// The palindromic sweeps of a coarsest level of at most 64 cells in the
-// first wavefront: each lane holds one cell's x in a register and reads its
-// neighbours' by lane shuffle, so the passes need no workgroup barrier.
-// Per cell the arithmetic of gct_pass, in the same order.
+// The last levels of at most 64 cells in the first wavefront: a lane holds one
+// cell of a level with its x in a register and reads its neighbours' by lane
+// shuffle, so that nothing from a level's pre-smoothing to its
+// post-smoothing needs a workgroup barrier (16^3 down to 2^3, 4^3 included:
+// 22.3 -> 20.8 us). Per cell the arithmetic of gct_pass, in the same order.
+constexpr int WAVE_CELLS = 64;
+
 template <int ST>
-__device__ __forceinline__ void gct_coarsest_wave(float* lds, const GcTailLvl& L, int count, bool from_zero) {
-#pragma clang fp contract(off)
+struct GctWave {
   using SV = Store<ST>;
-  if (threadIdx.x < 64) {
-    const int c = (int)threadIdx.x;
+  float a[6], dd, dg, r, x;
+  int src[6], colour;  // colour: -1: no cell
+  int edge;            // bit f: no neighbour f
+
+  __device__ __forceinline__ void load(const float* lds, const GcTailLvl& L, bool with_r) {
+#pragma clang fp contract(off)
+    const int c = (int)threadIdx.x, plane = L.nx * L.ny;
     const bool in = c < L.n;
     int i = 0, j = 0, k = 0;
     if (in) gct_decode(L, c, i, j, k);
-    const int plane = L.nx * L.ny;
-    float a[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float dd = 0.f, r = 0.f, x = 0.f;
+    const bool has[6] = {in && i > 0, in && i + 1 < L.nx, in && j > 0, in && j + 1 < L.ny, in && k > 0,
+                         in && k + 1 < L.nz};
+    const int off[6] = {-1, 1, -L.nx, L.nx, -plane, plane};
+    edge = 0;
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+      src[f] = has[f] ? c + off[f] : c;
+      edge |= has[f] ? 0 : 1 << f;
+      a[f] = 0.f;
+    }
+    dd = r = x = 0.f;
     if (in) {
       gct_faces(lds, L, i, j, k, c, a);
       dd = lds[L.o_dd + c];
-      r = lds[L.o_r + c];
-      if (!from_zero) x = lds[L.o_x + c];
+      if (with_r) r = lds[L.o_r + c];
     }
-    const bool has[6] = {in && i > 0, in && i + 1 < L.nx, in && j > 0, in && j + 1 < L.ny, in && k > 0,
-                         in && k + 1 < L.nz};
-    const int src[6] = {has[0] ? c - 1 : c, has[1] ? c + 1 : c, has[2] ? c - L.nx : c,
-                        has[3] ? c + L.nx : c, has[4] ? c - plane : c, has[5] ? c + plane : c};
-    const float dg = gc_diag(a, dd, L.inv);
-    const int mine = (i + j + k) & 1;
-    auto pass = [&](int col, bool first) {
-      float nb[6];
+    dg = gc_diag(a, dd, L.inv);
+    colour = in ? (i + j + k) & 1 : -1;
+  }
+  __device__ __forceinline__ float row(float inv) const {
+    float nb[6];
 #pragma unroll
-      for (int f = 0; f < 6; ++f) {
-        const float v = __shfl(x, src[f]);
-        nb[f] = has[f] ? v : 0.f;
+    for (int f = 0; f < 6; ++f) {
+      const float v = __shfl(x, src[f]);
+      nb[f] = edge >> f & 1 ? 0.f : v;
+    }
+    return gc_row(a, dd, inv, x, nb);
+  }
+  __device__ __forceinline__ void sweeps(const GcTailLvl& L, int count, bool forward, bool coarsest) {
+#pragma clang fp contract(off)
+    const int passes = sweep_passes(coarsest, count);
+    for (int p = 0; p < passes; ++p) {
+      const int col = sweep_colour(coarsest, forward, count, p);
+      if (forward && p == 0) {
+        x = colour == col && dg > 0.f ? SV::rnd(r / dg) : 0.f;
+        continue;
       }
-      if (!in) return;
-      if (mine != col) {
-        if (first) x = 0.f;
-        return;
-      }
-      if (first) { x = dg > 0.f ? SV::rnd(r / dg) : 0.f; return; }
-      if (dg > 0.f) x = SV::rnd(x + (r - gc_row(a, dd, L.inv, x, nb)) / dg);
-    };
-    bool fz = from_zero;
-    const int half = count / 2;
-    for (int s = 0; s < half; ++s) { pass(0, fz); fz = false; pass(1, false); }
-    if (count & 1) { pass(0, fz); fz = false; }
-    for (int s = 0; s < half; ++s) { pass(1, fz); fz = false; pass(0, false); }
-    if (in) lds[L.o_x + c] = x;
+      const float next = SV::rnd(x + (r - row(L.inv)) / dg);
+      if (colour == col && dg > 0.f) x = next;
+    }
+  }
+  // r of the level C in `to` = restriction of the residual, children in order
+  __device__ __forceinline__ void restrict_to(const GcTailLvl& L, const GcTailLvl& C, GctWave& to) const {
+#pragma clang fp contract(off)
+    const float t = r - row(L.inv);
+    int i = 0, j = 0, k = 0;
+    if (to.colour >= 0) gct_decode(C, (int)threadIdx.x, i, j, k);
+    float sum = 0.f;
+#pragma unroll
+    for (int m = 0; m < 8; ++m)
+      sum += __shfl(t, ((2 * k + (m >> 2)) * L.ny + 2 * j + (m >> 1 & 1)) * L.nx + 2 * i + (m & 1));
+    to.r = SV::rnd(0.125f * sum);
+  }
+  __device__ __forceinline__ void prolong(const GcTailLvl& L, const GcTailLvl& C, const GctWave& from) {
+#pragma clang fp contract(off)
+    int i = 0, j = 0, k = 0;
+    if (colour >= 0) gct_decode(L, (int)threadIdx.x, i, j, k);
+    const float xp = __shfl(from.x, ((k >> 1) * C.ny + (j >> 1)) * C.nx + (i >> 1));
+    x = SV::rnd(x + xp);
+  }
+};
+
+// Levels first .. last (one or two: the second has at most eight cells, which
+// do not halve): r of `first` is restricted; leaves its x in LDS.
+template <int ST>
+__device__ __forceinline__ void gct_wave_cycle(float* lds, const GcTailLvl* tl, int first, int last, const TailSet& T) {
+  if (threadIdx.x < WAVE_CELLS) {
+    const GcTailLvl L = tl[first];
+    GctWave<ST> w;
+    w.load(lds, L, true);
+    if (first == last) {
+      w.sweeps(L, T.coarse, true, true);
+    } else {
+      const GcTailLvl C = tl[last];
+      GctWave<ST> v;
+      v.load(lds, C, false);
+      w.sweeps(L, T.pre, true, false);
+      w.restrict_to(L, C, v);
+      v.sweeps(C, T.coarse, true, true);
+      w.prolong(L, C, v);
+      w.sweeps(L, T.post, false, false);
+    }
+    if (w.colour >= 0) lds[L.o_x + (int)threadIdx.x] = w.x;
   }
   __syncthreads();
 }
 
-// The passes of a level with even rows and at most 4096 cells, each thread's
-// cells in registers: two of each colour (pairs q = thread, thread + 1024;
-// a pair holds one cell of each colour), with their couplings, Dirichlet part,
-// diagonal and r loaded once for the whole sequence, so that a pass reads
-// only the six neighbours from LDS. A neighbour index past the level's edge
-// reads another array of the workgroup's LDS (x lies between the couplings
-// and r, both at least a plane long); its coupling is zero and the row
-// leaves it out. Per cell the arithmetic of gct_pass, in the same order.
+// The passes of a level below the tail's first with even rows, each thread's
+// cells in registers: one of each colour (a pair of cells q = thread holds
+// one of each), with their couplings, Dirichlet part, diagonal and r loaded once for
+// the whole sequence, so that a pass reads only the six neighbours from LDS. A
+// neighbour index past the level's edge reads another array of the
+// workgroup's LDS (x lies between the couplings and r, both at least a plane
+// long); its coupling is zero and the row leaves it out. Per cell the
+// arithmetic of gct_pass, in the same order.
 template <int ST>
 struct GctCells {
   using SV = Store<ST>;
-  static constexpr int S = 2;  // pairs per thread
+  static constexpr int S = 1;  // pairs per thread
   float a[2][S][6], dd[2][S], dg[2][S], r[2][S];
   int c[2][S];  // -1: no cell
 
@@ -863,10 +917,6 @@ __device__ __forceinline__ void gct_sweeps(float* lds, const GcTailLvl& L, int c
     return;
   }
   bool fz = from_zero;
-  if (coarsest && L.n <= 64) {
-    gct_coarsest_wave<ST>(lds, L, count, from_zero);
-    return;
-  }
   const int passes = sweep_passes(coarsest, count);
   if ((L.nx & 1) == 0 && L.n <= 2 * GctCells<ST>::S * TAIL_THREADS) {
     GctCells<ST> cells;
@@ -883,6 +933,167 @@ __device__ __forceinline__ void gct_sweeps(float* lds, const GcTailLvl& L, int c
     fz = false;
   }
 }
+
+// The tail's first level with even rows, held in registers for the whole
+// kernel: a thread owns two pairs of cells (q = thread, thread + 1024; a pair
+// holds one cell of each colour) with their couplings, loaded straight from
+// global memory, Dirichlet parts, diagonals, r and x. LDS holds x by colour, a
+// pair's cell at X[colour * H + q], so that a pass reads the five neighbours
+// outside the pair at unit stride: the two cells of a pair are each other's
+// neighbour in x. A missing neighbour reads another cell, or the H floats of
+// LDS kept before and after X; its coupling is zero and the row leaves it out.
+// The kernel is bound by the vector instructions and latencies of one CU: with
+// 16^3 as its first level 29.4 us when each step gathered that level's
+// couplings and x from LDS, 22.3 with it in registers.
+template <int ST>
+struct GctTop {
+  using SV = Store<ST>;
+  using T = typename SV::T;
+  static constexpr int S = 2, H = TAIL_CELLS / 2;
+  float a[2][S][6], dd[2][S], dg[2][S], r[2][S], x[2][S];
+  int q;                 // the thread's first pair
+  int ym, yp, zm, zp;    // its neighbours' pairs; the second pair's lie TAIL_THREADS on
+  int side[S];           // the x neighbour's pair of the colour-1 cell
+  bool in[S], odd[S];    // odd: the pair's first cell has colour 1
+
+  __device__ __forceinline__ void load(const float* pack, const Level& g, const GcTailLvl& L) {
+#pragma clang fp contract(off)
+    const int hx = L.nx >> 1, m = L.n >> 1, plane = hx * L.ny;
+    const T* gr = reinterpret_cast<const T*>(g.r);
+    auto ld2 = [](const float* p) { return *reinterpret_cast<const float2*>(p); };
+    q = (int)threadIdx.x;
+    ym = q - hx;
+    yp = q + hx;
+    zm = q - plane;
+    zp = q + plane;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      in[s] = q + s * TAIL_THREADS < m;
+      const int c = in[s] ? q + s * TAIL_THREADS : 0;  // (any cell for the loads)
+      const int row = (int)(((float)c + 0.5f) * L.rhx);
+      const int u = c - row * hx;
+      const int k = (int)(((float)row + 0.5f) * L.rny);
+      const int j = row - k * L.ny;
+      odd[s] = ((j + k) & 1) != 0;
+      side[s] = q + (odd[s] ? -1 : 1);
+      const bool hxp = u + 1 < hx, hyp = j + 1 < L.ny, hzp = k + 1 < L.nz;
+      const float *fx = pack + 2 * c, *fy = fx + L.n, *fz = fy + L.n;
+      const float2 x2 = ld2(fx), y2 = ld2(fy), z2 = ld2(fz), d2 = ld2(fz + L.n), r2 = SV::ld2(gr, (size_t)(2 * c));
+      const float xn = fx[hxp ? 2 : 0];
+      const float2 yn = ld2(fy + (hyp ? L.nx : 0)), zn = ld2(fz + (hzp ? 2 * plane : 0));
+#pragma unroll
+      for (int col = 0; col < 2; ++col) {
+        const bool second = (col == 1) != odd[s];  // the pair's second cell
+        float* f = a[col][s];
+        f[0] = second ? x2.y : x2.x;
+        f[1] = second ? (hxp ? xn : 0.f) : x2.y;
+        f[2] = second ? y2.y : y2.x;
+        f[3] = hyp ? (second ? yn.y : yn.x) : 0.f;
+        f[4] = second ? z2.y : z2.x;
+        f[5] = hzp ? (second ? zn.y : zn.x) : 0.f;
+        dd[col][s] = second ? d2.y : d2.x;
+        r[col][s] = second ? r2.y : r2.x;
+        dg[col][s] = in[s] ? gc_diag(f, dd[col][s], L.inv) : 0.f;
+        x[col][s] = 0.f;
+      }
+    }
+  }
+  template <int COL>
+  __device__ __forceinline__ float row(const float* X, const GcTailLvl& L, int s) const {
+    const float* o = X + (COL ^ 1) * H + s * TAIL_THREADS;  // the other colour
+    const bool second = (COL == 1) != odd[s];
+    const float own = x[COL ^ 1][s], xs = o[COL == 1 ? side[s] : 2 * q - side[s]];
+    const float nb[6] = {second ? own : xs, second ? xs : own, o[ym], o[yp], o[zm], o[zp]};
+    return gc_row(a[COL][s], dd[COL][s], L.inv, x[COL][s], nb);
+  }
+  // One colour; first: x starts at zero.
+  template <int COL>
+  __device__ __forceinline__ void pass(float* X, const GcTailLvl& L, bool first) {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      if (!in[s]) continue;
+      const float d = dg[COL][s];
+      if (first) {
+        x[COL][s] = d > 0.f ? SV::rnd(r[COL][s] / d) : 0.f;
+        X[(COL ^ 1) * H + s * TAIL_THREADS + q] = 0.f;
+      } else if (d > 0.f) {
+        x[COL][s] = SV::rnd(x[COL][s] + (r[COL][s] - row<COL>(X, L, s)) / d);
+      }
+      X[COL * H + q + s * TAIL_THREADS] = x[COL][s];
+    }
+    __syncthreads();
+  }
+  __device__ __forceinline__ void sweeps(float* X, const GcTailLvl& L, int count, bool forward, bool coarsest) {
+    const int passes = sweep_passes(coarsest, count);
+    for (int i = 0; i < passes; ++i) {
+      if (sweep_colour(coarsest, forward, count, i) == 0) pass<0>(X, L, forward && i == 0);
+      else pass<1>(X, L, forward && i == 0);
+    }
+    if (passes == 0 && forward) clear(X);
+  }
+  // x = 0, in LDS too
+  __device__ __forceinline__ void clear(float* X) {
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      if (in[s]) X[q + s * TAIL_THREADS] = X[H + q + s * TAIL_THREADS] = 0.f;
+    __syncthreads();
+  }
+  // r of C = restriction of the residual: the residuals in LDS in place of x
+  // (the owners have it; the prolongation writes it again), a coarse cell's
+  // children summed in order (z, y, x; x fastest).
+  __device__ __forceinline__ void restrict_to(float* X, float* lds, const GcTailLvl& L, const GcTailLvl& C) {
+#pragma clang fp contract(off)
+    float t[2][S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      t[0][s] = r[0][s] - row<0>(X, L, s);
+      t[1][s] = r[1][s] - row<1>(X, L, s);
+    }
+    __syncthreads();
+    float2* res = reinterpret_cast<float2*>(X);
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      if (in[s]) res[q + s * TAIL_THREADS] = odd[s] ? make_float2(t[1][s], t[0][s]) : make_float2(t[0][s], t[1][s]);
+    __syncthreads();
+    const int hx = L.nx >> 1, plane = hx * L.ny;
+    for (int cc = (int)threadIdx.x; cc < C.n; cc += TAIL_THREADS) {
+      int i, j, k;
+      gct_decode(C, cc, i, j, k);
+      const int f = 2 * (k * plane + j * hx) + i;
+      const float2 v[4] = {res[f], res[f + hx], res[f + plane], res[f + plane + hx]};
+      float sum = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { sum += v[e].x; sum += v[e].y; }
+      lds[C.o_r + cc] = SV::rnd(0.125f * sum);
+    }
+    __syncthreads();
+  }
+  // x += x of its parent (one for both cells of a pair)
+  __device__ __forceinline__ void prolong(float* X, const float* lds, const GcTailLvl& L, const GcTailLvl& C) {
+#pragma clang fp contract(off)
+    const int hx = L.nx >> 1;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      if (!in[s]) continue;
+      const int c = q + s * TAIL_THREADS;
+      const int row = (int)(((float)c + 0.5f) * L.rhx);
+      const int k = (int)(((float)row + 0.5f) * L.rny);
+      const int j = row - k * L.ny;
+      const float xp = lds[C.o_x + ((k >> 1) * C.ny + (j >> 1)) * hx + c - row * hx];
+#pragma unroll
+      for (int col = 0; col < 2; ++col) X[col * H + c] = x[col][s] = SV::rnd(x[col][s] + xp);
+    }
+    __syncthreads();
+  }
+  __device__ __forceinline__ void store(const Level& g) const {
+    T* gx = reinterpret_cast<T*>(g.x);
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      if (in[s])
+        SV::st2(gx, (size_t)(2 * (q + s * TAIL_THREADS)), odd[s] ? make_float2(x[1][s], x[0][s]) : make_float2(x[0][s], x[1][s]));
+  }
+};
 
 // r of level C = restriction of the residual of level L. Eight consecutive
 // lanes take the eight children of one coarse cell, one residual each, and
@@ -926,50 +1137,56 @@ __device__ __forceinline__ void gct_prolong(float* lds, const GcTailLvl& L, cons
 
 // coarse_cycle3 (delta3d_multigrid.rs:303-332) over the tail levels, red-black
 // smoothing, Galerkin levels; the first level's r is restricted, its x is
-// written back.
-template <int ST>
+// written back. TOP: the first level has even rows and is held in registers
+// (GctTop), its x between two guards in the first 2 TAIL_CELLS floats of LDS; else (a single level:
+// odd rows do not halve) it is in LDS as the levels below are.
+template <int ST, bool TOP>
 __global__ void __launch_bounds__(TAIL_THREADS) k_gc_tail(TailSet T, Ctl* ctl) {
 #pragma clang fp contract(off)
   using SV = Store<ST>;
+  using SVT = typename SV::T;
   if (!ctl->active) return;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   __shared__ GcTailLvl tl[TAIL_MAX_LEVELS];
   static_assert(sizeof(tl) <= TAIL_STATIC_LDS, "static LDS of the tail");
-  int total = 0;  // cells of all tail levels
-  for (int l = 0; l < T.count; ++l) total += (int)T.lv[l].n;
-  if (threadIdx.x == 0) {
-    int off = 0, xr = 4 * total;
-    for (int l = 0; l < T.count; ++l) {
-      const Level& g = T.lv[l];
-      GcTailLvl& L = tl[l];
-      L.nx = g.nx; L.ny = g.ny; L.nz = g.nz; L.n = (int)g.n; L.inv = g.inv;
-      L.rnx = 1.0f / (float)g.nx; L.rny = 1.0f / (float)g.ny; L.rhx = 1.0f / (float)(g.nx >> 1 > 0 ? g.nx >> 1 : 1);
-      L.o_fx = off; off += L.n;
-      L.o_fy = off; off += L.n;
-      L.o_fz = off; off += L.n;
-      L.o_dd = off; off += L.n;
-      L.o_x = xr; xr += L.n;
-      L.o_r = xr; xr += L.n;
-    }
+  constexpr int FIRST = TOP ? 1 : 0;  // the first level in LDS
+  constexpr int TOP_FLOATS = TOP ? 2 * TAIL_CELLS : 0;
+  int total = 0;                      // cells of the levels in LDS
+  for (int l = FIRST; l < T.count; ++l) total += (int)T.lv[l].n;
+  if (threadIdx.x < (unsigned)T.count) {
+    const int l = (int)threadIdx.x;
+    int before = 0;
+    for (int m = FIRST; m < l; ++m) before += (int)T.lv[m].n;
+    const Level& g = T.lv[l];
+    GcTailLvl& L = tl[l];
+    L.nx = g.nx; L.ny = g.ny; L.nz = g.nz; L.n = (int)g.n; L.inv = g.inv;
+    L.rnx = 1.0f / (float)g.nx; L.rny = 1.0f / (float)g.ny; L.rhx = 1.0f / (float)(g.nx >> 1 > 0 ? g.nx >> 1 : 1);
+    const int off = TOP_FLOATS + 4 * before, xr = TOP_FLOATS + 4 * total + 2 * before;
+    L.o_fx = off;
+    L.o_fy = off + L.n;
+    L.o_fz = off + 2 * L.n;
+    L.o_dd = off + 3 * L.n;
+    L.o_x = xr;
+    L.o_r = xr + L.n;
   }
-  // the couplings of every level: one contiguous copy of 4 * total floats
-  // (a multiple of four, 16-byte aligned at both ends), one round of loads
+  // the couplings of every level in LDS: one contiguous copy of 4 * total
+  // floats (a multiple of four, 16-byte aligned at both ends), one round of loads
   {
-    const float4* src = reinterpret_cast<const float4*>(T.pack);
-    float4* dst = reinterpret_cast<float4*>(lds);
-    constexpr int MAXQ = (GC_TAIL_LDS_FLOATS / 6 + TAIL_THREADS - 1) / TAIL_THREADS;  // float4s per thread
+    const float4* src = reinterpret_cast<const float4*>(T.pack) + (TOP ? T.lv[0].n : 0);
+    float4* dst = reinterpret_cast<float4*>(lds + TOP_FLOATS);
+    constexpr int MAXQ = ((TOP ? TAIL_CELLS / 4 : TAIL_CELLS) + TAIL_THREADS - 1) / TAIL_THREADS;  // float4s per thread
     float4 v[MAXQ];
 #pragma unroll
     for (int u = 0; u < MAXQ; ++u) {
       const int q = (int)threadIdx.x + u * TAIL_THREADS;
       v[u] = q < total ? src[q] : f4zero();
     }
-    constexpr int RQ = (TAIL_CELLS + TAIL_THREADS - 1) / TAIL_THREADS;
-    float rv[RQ];
+    constexpr int RQ = TOP ? 0 : (TAIL_CELLS + TAIL_THREADS - 1) / TAIL_THREADS;
+    float rv[RQ + 1];
 #pragma unroll
     for (int u = 0; u < RQ; ++u) {
       const int q = (int)threadIdx.x + u * TAIL_THREADS;
-      rv[u] = q < (int)T.lv[0].n ? SV::ld(reinterpret_cast<const typename SV::T*>(T.lv[0].r), q) : 0.f;
+      rv[u] = q < (int)T.lv[0].n ? SV::ld(reinterpret_cast<const SVT*>(T.lv[0].r), q) : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < MAXQ; ++u) {
@@ -977,33 +1194,62 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_gc_tail(TailSet T, Ctl* ctl) {
       if (q < total) dst[q] = v[u];
     }
     __syncthreads();  // tl
-    const int orr = tl[0].o_r, n0 = tl[0].n;
+    if (!TOP) {
+      const int orr = tl[0].o_r, n0 = tl[0].n;
 #pragma unroll
-    for (int u = 0; u < RQ; ++u) {
-      const int q = (int)threadIdx.x + u * TAIL_THREADS;
-      if (q < n0) lds[orr + q] = rv[u];
+      for (int u = 0; u < RQ; ++u) {
+        const int q = (int)threadIdx.x + u * TAIL_THREADS;
+        if (q < n0) lds[orr + q] = rv[u];
+      }
     }
   }
-  __syncthreads();
-  // down to the coarsest level and back up
   const int last = T.count - 1;
-  for (int step = 0; step <= 2 * last; ++step) {
-    const bool down = step <= last;
-    const int l = down ? step : 2 * last - step;
+  GctTop<ST> top;
+  const GcTailLvl L0 = tl[0];
+  float* X = lds + GctTop<ST>::H;
+  if (TOP) {
+    top.load(T.pack, T.lv[0], L0);
+    top.sweeps(X, L0, last == 0 ? T.coarse : T.pre, true, last == 0);
+    if (last > 0) top.restrict_to(X, lds, L0, tl[1]);
+  } else {
+    __syncthreads();
+  }
+  // down to the coarsest level and back up; the levels from `wave` on in the first wavefront
+  int wave = T.count;
+  while (wave > FIRST && T.lv[wave - 1].n <= (size_t)WAVE_CELLS && wave + 2 > T.count) --wave;
+  const int bottom = wave <= last ? wave : last;
+  for (int step = FIRST; step <= 2 * bottom - FIRST; ++step) {
+    const bool down = step <= bottom;
+    const int l = down ? step : 2 * bottom - step;
+    if (l == wave) {
+      gct_wave_cycle<ST>(lds, tl, wave, last, T);
+      continue;
+    }
     // level descriptors in registers: the passes do not reload them after each barrier
     const GcTailLvl L = tl[l];
     if (!down) gct_prolong<ST>(lds, L, tl[l + 1]);
     gct_sweeps<ST>(lds, L, l == last ? T.coarse : down ? T.pre : T.post, down, l == last, down);
     if (l < last && down) gct_restrict<ST>(lds, L, tl[l + 1]);
   }
-  const GcTailLvl L0 = tl[0];
-  for (int q = threadIdx.x; q < L0.n; q += TAIL_THREADS)
-    SV::st(reinterpret_cast<typename SV::T*>(T.lv[0].x), q, lds[L0.o_x + q]);
+  if (TOP) {
+    if (last > 0) {
+      top.prolong(X, lds, L0, tl[1]);
+      top.sweeps(X, L0, T.post, false, false);
+    }
+    top.store(T.lv[0]);
+  } else {
+    for (int q = threadIdx.x; q < L0.n; q += TAIL_THREADS)
+      SV::st(reinterpret_cast<SVT*>(T.lv[0].x), q, lds[L0.o_x + q]);
+  }
 }
 
+// The first level in registers (GctTop): even rows.
+inline bool gc_tail_top(const Level* lv) { return lv[0].nx % 2 == 0; }
+
 inline size_t gc_tail_lds_bytes(const Level* lv, int count) {
-  size_t floats = 0;
-  for (int l = 0; l < count; ++l) floats += 6 * lv[l].n;
+  const bool top = gc_tail_top(lv);
+  size_t floats = top ? 2 * (size_t)TAIL_CELLS : 0;
+  for (int l = top ? 1 : 0; l < count; ++l) floats += 6 * lv[l].n;
   return floats * sizeof(float);
 }
 

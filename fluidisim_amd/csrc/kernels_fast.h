@@ -1440,11 +1440,11 @@ __global__ void __launch_bounds__(QBLOCK) k_q_update(size_t nquads, double* p, f
 constexpr int TAIL_THREADS = 1024;
 constexpr int TAIL_MAX_LEVELS = 8;
 constexpr int TAIL_CELLS = 4096;                // largest first level of the tail
-// LDS of the compact tail workgroup: the levels from one of TAIL_CELLS cells
-// down (4096 + 512 + ... = 4681 cells of 6 floats, 110 KiB). A closed box of
-// 64^3 with its coarsest level of 16^3 ran that level's 16 colour passes as
-// launches of their own when the limit was 64 KiB.
-constexpr int GC_TAIL_LDS_FLOATS = 6 * (TAIL_CELLS + TAIL_CELLS / 4);
+// Limit of a tail workgroup's LDS (the row-coefficient tail's; the compact
+// tail holds its first level in registers and takes half). With a limit of 64 KiB
+// on levels held in LDS a closed box of 64^3 ran the 16 colour passes of its
+// coarsest level, 16^3, as launches of their own.
+constexpr int TAIL_LDS_FLOATS = 6 * (TAIL_CELLS + TAIL_CELLS / 4);
 
 struct TailSet {
   Level lv[TAIL_MAX_LEVELS];  // global arrays of the tail levels (first .. last)

@@ -52,6 +52,14 @@ def assert_vcycle_is_the_oracles(wl, **overrides):
     ((20, 12, 12), 1, (2, 2, 1)),   # 10 x 6 x 6, one coarsest sweep
     ((36, 32, 32), 1, (2, 2, 2)),   # 18 x 16 x 16: one level too large for the tail
     ((52, 8, 24), 2, (2, 2, 3)),    # 26 x 12 x 4 over 13 x 6 x 2: odd rows
+    ((16, 8, 16), -1, (2, 2, 4)),   # 8 x 8 x 4 over 4 x 4 x 2: the last level in one wavefront
+    ((16, 16, 16), -1, (1, 3, 3)),  # 8^3 over 4^3 over 2^3: two levels in one wavefront
+    ((16, 16, 16), -1, (2, 2, 0)),  # no coarsest sweep
+    ((20, 12, 12), -1, (2, 1, 5)),  # 10 x 6 x 6 over 5 x 3 x 3
+    ((8, 8, 8), 1, (2, 2, 2)),      # 4^3 alone
+    ((12, 8, 8), -1, (2, 2, 3)),    # 6 x 4 x 4 over 3 x 2 x 2
+    ((128, 8, 64), 1, (2, 2, 2)),   # 64 x 32 x 4 = 8192: above the tail
+    ((128, 4, 64), 1, (2, 2, 3)),   # 64 x 32 x 2: the longest plane
 ])
 def test_tail_levels_match_the_oracle(size, levels, sweeps):
     wl = W.tank(*size, seed=21)
