@@ -53,6 +53,7 @@ struct fsp_solver {
   // padded with solid cells in x to rows that do: its solver (null: none), on
   // this solver's stream. This solver keeps the caller's arrays and geometry.
   fsp_solver* inner = nullptr;
+  uint32_t *wetq = nullptr, *wetb = nullptr;  // Fine::wetq, wetb
   FinishSet fins{};  // folds put off to the next launch of k_finish
   bool shares_stream = false;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -176,6 +177,8 @@ struct fsp_solver {
     G.gk0 = gk0;
     G.gtab = gtab;
     G.precv = precv;
+    G.wetq = wetq;
+    G.wetb = wetb;
     const bool indexed = (frac || levelset) && gidx;
     G.gq = indexed ? gidx : nullptr;
     G.gent = gent;
@@ -339,9 +342,11 @@ bool coarsens3(size_t nx, size_t ny, size_t nz) {
   return nx % 2 == 0 && ny % 2 == 0 && nz % 2 == 0 && nx >= 4 && ny >= 4 && nz >= 4;
 }
 
-__global__ void k_reset(Ctl* ctl, int gauge) {
+// wetb: the wet flags of `bricks` bricks, cleared too.
+__global__ void __launch_bounds__(BLOCK) k_reset(Ctl* ctl, int gauge, uint32_t* wetb, int bricks) {
   static_assert(sizeof(Ctl) % 4 == 0, "cleared in words");
   for (int q = (int)threadIdx.x; q < (int)(sizeof(Ctl) / 4); q += (int)blockDim.x) reinterpret_cast<uint32_t*>(ctl)[q] = 0;
+  for (int q = (int)threadIdx.x; q < bricks; q += (int)blockDim.x) wetb[q] = 0;
   __syncthreads();
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   ctl->first_dir = 1;
@@ -393,13 +398,14 @@ struct Launch {
       // labels and level set: no column structure, no ghost-row table
       FSP_LAUNCH(S, k_mask_ls, g, st, G, S->mask, S->ctl, S->partials);
       FSP_DEFER(S, OP_COUNT, g, false, 0);
+      if (S->quad) FSP_LAUNCH(S, k_wet_flags, qgrid(S->qfine), st, G, S->qfine, S->brick);
       ghost_rows();
       if (S->precv) FSP_LAUNCH(S, k_prec, g, st, G, S->precv);
       return;
     }
     if (S->quad) {
       const dim3 gq((unsigned)(S->qfine.nbx * S->qfine.nby * S->qfine.planes));
-      FSP_LAUNCH(S, k_mask_q, gq, st, G, S->qfine, S->mask, S->ctl, S->partials);
+      FSP_LAUNCH(S, k_mask_q, gq, st, G, S->qfine, S->brick, S->mask, S->ctl, S->partials);
       FSP_DEFER(S, OP_COUNT, gq, false, 0);
     } else {
       FSP_LAUNCH(S, k_mask, g, st, G, S->mask, S->ctl, S->partials);
@@ -675,10 +681,7 @@ struct Launch {
       if (l < last) {
         Level& C = S->levels[l + 1];
         if (L.compact) {
-          // the restriction's grid for 128-thread halves (k_gc_restrict2)
-          QuadGrid H = S->cqr[l];
-          H.RY = (QBLOCK / 2) / H.QX;
-          H.nby = (H.rows + H.RY - 1) / H.RY;
+          const QuadGrid H = half_grid(S->cqr[l]);
           FSP_LAUNCH_N(S, "k_gc_restrict", (k_gc_restrict2<ST>), qgrid(H), st, L, H, (const TS<ST>*)xcur[l], C,
                        S->ctl);
         } else {
@@ -792,10 +795,7 @@ struct Launch {
   // The residual of z on quads restricted to the first coarse level (k_q_restrict2).
   template <int ST>
   void restrict_quads(const TS<ST>* z, const Level& L0) {
-    // the restriction's grid for 128-thread halves
-    QuadGrid H = S->qrestr;
-    H.RY = (QBLOCK / 2) / H.QX;
-    H.nby = (H.rows + H.RY - 1) / H.RY;
+    const QuadGrid H = half_grid(S->qrestr);
     const dim3 gr((unsigned)(H.nbx * H.nby * H.planes));
     FSP_LAUNCH_FORM(S, "k_q_restrict", (k_q_restrict2<ST, FORM_TABLE>), (k_q_restrict2<ST, FORM_INDEX>),
                     (k_q_restrict2<ST, FORM_GENERAL>), gr, BLOCK, st, G, H, z, (const float*)S->r, L0, S->ctl);
@@ -961,11 +961,9 @@ struct Launch {
       const unsigned folded = g.x <= (unsigned)FSP_FOLD_PARTIALS ? g.x : 0u;
       if (folded) FSP_DEFER(S, OP_DQ, g, false, 1);
       else FSP_FINISH(S, st, OP_DQ, g, false, 1);
-      const size_t nquads = G.n / 4;
-      const dim3 gu((unsigned)((nquads + QBLOCK - 1) / QBLOCK));
-      FSP_LAUNCH(S, k_q_update, gu, st, nquads, S->p64, S->r, (const float*)S->d0, (const float*)S->d1,
+      FSP_LAUNCH(S, k_q_update, g, st, G, Q, S->p64, S->r, (const float*)S->d0, (const float*)S->d1,
                  (const float*)S->q, S->ctl, S->partials, folded);
-      FSP_DEFER(S, OP_RN, gu, false, 1);
+      FSP_DEFER(S, OP_RN, g, false, 1);
     } else {
       FSP_LAUNCH(S, k_spmv_dir, dim3(grid_for(G.n)), st, G, S->zres, S->d0, S->d1, S->q, S->ctl, S->partials);
       FSP_FINISH(S, st, OP_DQ, dim3(grid_for(G.n)), false, 1);
@@ -1363,7 +1361,7 @@ fsp_status pad_geometry(fsp_solver* S, bool edge_open) {
 // (delta3d_mobile.rs:479-484). defer: OP_COUNT's fold is left to the caller.
 void build_geometry(fsp_solver* S, bool hierarchy, bool prec = true, bool defer = false) {
   Launch K(S);
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, K.st, S->ctl, S->opt.gauge);
+  k_reset<<<1, BLOCK, 0, K.st>>>(S->ctl, S->opt.gauge, S->wetb, S->brick.bx * S->brick.by * S->brick.bz);
   S->fins.count = 0;
   K.mask(prec);
   if (!defer) flush_finish(S, K.st);
@@ -1959,28 +1957,22 @@ fsp_status create_solver(const fsp_domain* d, const fsp_options* o, fsp_solver* 
     }
   }
   // fast paths
-  auto make_q = [](int nq, int rows, int planes) {
-    QuadGrid Q{};
-    int qx = 1;
-    while (qx < nq && qx < FSP_QX_MAX) qx <<= 1;
-    Q.nq = nq; Q.QX = qx; Q.RY = QBLOCK / qx;
-    Q.nbx = (nq + qx - 1) / qx;
-    Q.nby = (rows + Q.RY - 1) / Q.RY;
-    Q.rows = rows; Q.planes = planes;
-    return Q;
-  };
   if (nx % 4 == 0) {
-    S->qfine = make_q((int)nx / 4, (int)ny, (int)nz);
-    S->qrestr = make_q((int)nx / 4, (int)ny / 2, (int)nz / 2);
+    S->qfine = quad_grid((int)nx / 4, (int)ny, (int)nz);
+    S->qrestr = quad_grid((int)nx / 4, (int)ny / 2, (int)nz / 2);
     const size_t blocks = (size_t)S->qfine.nbx * S->qfine.nby * S->qfine.planes;
     S->quad = blocks <= (size_t)MAX_PARTIALS && (S->n / 4 + QBLOCK - 1) / QBLOCK <= (size_t)MAX_PARTIALS;
     if (S->quad && opt.fine_sweeps == FSP_SWEEP_FUSED) {
       S->brick.bx = ((int)nx / 4 + BR_QX - 1) / BR_QX;
       S->brick.by = ((int)ny + BR_Y - 1) / BR_Y;
       S->brick.bz = ((int)nz + BR_Z - 1) / BR_Z;
+      S->brick.mx = block_divisor(S->brick.bx);
+      S->brick.mz = block_divisor(S->brick.bz);
       if ((size_t)S->brick.bx * S->brick.by * S->brick.bz > (size_t)MAX_PARTIALS) S->brick = BrickGrid{};
     }
   }
+  if (S->quad && ((st = dalloc(S, &S->wetq, (size_t)MAX_PARTIALS)) || (st = dalloc(S, &S->wetb, (size_t)MAX_PARTIALS))))
+    return fail(st);
   if (opt.preconditioner == FSP_PRECOND_LEARNED && opt.learned_vcycle && !quad_vcycle_ok(S->quad, opt))
     return fail(FSP_INVALID);
   if (opt.preconditioner != FSP_PRECOND_JACOBI && (quad_vcycle_ok(S->quad, opt) || quad_jacobi_ok(S->quad, opt)) &&
@@ -2015,7 +2007,7 @@ fsp_status create_solver(const fsp_domain* d, const fsp_options* o, fsp_solver* 
     for (int l = 0; l < S->tail_first && l < 5; ++l) {
       Level& L = S->levels[l];
       if (L.nx % 4 != 0) continue;
-      QuadGrid q = make_q(L.nx / 4, L.ny, L.nz);
+      QuadGrid q = quad_grid(L.nx / 4, L.ny, L.nz);
       const size_t blocks = (size_t)q.nbx * q.nby * q.planes;
       if (blocks > 0xFFFFFFFFu) continue;
       if ((st = dalloc(S, &L.cx, L.n)) || (st = dalloc(S, &L.cy, L.n)) || (st = dalloc(S, &L.cz, L.n)) ||
@@ -2023,7 +2015,7 @@ fsp_status create_solver(const fsp_domain* d, const fsp_options* o, fsp_solver* 
         return fail(st);
       L.compact = 1;
       S->cq[l] = q;
-      if (l + 1 < (int)S->levels.size()) S->cqr[l] = make_q(L.nx / 4, L.ny / 2, L.nz / 2);
+      if (l + 1 < (int)S->levels.size()) S->cqr[l] = quad_grid(L.nx / 4, L.ny / 2, L.nz / 2);
     }
   }
   // every other level above the compact tail: row coefficients
@@ -2862,14 +2854,6 @@ fsp_status fsp_autotune(fsp_solver* S, int32_t* tile_x, double* us) {
   hipLaunchKernelGGL(k_fill, dim3(grid_for(S->n)), dim3(BLOCK), 0, K.st, S->z, S->n, 0.f);
   hipLaunchKernelGGL(k_fill, dim3(grid_for(S->n)), dim3(BLOCK), 0, K.st, S->r, S->n, 1.f);
   K.set_pass(1, 0.0, 0.0, 0.0, 0, 1);
-  auto make_q = [](int nqv, int rows, int planes, int qx) {
-    QuadGrid Q{};
-    Q.nq = nqv; Q.QX = qx; Q.RY = QBLOCK / qx;
-    Q.nbx = (nqv + qx - 1) / qx;
-    Q.nby = (rows + Q.RY - 1) / Q.RY;
-    Q.rows = rows; Q.planes = planes;
-    return Q;
-  };
   int widest = 1;
   while (widest < nq && widest < 64) widest <<= 1;
   int best = S->qfine.QX;
@@ -2877,7 +2861,7 @@ fsp_status fsp_autotune(fsp_solver* S, int32_t* tile_x, double* us) {
   const Level none_l{};
   const float* none = nullptr;
   for (int qx = widest; qx >= 4; qx >>= 1) {
-    const QuadGrid Q = make_q(nq, ny, nz, qx);
+    const QuadGrid Q = quad_grid(nq, ny, nz, qx, QBLOCK);
     const size_t blocks = (size_t)Q.nbx * Q.nby * Q.planes;
     if (blocks > (size_t)MAX_PARTIALS) continue;
     const dim3 g((unsigned)blocks);
@@ -2896,8 +2880,8 @@ fsp_status fsp_autotune(fsp_solver* S, int32_t* tile_x, double* us) {
     const double t = 1000.0 * ms / reps;
     if (t < best_us) { best_us = t; best = qx; }
   }
-  S->qfine = make_q(nq, ny, nz, best);
-  S->qrestr = make_q(nq, ny / 2, nz / 2, best);
+  S->qfine = quad_grid(nq, ny, nz, best, QBLOCK);
+  S->qrestr = quad_grid(nq, ny / 2, nz / 2, best, QBLOCK);
   // graphs hold the previous launch shapes: capture them again
   for (int gi = 0; gi < 2; ++gi) drop_graph(S, gi);
   fsp_status gst = prepare_graph(S, 0);

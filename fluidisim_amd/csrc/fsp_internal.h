@@ -130,6 +130,10 @@ struct Fine {
   const uint16_t* gk0;   // columns: lowest ghost row (0xFFFF: none)
   const float* gtab;     // columns x G_SLOTS x 8: 1/theta of the ghost faces
   const float* precv;    // cells: row_prec of every row (k_prec)
+  // On grids of quads, a word per block of the quad grid (in logical order)
+  // and per brick: a wet cell in it. On dry cells r, z, d and q are 0 or not
+  // read, and p keeps its value. (Words: a scalar load.)
+  uint32_t *wetq, *wetb;
   // Ghost rows of a geometry without column tables (fractional apertures, a
   // level set), on grids of quads: gq[quad] is the entry of the quad's first
   // ghost row, the others follow; GE_FLOATS floats an entry (1/theta of the

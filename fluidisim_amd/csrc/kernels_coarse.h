@@ -274,11 +274,11 @@ __global__ void __launch_bounds__(QBLOCK) k_gc_restrict2(Level F, QuadGrid H, co
   __shared__ float2 carry[QBLOCK / 2];
   if (!ctl->active) return;
   const int local = (int)(threadIdx.x & (QBLOCK / 2 - 1)), dz = (int)(threadIdx.x / (QBLOCK / 2));
-  const unsigned Lb = xcd_block(blockIdx.x, gridDim.x);
-  const unsigned bx = Lb % (unsigned)H.nbx, tb = Lb / (unsigned)H.nbx;
-  const int qx = (int)bx * H.QX + (local & (H.QX - 1));
-  const int J = (int)(tb % (unsigned)H.nby) * H.RY + local / H.QX;
-  const int K = (int)(tb / (unsigned)H.nby);
+  unsigned bx, by;
+  int K;
+  quad_block(H, xcd_block(blockIdx.x, gridDim.x), bx, by, K);
+  const int qx = ((int)bx << H.sx) + (local & (H.QX - 1));
+  const int J = (int)by * H.RY + (local >> H.sx);
   const bool valid = qx < H.nq && J < H.rows && K < H.planes;
   const size_t plane = (size_t)F.nx * F.ny;
   const T* fr = reinterpret_cast<const T*>(F.r);
