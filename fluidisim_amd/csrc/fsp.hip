@@ -6,9 +6,9 @@
 // after each pass, acceptance on the plain-row divergence with target
 // tightening, floor stops on the backward error or a repeated state of p.
 // The iterations themselves run on the device: every scalar of the CG
-// (alpha, beta, the loop test) is computed by the last block of the kernel
-// that produced its reduction, so the host only polls a small control block
-// between batches of iterations.
+// (alpha, beta, the loop test) is computed by k_finish, and the host launches
+// one iteration ahead of the running one, as the device reports their ends in
+// pinned memory.
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 

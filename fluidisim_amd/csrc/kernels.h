@@ -110,8 +110,8 @@ __device__ __forceinline__ void block_partial(double a, double b, int slot, doub
   }
 }
 
-// Scalar updates of the conjugate gradient, done on the device by the last
-// block of the kernel that produced the reduction (delta3d_mobile.rs:513-545).
+// Scalar updates of the conjugate gradient after a reduction's fold
+// (delta3d_mobile.rs:513-545).
 __device__ void finish(int op, Ctl* ctl, double a, double b) {
   switch (op) {
     case OP_B2:
