@@ -2576,6 +2576,10 @@ fsp_status fsp_precondition_device(fsp_solver* S, const float* d_r, float* d_z) 
   if (!S->geom) return FSP_DOMAIN;
   FSP_HIP(hipSetDevice(S->opt.device));
   build_geometry(S, true);
+  // r may be anything on dry cells too, and what the restriction takes of
+  // them reaches wet cells of the coarse levels: no block is left out (of a
+  // projection's r the dry cells are 0)
+  if (S->quad) FSP_HIP(hipMemsetAsync(S->wetq, 1, (size_t)MAX_PARTIALS * sizeof(uint32_t), S->stream));
   // the fine kernels' form a projection on this geometry takes
   if (const fsp_status st = sync_ctl(S)) return st;
   struct TableGuard {

@@ -201,3 +201,30 @@ def test_blocks_that_fall_dry_and_wet_leave_no_trace(size, options):
         for a, b in zip(got, ref):
             assert np.array_equal(bits(a), bits(b)), (step, fill)
     used.close()
+
+
+@pytest.mark.parametrize("options", [
+    dict(smoother=_lib.SMOOTH_RBGS, coarse_operator=_lib.COARSE_GALERKIN),
+    dict(smoother=_lib.SMOOTH_RBGS, coarse_operator=_lib.COARSE_GALERKIN, fine_sweeps=_lib.SWEEP_SINGLE),
+    dict(smoother=_lib.SMOOTH_JACOBI, coarse_operator=_lib.COARSE_REDISCRETISED),
+], ids=["bricks", "single", "jacobi"])
+@pytest.mark.parametrize("size", [(32, 24, 32), (128, 16, 32), (34, 24, 32)], ids=str)
+@pytest.mark.parametrize("tuned", [False, True], ids=["tile", "tuned"])
+def test_a_residual_on_air_is_restricted_with_the_rest(size, options, tuned):
+    """The preconditioner's argument is any vector: on the dry layers just
+    above the surface it reaches the second coarse level, whatever blocks the
+    fine kernels are split into."""
+    nx, ny, nz = size
+    wl = W.tank(nx, nz, ny, seed=91)
+    rng = np.random.default_rng(92)
+    # layers 16 and below wet: 18 and 19 are dry beside wet ones in a cell of the second coarse level
+    wl.eta = rng.uniform(17.1, 17.4, nx * ny).astype(np.float32)
+    wl.options.update(options)
+    vol = W.build_volume(wl)
+    if tuned:
+        vol.autotune()
+    r = rng.uniform(-1.0, 1.0, wl.domain.cells).astype(np.float32)
+    z = vol.precondition(torch.from_numpy(r).cuda()).cpu().numpy()
+    vol.close()
+    z_ref = po.vcycle(problem(wl), r, oracle_options(wl)).astype(np.float32)
+    assert np.array_equal(bits(z), bits(z_ref)), f"max diff {np.abs(z - z_ref).max()}"
