@@ -45,6 +45,15 @@ struct HostBlock {
   alignas(64) int stored;  // k_store_p has written p
 };
 
+// Live timing of one kernel (fsp_profile_begin / fsp_profile_end).
+struct Profile {
+  bool on = false;
+  std::string name;
+  std::vector<hipEvent_t> events;
+  size_t used = 0;
+  int32_t* active = nullptr;  // per timed launch: the loop-active flag it started with
+};
+
 struct fsp_solver {
   fsp_domain dom{};
   fsp_options opt{};
@@ -118,7 +127,6 @@ struct fsp_solver {
   uint32_t pass = 0;             // passes of the CG loop so far
   unsigned long long* hhash = nullptr;
   std::vector<void*> allocs;
-  // live timing of one kernel (fsp_profile_begin / fsp_profile_end)
   // one CG iteration captured as a graph, replayed per iteration
   // one CG iteration per (phase, kernel form): [FORMS * phase + form],
   // phase 0 as configured, 1 the learned phase
@@ -134,11 +142,8 @@ struct fsp_solver {
   float *flux_x = nullptr, *flux_y = nullptr;
   StepScalars* step_sc = nullptr;
   StepScalars* hstep = nullptr;
-  bool prof_on = false;
-  std::string prof_name;
-  std::vector<hipEvent_t> prof_events;
-  size_t prof_used = 0;
-  int32_t* prof_active = nullptr;  // per timed launch: the loop-active flag it started with
+  Profile own_prof;
+  Profile* prof = &own_prof;  // of a padded solver: the outer one's
 
   GradedCol graded_col() const {
     GradedCol D;
@@ -239,12 +244,12 @@ __global__ void k_prof_flag(const Ctl* ctl, int32_t* out) {
 // then goes through hipExtLaunchKernelGGL, whose events take the dispatch's
 // own start and end timestamps (no marker packets around it).
 inline bool prof_begin(fsp_solver* S, const char* name, hipStream_t stream, hipEvent_t* e0, hipEvent_t* e1) {
-  const bool on = S->prof_on && S->prof_name == name && S->prof_used + 2 <= S->prof_events.size();
+  const bool on = S->prof->on && S->prof->name == name && S->prof->used + 2 <= S->prof->events.size();
   if (on) {
-    k_prof_flag<<<1, 64, 0, stream>>>(S->ctl, S->prof_active + S->prof_used / 2);
-    *e0 = S->prof_events[S->prof_used];
-    *e1 = S->prof_events[S->prof_used + 1];
-    S->prof_used += 2;
+    k_prof_flag<<<1, 64, 0, stream>>>(S->ctl, S->prof->active + S->prof->used / 2);
+    *e0 = S->prof->events[S->prof->used];
+    *e1 = S->prof->events[S->prof->used + 1];
+    S->prof->used += 2;
   }
   return on;
 }
@@ -1040,10 +1045,10 @@ void cleanup(fsp_solver* S) {
     S->iter_exec[g] = nullptr;
     S->iter_graph[g] = nullptr;
   }
-  for (hipEvent_t e : S->prof_events) (void)hipEventDestroy(e);
-  S->prof_events.clear();
-  if (S->prof_active) (void)hipFree(S->prof_active);
-  S->prof_active = nullptr;
+  for (hipEvent_t e : S->own_prof.events) (void)hipEventDestroy(e);
+  S->own_prof.events.clear();
+  if (S->own_prof.active) (void)hipFree(S->own_prof.active);
+  S->own_prof.active = nullptr;
   for (void* p : S->allocs) (void)hipFree(p);
   S->allocs.clear();
   if (S->host) (void)hipHostFree(S->host);
@@ -1137,9 +1142,9 @@ fsp_status fingerprint(fsp_solver* S, const double* p, uint64_t& h) {
   return FSP_OK;
 }
 
-// The padded solver, where it projects (a kernel being timed runs in S itself).
+// The padded solver, where it projects.
 fsp_solver* padded(const fsp_solver* S) {
-  return S->inner && S->inner->geom && !S->prof_on ? S->inner : nullptr;
+  return S->inner && S->inner->geom && S->gnodes.empty() ? S->inner : nullptr;
 }
 
 // The kernel form of the geometry in place when every ghost row is where the
@@ -1155,8 +1160,8 @@ int fast_form(const fsp_solver* S) {
 fsp_status capture_iteration(fsp_solver* S) {
   const int slot = FORMS * S->net_phase + S->form;
   if (S->iter_exec[slot]) return FSP_OK;
-  const bool prof = S->prof_on;
-  S->prof_on = false;
+  const bool prof = S->prof->on;
+  S->prof->on = false;
   FSP_HIP(hipStreamBeginCapture(S->stream, hipStreamCaptureModeThreadLocal));
   {
     Launch K(S);
@@ -1164,7 +1169,7 @@ fsp_status capture_iteration(fsp_solver* S) {
   }
   hipGraph_t g = nullptr;
   const hipError_t e = hipStreamEndCapture(S->stream, &g);
-  S->prof_on = prof;
+  S->prof->on = prof;
   if (e != hipSuccess || !g) {
     std::fprintf(stderr, "fsp: graph capture failed: %s\n", hipGetErrorString(e));
     return FSP_DEVICE;
@@ -1201,9 +1206,9 @@ fsp_status prepare_graph(fsp_solver* S, int phase) {
   if (!S->opt.graph || (S->iter_exec[FORMS * phase + forms[0]] && S->iter_exec[FORMS * phase + forms[1]])) return FSP_OK;
   if (phase == 1 && !S->net) return FSP_OK;
   const int saved = S->net_phase, saved_form = S->form;
-  const bool prof = S->prof_on;
+  const bool prof = S->prof->on;
   S->net_phase = phase;
-  S->prof_on = false;
+  S->prof->on = false;
   hipError_t e = hipStreamBeginCapture(S->stream, hipStreamCaptureModeThreadLocal);
   if (e == hipSuccess) {
     {
@@ -1214,7 +1219,7 @@ fsp_status prepare_graph(fsp_solver* S, int phase) {
     e = hipStreamEndCapture(S->stream, &g);
     if (g) (void)hipGraphDestroy(g);
   }
-  S->prof_on = prof;
+  S->prof->on = prof;
   fsp_status st = e == hipSuccess ? FSP_OK : FSP_DEVICE;
   for (int t = 0; t < 2 && st == FSP_OK; ++t) {
     S->form = forms[t];
@@ -1274,6 +1279,18 @@ struct RowCopy {
   }
   void out(const float* a, float* b, size_t rows, int extra = 0) {
     add(a, b, I->dom.nx + extra, S->dom.nx + extra, rows);
+  }
+  // the surface, for a call that builds the padded geometry
+  void surface() {
+    const size_t ny = S->dom.ny, nz = S->dom.nz;
+    I->surf = S->surf;
+    in(S->eta, I->eta, ny);
+    in(S->eta_rt, I->eta_rt, ny);
+    if (!S->coupled) return;
+    in(S->total, I->total, ny);
+    in(S->bg_up, I->bg_up, ny);
+    in(S->bg_x, I->bg_x, ny * nz, 1);
+    in(S->bg_y, I->bg_y, (ny + 1) * nz);
   }
   void launch() {
     if (R.count == 0) return;
@@ -1560,21 +1577,13 @@ fsp_status run_padded(fsp_solver* S, const float* us, const float* vs, const flo
                       float* v, float* w, float scale, float k1, double rel_tol, uint32_t max_iters, fsp_report* rep) {
   fsp_solver* I = S->inner;
   const size_t ny = S->dom.ny, nz = S->dom.nz;
-  I->surf = S->surf;
   FSP_HIP(hipEventRecord(S->ev0, S->stream));
   RowCopy in(S);
   in.in(us, I->us, ny * nz, 1);
   in.in(vs, I->vs, (ny + 1) * nz);
   in.in(ws, I->ws, ny * (nz + 1));
   if (warm) in.in(p, I->p, ny * nz);
-  in.in(S->eta, I->eta, ny);
-  in.in(S->eta_rt, I->eta_rt, ny);
-  if (S->coupled) {
-    in.in(S->total, I->total, ny);
-    in.in(S->bg_up, I->bg_up, ny);
-    in.in(S->bg_x, I->bg_x, ny * nz, 1);
-    in.in(S->bg_y, I->bg_y, (ny + 1) * nz);
-  }
+  in.surface();
   in.launch();
   fsp_report R{};
   const fsp_status st =
@@ -1706,8 +1715,8 @@ fsp_status run(fsp_solver* S, const float* us, const float* vs, const float* ws,
       // launched one to three iterations too many and stopped the stream three
       // times a projection: 2.10 against 1.87 ms at 128^3, 4.50 against 4.08 at
       // 256x256x128.)
-      if (S->opt.graph && !S->prof_on && (st = capture_iteration(S))) return st;
-      const hipGraphExec_t gx = S->prof_on ? nullptr : S->iter_exec[FORMS * S->net_phase + S->form];
+      if (S->opt.graph && !S->prof->on && (st = capture_iteration(S))) return st;
+      const hipGraphExec_t gx = S->prof->on ? nullptr : S->iter_exec[FORMS * S->net_phase + S->form];
       const double goal = std::min(tol_b2, physical_target);
       PassState done{it, true, false, rr};
       double rate = 1.0;  // |r|^2 per iteration, observed
@@ -1905,6 +1914,7 @@ fsp_status create_solver(const fsp_domain* d, const fsp_options* o, fsp_solver* 
   if (outer) {
     S->stream = outer->stream;
     S->shares_stream = true;
+    S->prof = outer->prof;
   } else if (hipStreamCreateWithFlags(&S->stream, hipStreamNonBlocking) != hipSuccess) {
     return fail(FSP_DEVICE);
   }
@@ -2575,6 +2585,20 @@ fsp_status fsp_precondition_device(fsp_solver* S, const float* d_r, float* d_z) 
   if (!S || !d_r || !d_z) return FSP_INVALID;
   if (!S->geom) return FSP_DOMAIN;
   FSP_HIP(hipSetDevice(S->opt.device));
+  if (fsp_solver* I = padded(S)) {
+    const size_t rows = (size_t)S->dom.ny * S->dom.nz;
+    RowCopy in(S);
+    in.in(d_r, I->b, rows);
+    in.surface();
+    in.launch();
+    if (const fsp_status st = fsp_precondition_device(I, I->b, I->p)) return st;
+    RowCopy out(S);
+    out.out(I->p, d_z, rows);
+    out.launch();
+    FSP_HIP(hipGetLastError());
+    FSP_HIP(hipStreamSynchronize(S->stream));
+    return FSP_OK;
+  }
   build_geometry(S, true);
   // r may be anything on dry cells too, and what the restriction takes of
   // them reaches wet cells of the coarse levels: no block is left out (of a
@@ -2718,7 +2742,7 @@ fsp_status fsp_step_surface_mobile_device(fsp_solver* S, float* d_u, float* d_v,
   const Fine G = S->fine();
   k_step_reset<<<1, 1, 0, S->stream>>>(S->step_sc);
   k_step_scalars<<<1, STEP_THREADS, 0, S->stream>>>(G, S->col_floor, S->flux_x, S->flux_y, S->step_sc);
-  const fsp_solver* P = S->gnodes.empty() && padded(S) ? padded(S) : S;  // the one that projected
+  const fsp_solver* P = padded(S) ? padded(S) : S;  // the one that projected
   const FiniteSet F{{d_u, d_v, d_w, d_p, S->eta, S->eta_rt, S->us, S->vs, S->ws, P->b, P->r},
                     {S->nu, S->nv, S->nw, S->n, S->ncols, S->ncols, S->nu, S->nv, S->nw, P->n, P->n}};
   size_t longest = 0;
@@ -2846,6 +2870,13 @@ fsp_status fsp_project_batch(fsp_solver* const* solvers, const fsp_patch_io* io,
 fsp_status fsp_autotune(fsp_solver* S, int32_t* tile_x, double* us) {
   if (!S) return FSP_INVALID;
   if (!S->geom) return FSP_DOMAIN;
+  if (fsp_solver* I = padded(S)) {
+    FSP_HIP(hipSetDevice(S->opt.device));
+    RowCopy in(S);
+    in.surface();
+    in.launch();
+    return fsp_autotune(I, tile_x, us);
+  }
   if (!S->quad) {
     if (tile_x) *tile_x = 0;
     if (us) *us = 0.0;
@@ -2900,16 +2931,16 @@ fsp_status fsp_profile_begin(fsp_solver* S, const char* kernel, uint32_t max_lau
   if (!S || !kernel || max_launches == 0) return FSP_INVALID;
   FSP_HIP(hipSetDevice(S->opt.device));
   FSP_HIP(hipStreamSynchronize(S->stream));
-  for (hipEvent_t e : S->prof_events) (void)hipEventDestroy(e);
-  S->prof_events.clear();
-  if (S->prof_active) (void)hipFree(S->prof_active);
-  S->prof_active = nullptr;
-  FSP_HIP(hipMalloc((void**)&S->prof_active, (size_t)max_launches * sizeof(int32_t)));
-  S->prof_events.assign(2 * (size_t)max_launches, nullptr);
-  for (auto& e : S->prof_events) FSP_HIP(hipEventCreate(&e));
-  S->prof_name = kernel;
-  S->prof_used = 0;
-  S->prof_on = true;
+  for (hipEvent_t e : S->prof->events) (void)hipEventDestroy(e);
+  S->prof->events.clear();
+  if (S->prof->active) (void)hipFree(S->prof->active);
+  S->prof->active = nullptr;
+  FSP_HIP(hipMalloc((void**)&S->prof->active, (size_t)max_launches * sizeof(int32_t)));
+  S->prof->events.assign(2 * (size_t)max_launches, nullptr);
+  for (auto& e : S->prof->events) FSP_HIP(hipEventCreate(&e));
+  S->prof->name = kernel;
+  S->prof->used = 0;
+  S->prof->on = true;
   return FSP_OK;
 }
 
@@ -2917,21 +2948,21 @@ fsp_status fsp_profile_end(fsp_solver* S, uint32_t* launches, double* total_ms, 
                            int32_t* active, uint32_t max_durations) {
   if (!S) return FSP_INVALID;
   FSP_HIP(hipStreamSynchronize(S->stream));
-  const size_t count = S->prof_used / 2;
+  const size_t count = S->prof->used / 2;
   double total = 0.0;
   for (size_t q = 0; q < count; ++q) {
     float ms = 0.f;
-    FSP_HIP(hipEventElapsedTime(&ms, S->prof_events[2 * q], S->prof_events[2 * q + 1]));
+    FSP_HIP(hipEventElapsedTime(&ms, S->prof->events[2 * q], S->prof->events[2 * q + 1]));
     total += ms;
     if (durations_ms && q < max_durations) durations_ms[q] = ms;
   }
   if (active && count > 0)
-    FSP_HIP(hipMemcpy(active, S->prof_active, std::min<size_t>(count, max_durations) * sizeof(int32_t),
+    FSP_HIP(hipMemcpy(active, S->prof->active, std::min<size_t>(count, max_durations) * sizeof(int32_t),
                       hipMemcpyDeviceToHost));
   if (launches) *launches = (uint32_t)count;
   if (total_ms) *total_ms = total;
-  S->prof_on = false;
-  S->prof_used = 0;
+  S->prof->on = false;
+  S->prof->used = 0;
   return FSP_OK;
 }
 

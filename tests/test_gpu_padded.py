@@ -1,7 +1,7 @@
 """Domains whose rows do not split into quads are projected in a domain padded
 with solid cells in x. One solver goes through every kind of geometry, each
-projected in the padded domain and, while a kernel of it is being timed, by
-the solver's own general kernels: the same iterations, status and fields.
+projected as it is and while a kernel of it is being timed: the same
+iterations, status and fields.
 
 Tolerances: at a relative residual of 1e-10 and a condition of at most 1e4
 (ghost fractions of 0.01 at least, small grids) the two solutions agree to 1e-6
@@ -137,4 +137,68 @@ def test_padded_projection_is_the_general_one(size, options):
     vol.set_surface_mode(True, True)
     vol.set_free_surface(np.full(nx * ny, 2 * nz * DX, np.float32), rest)
     compare(vol, faces, "closed box", 1e-8)
+    vol.close()
+
+
+# ---------------------------------------------------------------- which kernels ran
+def launches(vol, kernel, call):
+    """What `call` returns, and how often it launched `kernel`."""
+    L = _lib.lib()
+    assert L.fsp_profile_begin(vol._h, kernel.encode(), 4096) == 0
+    out = call()
+    n, total = C.c_uint32(), C.c_double()
+    assert L.fsp_profile_end(vol._h, C.byref(n), C.byref(total), None, None, 0) == 0
+    return out, n.value
+
+
+def runs_padded(vol):
+    """Whether vol's projections run in the padded domain (whose CG update
+    takes quads of cells), from one that is thrown away."""
+    p = vol.p.clone()
+    run = lambda: vol.project_mobile3(SCALE, K1, 3, warm=False)
+    quads, cells = launches(vol, "k_q_update", run)[1], launches(vol, "k_update", run)[1]
+    vol.p.copy_(p)
+    assert (quads > 0) != (cells > 0)
+    return quads > 0
+
+
+def tank(nx, ny, nz, rng, **o):
+    """A half-full tank at rest level 0.5 nz dx, a tenth of a cell or more
+    from the cell centres, and faces that vanish on the walls."""
+    opts = dict(preconditioner=_lib.PRECOND_MULTIGRID, smoother=_lib.SMOOTH_RBGS, max_levels=-1, pre_sweeps=2,
+                post_sweeps=2, coarse_sweeps=4, coarse_operator=_lib.COARSE_GALERKIN)
+    opts.update(o)
+    vol = Volume3.configure(Domain3(nx, ny, nz, DX), rho=RHO, g_eff=G, **opts)
+    eta = (DX * (np.round(0.5 * nz + np.sin(2 * np.pi * np.arange(nx) / nx)) - 0.5 +
+                 rng.uniform(0.1, 0.9, (ny, nx)))).astype(np.float32).ravel()
+    faces = [(0.2 * rng.standard_normal(s)).astype(np.float32)
+             for s in ((nz, ny, nx + 1), (nz, ny + 1, nx), (nz + 1, ny, nx))]
+    faces[0][:, :, [0, nx]] = 0
+    faces[1][:, [0, ny]] = 0
+    faces[2][[0, nz]] = 0
+    vol.set_surface_mode(False, False)
+    vol.set_free_surface(eta, 0.5 * nz * DX)
+    vol.set_velocity(*[f.ravel() for f in faces])
+    return vol, eta, [f.ravel() for f in faces]
+
+
+def blocks(nx, ny, nz, rng):
+    solid = (rng.random((nz, ny, nx)) < 0.05).astype(np.uint8)
+    solid[0, 0, nx - 1] = 1
+    return solid.ravel()
+
+
+def test_timing_preconditioner_and_tuning_act_on_the_kernels_that_project():
+    rng = np.random.default_rng(3)
+    vol, eta, faces = tank(34, 20, 24, rng)
+    vol.set_solid(blocks(34, 20, 24, rng))
+    assert runs_padded(vol)
+    r = torch.from_numpy(rng.uniform(-1, 1, vol.domain.cells).astype(np.float32)).cuda()
+    z, n = launches(vol, "k_q_restrict", lambda: vol.precondition(r))
+    assert n == 1 and float(z.abs().max()) > 0
+    # the padded width, 40 cells, is ten quads: tiles of 4, 8 or 16
+    tile, us = vol.autotune()
+    assert tile in (4, 8, 16) and us > 0
+    rep = vol.project_mobile3(SCALE, K1, 400, warm=False)
+    assert not rep.degraded
     vol.close()
