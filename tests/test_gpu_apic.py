@@ -82,6 +82,21 @@ def test_apic_projection_matches_the_f64_oracle(opts):
     assert err <= 1e-4 and ferr <= 1e-4 and metric <= 1e-5
 
 
+@pytest.mark.parametrize("size", [(34, 24, 28), (33, 20, 18), (18, 12, 20)], ids=str)
+def test_apic_projection_on_widths_that_do_not_split_into_quads(size):
+    nx, ny, nz = size
+    dx = 0.025
+    label, phi, u, v, w = scene(nx, ny, nz, dx, seed=5)
+    rep, (p, u2, v2, w2) = project_on_card(nx, ny, nz, dx, label, phi, u, v, w)
+    p64, ur, vr, wr, it, res, div = po.apic_project(nx, ny, nz, dx, RHO, DT, label, phi, u, v, w, precision=64)
+    water = label == _lib.LABEL_WATER
+    umax = max(np.abs(a).max() for a in (ur, vr, wr))
+    assert not rep.degraded and rep.residual <= 1e-6
+    assert np.linalg.norm(p[water] - p64[water]) <= 1e-4 * np.linalg.norm(p64[water])
+    assert max(np.abs(a.astype(np.float64) - b).max() for a, b in ((u2, ur), (v2, vr), (w2, wr))) <= 1e-4 * umax
+    assert po.apic_divergence_metric(nx, ny, nz, label, u2, v2, w2) <= 1e-5
+
+
 def test_apic_pool_at_rest_is_hydrostatic():
     """Gravity on a flat pool, no body: p = rho g (h - z_c) and the water
     faces back to 0 (the ghost-fluid closed form)."""
