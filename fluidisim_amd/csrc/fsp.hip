@@ -1328,7 +1328,7 @@ fsp_status pad_modes(fsp_solver* S) {
     return give_up_padding(S);
   const bool recapture = I->frac != S->frac || I->levelset != S->levelset || I->coupled != S->coupled ||
                          (S->levelset && I->theta_min != S->theta_min);
-  I->cut = S->cut;
+  I->cut = 1;
   I->frac = S->frac;
   I->levelset = S->levelset;
   I->coupled = S->coupled;
@@ -1338,13 +1338,15 @@ fsp_status pad_modes(fsp_solver* S) {
 
 // The geometry of S (set on the device) in its padded solver: the added cells
 // are solid, their faces closed. edge_open: a face of the wall at +x has an
-// aperture, which must stay a wall's: S projects by itself.
+// aperture, which must stay a wall's: S projects by itself. (An uncut domain
+// has no apertures: its walls' faces count in the divergence as they are, with
+// the code of an open face in the padded domain, which is cut by its added
+// cells, and are no coupling in either. A 90x70x54 basin without solids takes
+// 3.17 ms so, 4.60 by its own kernels.)
 fsp_status pad_geometry(fsp_solver* S, bool edge_open) {
   if (!S->inner) return FSP_OK;
-  if (edge_open) {
-    S->inner->geom = false;
-    return prepare_graph(S, 0);
-  }
+  S->inner->geom = false;
+  if (edge_open) return prepare_graph(S, 0);
   if (const fsp_status st = pad_modes(S)) return st;
   fsp_solver* I = S->inner;
   if (!I) return FSP_OK;
@@ -2252,7 +2254,7 @@ fsp_status fsp_set_geometry(fsp_solver* S, const fsp_surface* surf, const float*
   if (recapture)
     if (const fsp_status gst = regraph(S)) return gst;
   bool edge_open = false;  // an aperture in the wall at +x
-  for (size_t row = 0; row < ny * nz; ++row) edge_open |= hu[row * (nx + 1) + nx] != 0;
+  for (size_t row = 0; cut && row < ny * nz; ++row) edge_open |= hu[row * (nx + 1) + nx] != 0;
   return pad_geometry(S, edge_open);
 }
 
