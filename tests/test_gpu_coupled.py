@@ -202,6 +202,24 @@ def test_refine_of_an_unconverged_projection_on_the_card():
     vol.close()
 
 
+@pytest.mark.parametrize("nx", [34, 33])
+def test_coupled_projection_and_refinement_of_ragged_widths(nx):
+    """The same where rows do not split into quads (33: no coarse level)."""
+    prob, total, bg, faces = scene(nx=nx, ny=24, nz=28, seed=10)
+    p64 = po.project_coupled(prob, *faces, SCALE, K1, total, *bg, opts=po.options(rel_tol=1e-10), precision=64)[5]
+    vol = volume(prob)
+    vol.set_coupling(total, *bg)
+    vol.set_velocity(*faces)
+    rep = vol.project_mobile3(SCALE, K1, 2000, rel_tol=1e-7, warm=False)
+    assert not rep.degraded
+    compare(prob, total, bg, faces, fields(vol), p64, f"coupled {nx}")
+    assert vol.project_mobile3(SCALE, K1, 2, warm=False).degraded
+    rep = vol.refine_mobile3(SCALE, K1, 2000)
+    assert rep.refinements == 1 and not rep.degraded
+    compare(prob, total, bg, faces, fields(vol), p64, f"refine {nx}")
+    vol.close()
+
+
 def test_projection_path_of_the_step_refines_only_after_a_degraded_floor():
     prob, total, bg, faces = scene(seed=11)
     vol = volume(prob)

@@ -15,7 +15,8 @@ import numpy as np
 import pytest
 
 from fluidisim_amd import _lib
-from fluidisim_amd.volume import Domain3, Volume3
+from fluidisim_amd import workloads as W
+from fluidisim_amd.volume import Domain3, Error, ProjectionError, Volume3, project_batch
 from oracle import pyoracle as po
 
 pytestmark = pytest.mark.gpu
@@ -382,3 +383,66 @@ def test_an_uncut_basin_is_projected_in_the_padded_domain(size, options):
         vol.project_mobile3(SCALE, K1, 400, rel_tol=1e-10, warm=False)
         assert all(np.array_equal(a, b) for a, b in zip(fields(), padded))
     vol.close()
+
+
+def test_steps_in_the_padded_domain_follow_the_oracle():
+    """Ten steps of a sloshing tank of 34 x 24 columns with solid spheres
+    against the f32 oracle with the same V-cycle, within the step's tolerances
+    (heights 2e-6 m, fields 1e-3 relative L2); a step with a velocity that is
+    not finite is refused and leaves every field as it was."""
+    wl = W.slosh(34, 32, 24, seed=9, amplitude=0.03)
+    d, o = wl.domain, wl.options
+    vol = W.build_volume(wl)
+    reps = []
+    for step in range(10):
+        rep, n = launches(vol, "k_q_update", lambda: vol.step_surface_mobile(1000, 4000))
+        assert not rep.degraded and n >= rep.iterations > 0
+        reps.append(rep.iterations)
+    prob = po.Problem(d.nx, d.ny, d.nz, d.dx, wl.eta, rho=wl.rho, g_eff=wl.g_eff, rest=wl.rest,
+                      homogeneous_ghost=False, closed_lid=False, solid=wl.solid)
+    out = po.step_surface(prob, wl.us, wl.vs, wl.ws, np.zeros(d.cells, np.float32), 10, 1000, 4000,
+                          po.options(multigrid=1, smoother=o["smoother"], pre=o["pre_sweeps"], post=o["post_sweeps"],
+                                     coarse=o["coarse_sweeps"], coarse_op=o["coarse_operator"]))
+    assert out["status"] == 0 and out["done"] == 10
+    print("iterations", reps, "oracle", [r["iterations"] for r in out["reports"]])
+    assert np.abs(vol.surface()[0] - out["eta"]).max() <= 2e-6
+    for name, t in (("u", vol.u), ("v", vol.v), ("w", vol.w), ("p", vol.p)):
+        err = np.linalg.norm(t.cpu().numpy() - out[name]) / np.linalg.norm(out[name])
+        assert err <= 1e-3, (name, err)
+    bits = lambda: [np.ascontiguousarray(a).view(np.uint32).copy() for a in
+                    (*(t.cpu().numpy() for t in (vol.u, vol.v, vol.w, vol.p)), *vol.surface())]
+    vol.u[vol.u.numel() // 2] = float("inf")
+    before = bits()
+    with pytest.raises(ProjectionError) as e:
+        vol.step_surface_mobile(1000, 4000)
+    assert e.value.error == Error.NotFinite
+    assert all(np.array_equal(a, b) for a, b in zip(bits(), before))
+    vol.close()
+
+
+def test_batched_and_host_projections_of_ragged_widths_equal_single_ones():
+    wls = [W.tank(*s, seed=3 + q) for q, s in enumerate(((34, 30, 32), (50, 24, 20), (64, 32, 32), (33, 12, 16),
+                                                         (90, 40, 26), (34, 30, 32)))]
+    vols = [W.build_volume(wl) for wl in wls]
+    assert [runs_padded(v) for v in vols[:2]] == [True, True]
+    fields = lambda v: [t.cpu().numpy().view(np.uint32).copy() for t in (v.p, v.u, v.v, v.w)]
+    single = []
+    for wl, v in zip(wls, vols):
+        assert not v.project_mobile3(wl.scale, wl.k1, 2000, warm=False).degraded
+        single.append(fields(v))
+    for t in range(2):
+        project_batch(vols, [wl.scale for wl in wls], [wl.k1 for wl in wls], 2000, concurrency=4)
+        for v, s in zip(vols, single):
+            assert all(np.array_equal(a, b) for a, b in zip(fields(v), s))
+    host = [np.full(n, 7.0, np.float32) for n in (wls[0].domain.cells, *wls[0].domain.faces)]
+    args = []
+    for a in (wls[0].us, wls[0].vs, wls[0].ws, host[0]):
+        args += [a.ctypes.data, a.size]
+    args.append(0)
+    for a in host[1:]:
+        args += [a.ctypes.data, a.size]
+    rep = _lib.Report()
+    assert _lib.lib().fsp_project(vols[0]._h, *args, wls[0].scale, wls[0].k1, 1e-6, 2000, C.byref(rep)) == 0
+    assert all(np.array_equal(a.view(np.uint32), b) for a, b in zip(host, single[0]))
+    for v in vols:
+        v.close()
