@@ -1548,11 +1548,13 @@ __global__ void __launch_bounds__(QBLOCK) k_q_update(Fine G, QuadGrid Q, double*
 constexpr int TAIL_THREADS = 1024;
 constexpr int TAIL_MAX_LEVELS = 8;
 constexpr int TAIL_CELLS = 4096;                // largest first level of the tail
-// Limit of a tail workgroup's LDS (the row-coefficient tail's; the compact
-// tail holds its first level in registers and takes half). With a limit of 64 KiB
-// on levels held in LDS a closed box of 64^3 ran the 16 colour passes of its
-// coarsest level, 16^3, as launches of their own.
-constexpr int TAIL_LDS_FLOATS = 6 * (TAIL_CELLS + TAIL_CELLS / 4);
+// Largest dynamic LDS of a tail workgroup, in floats: the compact tail's with
+// one level of odd rows, six floats a cell, 96 KiB. (With even rows the first
+// level is in registers, its x and two guards in LDS: 46 KiB with the levels
+// below. The row-coefficient tail takes three floats a cell, 55 KiB in all.)
+// With a limit of 64 KiB on levels held in LDS a closed box of 64^3 ran the
+// 16 colour passes of its coarsest level, 16^3, as launches of their own.
+constexpr int TAIL_LDS_FLOATS = 6 * TAIL_CELLS;
 
 struct TailSet {
   Level lv[TAIL_MAX_LEVELS];  // global arrays of the tail levels (first .. last)

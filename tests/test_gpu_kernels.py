@@ -1,5 +1,7 @@
 """Kernel forms at the sizes where they change, against the oracle: the
 V-cycle bit for bit (both sides do the same arithmetic in the same order)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -300,3 +302,38 @@ def test_blocks_that_fall_dry_and_wet_leave_no_trace_in_any_form(form):
         for a, b in zip(got, ref):
             assert np.array_equal(bits(a), bits(b)), (step, fill)
     used.close()
+
+
+@pytest.mark.parametrize("size", [(34, 30, 28), (30, 30, 30)], ids=str)
+@pytest.mark.parametrize("sweeps", [4, 7])
+def test_an_odd_coarsest_level_over_64_kib_in_the_tail_matches_the_oracle(size, sweeps):
+    """17 x 15 x 14 and 15^3 cells, 24 bytes of LDS each. (An aperture in the
+    wall at +x keeps these widths out of the padded domain, whose levels have
+    even rows.)"""
+    nx, ny, nz = size
+    wl = W.tank(nx, nz, ny, seed=101)
+    d = wl.domain
+    solid = np.asarray(wl.solid).reshape(nz, ny, nx) != 0
+    opens = []
+    for axis, shape in ((2, (nz, ny, nx + 1)), (1, (nz, ny + 1, nx)), (0, (nz + 1, ny, nx))):
+        a = np.ones(shape, np.float32)
+        lo, hi = [slice(None)] * 3, [slice(None)] * 3
+        lo[axis], hi[axis] = slice(0, -1), slice(1, None)
+        a[tuple(lo)][solid] = 0
+        a[tuple(hi)][solid] = 0
+        lo[axis], hi[axis] = 0, -1
+        a[tuple(lo)] = 0
+        a[tuple(hi)] = 0
+        opens.append(a)
+    opens[0][:, :, nx] = ~solid[:, :, nx - 1]
+    wl.open_u, wl.open_v, wl.open_w = [a.ravel() for a in opens]
+    assert_vcycle_is_the_oracles(wl, max_levels=1, coarse_sweeps=sweeps)
+    # in the tail: no pass over the level in a launch of its own
+    vol = W.build_volume(wl)
+    L = _lib.lib()
+    assert L.fsp_profile_begin(vol._h, b"k_r6_gs", 64) == 0
+    vol.precondition(torch.ones(d.cells, device="cuda"))
+    n, total = C.c_uint32(), C.c_double()
+    assert L.fsp_profile_end(vol._h, C.byref(n), C.byref(total), None, None, 0) == 0
+    vol.close()
+    assert n.value == 0
