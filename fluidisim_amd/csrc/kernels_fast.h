@@ -1504,8 +1504,11 @@ __device__ __forceinline__ double fold_partials(const double* partials, int slot
 // number of partials of <d, q> that every workgroup folds itself (the
 // iteration's k_finish records the sum, the step and the buffer switch), or 0
 // where k_finish has run in between (above FSP_FOLD_PARTIALS the folds read
-// more than that launch costs: 2048 partials take 128^3 cells from 1.923 to 1.911
-// ms, 1024 leave it there).
+// more than that launch costs). Folded against not, projections of tanks from
+// 32^3 cells up, by their number of partials: to 1024 1.2 to 1.5 % faster (64^3
+// 0.901 -> 0.887 ms, 128x64x128 1.299 -> 1.280), 1536 0.6, 2048 0.2, 3072 to
+// 4096 0.1 to 0.3 % slower (128x192x128 1.786 -> 1.792), 6144 1.4 (256x192x128
+// 2.396 -> 2.429), 8192 3 (256x128x256 3.43 -> 3.53).
 __global__ void __launch_bounds__(QBLOCK) k_q_update(Fine G, QuadGrid Q, double* p, float* r, const float* d0,
                                                      const float* d1, const float* q, Ctl* ctl, double* partials,
                                                      unsigned dq_parts) {
