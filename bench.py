@@ -48,6 +48,43 @@ def bytes_per_cell(kernel, zb):
     return table.get(kernel)
 
 
+# The kernels that leave a block without a wet cell at once: the block's cells
+# in x, y and z (of a brick, or of a workgroup of the quad grid, the
+# restriction's over two planes), and the bytes per cell such a block still
+# writes (z' = 0, coarse r = 0).
+def dry_blocks(kernel, zb, nx):
+    quads = 1
+    while quads < nx // 4 and quads < 64:
+        quads *= 2
+    grid = (4 * quads, 256 // quads, 1)
+    table = {
+        "k_q_brick<0>": ((32, 8, 8), zb), "k_q_brick<2>": ((32, 8, 8), zb), "k_q_gs_first": (grid, zb),
+        "k_q_spmv_dir": (grid, 0), "k_q_update": (grid, 0), "k_q_restrict": (grid[:2] + (2,), zb / 8),
+    }
+    return table.get(kernel)
+
+
+def bytes_per_launch(kernel, wl, zb):
+    """Algorithmic bytes of one launch on wl, and the share of the cells that
+    lie in blocks with a wet cell (1 for kernels that leave none out)."""
+    bpc, d = bytes_per_cell(kernel, zb), wl.domain
+    skipped = dry_blocks(kernel, zb, d.nx)
+    if bpc is None or skipped is None:
+        return bpc and bpc * d.cells, 1.0
+    block, dry = skipped
+    zc = ((np.arange(d.nz, dtype=np.float32) + np.float32(0.5)) * np.float32(d.dx))[:, None, None]
+    wet = zc < wl.eta.reshape(1, d.ny, d.nx)
+    if wl.solid is not None:
+        wet &= wl.solid.reshape(d.nz, d.ny, d.nx) == 0
+    cells = np.ones(wet.shape, np.int64)
+    for axis, step in zip((2, 1, 0), block):
+        at = np.arange(0, wet.shape[axis], step)
+        wet = np.logical_or.reduceat(wet, at, axis=axis)
+        cells = np.add.reduceat(cells, at, axis=axis)
+    work = int(cells[wet].sum())
+    return bpc * work + dry * (d.cells - work), work / d.cells
+
+
 def parse():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -398,14 +435,14 @@ def main():
     # Launches queued after convergence return at once: only the launches that
     # started with the CG loop active (the flag the library records on the
     # device in stream order before each timed launch) are averaged.
-    bpc = bytes_per_cell(args.kernel, 4 if args.storage == "f32" else 2)
+    # Blocks without a wet cell, which a kernel leaves at once, are not counted.
+    bytes_launch, at_work = bytes_per_launch(args.kernel, wl, 4 if args.storage == "f32" else 2)
     roofline = None
-    if bpc is not None and launches.value > 0:
+    if bytes_launch and launches.value > 0:
         m = min(launches.value, max_launches)
         d = durations[:m].astype(np.float64)
         eff = d[active[:m] != 0]
         avg_ms = float(eff.mean())
-        bytes_launch = bpc * wl.domain.cells
         achieved = bytes_launch / (avg_ms * 1e-3) / 1e9
         roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "instrumented_ms_per_step": round(1000.0 * (ti1 - ti0) / args.steps, 4),
@@ -413,7 +450,8 @@ def main():
                     "kernel": args.kernel, "copy_probe_gbs": round(copy_probe(torch), 1),
                     "launches": int(eff.size), "noop_launches": int(d.size - eff.size),
                     "launches_per_projection": round(eff.size / args.steps, 2),
-                    "avg_us": round(avg_ms * 1000.0, 2), "bytes_per_launch": int(bytes_launch)}
+                    "avg_us": round(avg_ms * 1000.0, 2), "bytes_per_launch": int(bytes_launch),
+                    "cells_at_work": round(at_work, 4)}
         log(f"[bench] {args.kernel}: {eff.size} launches, {avg_ms * 1000:.1f} us avg, {achieved:.0f} GB/s")
 
     host = None if args.no_host else host_pointer_line(vol, wl, max(1, min(args.steps, 3)), torch)
