@@ -112,7 +112,10 @@ const char* fsp_status_string(fsp_status s);
 void fsp_default_options(fsp_options* out);
 
 /* Replaces Volume3::configure + enable_multigrid (delta3d.rs:210-294,
- * delta3d_multigrid.rs:339-349): reserves every device buffer. */
+ * delta3d_multigrid.rs:339-349): reserves every device buffer. A width nx
+ * that is no multiple of 4 is projected in a domain padded in x, whose buffers
+ * stand beside these: about twice the memory, unless the padded ones would
+ * take an eighth of what is free. */
 fsp_status fsp_create(const fsp_domain* domain, const fsp_options* options, fsp_solver** out);
 void fsp_destroy(fsp_solver* s);
 /* Coarse levels the solver holds (Volume3::multigrid_levels, delta3d_multigrid.rs:352-354). */
@@ -268,7 +271,8 @@ fsp_status fsp_assemble_device(fsp_solver* s, const float* d_div, float scale, f
 
 /* One preconditioner application z = M^-1 r on the current geometry
  * (v_cycle3, delta3d_multigrid.rs:393-429), with the fine kernels a
- * projection on this geometry runs. Device pointers. */
+ * projection on this geometry runs; r may be anything, on dry cells too.
+ * Device pointers. */
 fsp_status fsp_precondition_device(fsp_solver* s, const float* d_r, float* d_z);
 
 /* Divergence of faces (delta3d.rs:747-763, :806-823). Device pointers. */
